@@ -4,7 +4,7 @@
 //
 // The work matrix stays in limb planes on the device for the whole call.  Per column block [k0, k1):
 //   1. the diagonal block, column by column in one workgroup (pivot, sqrt, then div of the entries below);
-//   2. the rows below it, one wavefront per row (chol_panel_kernel);
+//   2. the rows below it, one wavefront per row (tri_block_kernel);
 //   3. the trailing update a_ij = D(a_ij; l_i, l_j; [k0, k1)) for i >= j >= k1, in two parts as the
 //      reference splits it (linalg.mm:440-452): the next panel's columns [k1, k2) by the look-ahead kernel
 //      on the caller's stream, followed there by the next panel, while the rest (i >= j >= k2) runs as one
@@ -64,10 +64,9 @@ struct OwnedStream {
 };
 
 typedef hipError_t (*diag_fn)(const lf::FactorArgs&, uint32_t, hipStream_t);
-typedef hipError_t (*panel_fn)(const lf::FactorArgs&, hipStream_t);
+typedef hipError_t (*tri_fn)(const lf::TriArgs&, hipStream_t);
 typedef hipError_t (*lookahead_fn)(const lf::FactorArgs&, uint32_t, uint32_t, hipStream_t);
 typedef hipError_t (*invalid_fn)(uint32_t*, uint64_t, uint32_t, uint32_t, hipStream_t);
-typedef hipError_t (*solve_fn)(int, const lf::SolveArgs&, hipStream_t);
 typedef hipError_t (*solve_update_fn)(int, const lf::SolveArgs&, uint32_t, hipStream_t);
 typedef hipError_t (*recip_fn)(const uint32_t*, uint64_t, uint32_t, uint32_t*, uint64_t, hipStream_t);
 typedef hipError_t (*steps_fn)(const uint32_t*, uint64_t, uint32_t*, uint64_t, int32_t*, int, uint64_t*, uint32_t*, hipStream_t);
@@ -75,11 +74,10 @@ struct FactorTables;
 template <int N> void fill_factor(FactorTables& t);
 struct FactorTables {
     diag_fn diag[33] = {};
-    panel_fn panel[33] = {};
+    tri_fn tri_block[33] = {};
     lookahead_fn lookahead[33] = {};
     invalid_fn invalid[33] = {};
     hipError_t (*zero_upper[33])(uint32_t*, uint64_t, uint32_t, hipStream_t) = {};
-    solve_fn solve[33] = {};
     solve_update_fn solve_update[33] = {};
     recip_fn reciprocals[33] = {};
     steps_fn steps[33] = {};
@@ -88,11 +86,10 @@ struct FactorTables {
 template <int N> void fill_factor(FactorTables& t)
 {
     t.diag[N] = lf::launch_chol_diag<N>;
-    t.panel[N] = lf::launch_chol_panel<N>;
+    t.tri_block[N] = lf::launch_tri_block<N>;
     t.lookahead[N] = lf::launch_chol_lookahead<N>;
     t.invalid[N] = lf::launch_chol_invalid<N>;
     t.zero_upper[N] = lf::launch_zero_upper<N>;
-    t.solve[N] = lf::launch_solve<N>;
     t.solve_update[N] = lf::launch_solve_update<N>;
     t.reciprocals[N] = lf::launch_reciprocals<N>;
     t.steps[N] = lf::launch_factor_steps<N>;
@@ -233,10 +230,10 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
         return fail(LF_INVALID_ARGUMENT, "cholesky: the block is too large for the exact-dot scratch (use a smaller block)");
     FACTOR_HIP(dinfo.alloc(sizeof(lf::FactorInfo)), "hipMalloc (pivot)");
     FACTOR_HIP(dscratch.alloc(2 * swords * threads * 4), "hipMalloc (scratch)");
-    // reciprocals of the pivots (N+1 planes of n entries), for the divisions of the rows below each block
+    // reciprocals of the pivots (up to N+3 planes of n entries), for the divisions of the rows below each block
     DevBuf drecip;
     const uint64_t rpitch = (n + 63) / 64 * 64;
-    FACTOR_HIP(drecip.alloc((N + 1) * rpitch * 4), "hipMalloc (reciprocals)");
+    FACTOR_HIP(drecip.alloc((N + 3) * rpitch * 4), "hipMalloc (reciprocals)");
     // the pivot record comes back through pinned memory, so that reading it does not wait on the stream
     struct PinnedInfo {
         lf::FactorInfo* p = nullptr;
@@ -278,7 +275,11 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
         const lf::FactorArgs f = args(a, b);
         FACTOR_HIP(hipEventRecord(p0, s), "hipEventRecord");
         FACTOR_HIP(tables().diag[N](f, uint32_t(std::min<uint64_t>(256, (b - a + 63) / 64 * 64)), s), "panel launch");
-        FACTOR_HIP(tables().panel[N](f, s), "panel launch");
+        // the rows below: row i is the right-hand side of L_block l_i = a_i
+        const lf::TriArgs t{W, pitch, int64_t(a * n + a), int64_t(n), 1, W, pitch, int64_t(b * n + a), 1, int64_t(n), (const uint32_t*)drecip.p,
+                            rpitch, int64_t(a), 1, uint32_t(b - a), uint32_t(n - b), (uint32_t*)dscratch.p, swords, &f.info->error, f.info,
+                            uint32_t(a)};
+        FACTOR_HIP(tables().tri_block[N](t, s), "panel launch");
         FACTOR_HIP(hipEventRecord(p1, s), "hipEventRecord");
         FACTOR_HIP(hipMemcpyAsync(hinfo.p, dinfo.p, sizeof(lf::FactorInfo), hipMemcpyDeviceToHost, s), "download pivot");
         FACTOR_HIP(hipEventRecord(panel_done, s), "hipEventRecord");
@@ -397,7 +398,7 @@ int lf_solve(int bits, int passes, const lf_operand* L, uint64_t n, const lf_ope
     // reciprocals of the n diagonal entries, for every division of both passes
     DevBuf drecip;
     const uint64_t rpitch = (n + 63) / 64 * 64;
-    FACTOR_HIP(drecip.alloc((N + 1) * rpitch * 4), "hipMalloc (reciprocals)");
+    FACTOR_HIP(drecip.alloc((N + 3) * rpitch * 4), "hipMalloc (reciprocals)");
     FACTOR_HIP(tables().reciprocals[N](F, fpitch, uint32_t(n), (uint32_t*)drecip.p, rpitch, s), "reciprocals launch");
     double gpu = 0;
     // device time: an event pair around every in-block kernel and direct update, read after the last
@@ -420,10 +421,13 @@ int lf_solve(int bits, int passes, const lf_operand* L, uint64_t n, const lf_ope
         if ((e = launch()) != hipSuccess) return e;
         return hipEventRecord(b, s);
     };
+    // row r of the block is row r0 + r of L going forward, and row r1 - 1 - r of L^T (column of L) going backward
     auto block_solve = [&](int backward, uint64_t r0, uint64_t r1) {
-        lf::SolveArgs a{F, fpitch, Xp, xpitch, uint32_t(n), uint32_t(nrhs), uint32_t(r0), uint32_t(r1), (uint32_t*)dscratch.p, swords,
-                        (int32_t*)derr.p, (const uint32_t*)drecip.p, rpitch};
-        return timed([&] { return tables().solve[N](backward, a, s); });
+        const int64_t first = backward ? int64_t(r1 - 1) : int64_t(r0), step = backward ? -1 : 1;
+        const lf::TriArgs t{F, fpitch, first * int64_t(n) + first, backward ? -1 : int64_t(n), backward ? -int64_t(n) : 1, Xp, xpitch,
+                            first * int64_t(nrhs), step * int64_t(nrhs), 1, (const uint32_t*)drecip.p, rpitch, first, step, uint32_t(r1 - r0),
+                            uint32_t(nrhs), (uint32_t*)dscratch.p, swords, (int32_t*)derr.p, nullptr, 0};
+        return timed([&] { return tables().tri_block[N](t, s); });
     };
     float ms = 0;
     // An off-block update of fewer multiply-adds than solve_host_macs (the reference's threshold for taking
@@ -436,7 +440,7 @@ int lf_solve(int bits, int passes, const lf_operand* L, uint64_t n, const lf_ope
     };
     auto dot_update = [&](int backward, uint64_t r0, uint64_t r1) {
         lf::SolveArgs a{F, fpitch, Xp, xpitch, uint32_t(n), uint32_t(nrhs), uint32_t(r0), uint32_t(r1), (uint32_t*)dscratch.p, swords,
-                        (int32_t*)derr.p, (const uint32_t*)drecip.p, rpitch};
+                        (int32_t*)derr.p};
         return timed([&] { return tables().solve_update[N](backward, a, uint32_t(slots), s); });
     };
     if (passes & 1)

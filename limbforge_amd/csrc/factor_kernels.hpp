@@ -529,27 +529,32 @@ __device__ Num<N> wave_dot_sub(const Num<N>& c, const VecView& x, const VecView&
     return r;
 }
 
+} // namespace lf
+#include "factor_wave.hpp"
+namespace lf {
+
 // ---------------------------------------------------------------- Cholesky
 template <int N> __device__ __forceinline__ Num<N> element(const FactorArgs& f, u32 i, u32 j)
 {
     return load_out<N>(f.w, f.pitch, (u64)i * f.n + j);
 }
 
-// The reciprocal (limb_core.hpp reciprocal) of the pivot or diagonal entry i, N+1 planes.
-template <int N> __device__ __forceinline__ void load_recip(const u32* r, u64 rpitch, u32 i, u32 (&v)[N + 1])
+// The reciprocal of the pivot or diagonal entry i: its leading N+1 words (limb_core.hpp reciprocal) are the last
+// planes stored.
+template <int N> __device__ __forceinline__ void load_recip(const u32* r, u64 rpitch, u64 i, u32 (&v)[N + 1])
 {
 #pragma unroll
-    for (int k = 0; k <= N; ++k) v[k] = r[(u64)k * rpitch + i];
+    for (int k = 0; k <= N; ++k) v[k] = r[(u64)(k + recip_words<N>() - (N + 1)) * rpitch + i];
 }
 template <int N> __device__ __forceinline__ void store_recip(u32* r, u64 rpitch, u32 i, const Num<N>& d)
 {
-    u32 v[N + 1];
-    if (d.s && !d.st) reciprocal<N>(d.w, v);
+    u32 v[recip_words<N>()];
+    if (d.s && !d.st) reciprocal_words<N>(d.w, v);
     else
 #pragma unroll
-        for (int k = 0; k <= N; ++k) v[k] = 0; // never used: division by zero or a status is decided first
+        for (int k = 0; k < recip_words<N>(); ++k) v[k] = 0; // never used: division by zero or a status is decided first
 #pragma unroll
-    for (int k = 0; k <= N; ++k) r[(u64)k * rpitch + i] = v[k];
+    for (int k = 0; k < recip_words<N>(); ++k) r[(u64)k * rpitch + i] = v[k];
 }
 
 // Waves of the diagonal-block workgroup: 12 up to 4 limbs (three waves per SIMD leave 168 VGPRs a lane,
@@ -611,29 +616,6 @@ template <int N> __global__ void __launch_bounds__(diag_waves<N>() * WAVE) chol_
     }
 }
 
-// The rows below the diagonal block, one wavefront per row i >= k1: columns [k0, p) in order, p the
-// failing pivot of the block or k1.
-template <int N> __global__ void __launch_bounds__(64) chol_panel_kernel(FactorArgs f)
-{
-    __shared__ WaveLds<N> L;
-    const u32 r = blockIdx.x, lane = threadIdx.x;
-    const u32 i = f.k1 + r;
-    const int32_t piv = f.info->pivot;
-    const u32 pe = piv >= 0 ? (u32)piv : f.k1;
-    const DotScratch sc{f.scratch + (u64)r * 2 * f.swords, f.swords, &f.info->error};
-    const VecView ri{f.w, f.pitch, (i64)i * f.n + f.k0, 1};
-    for (u32 j = f.k0; j < pe; ++j) {
-        const VecView rj{f.w, f.pitch, (i64)j * f.n + f.k0, 1};
-        const Num<N> v = wave_dot_sub<N>(element<N>(f, i, j), ri, rj, j - f.k0, lane, L, sc);
-        if (lane == 0) {
-            u32 rv[N + 1];
-            load_recip<N>(f.recip, f.rpitch, j, rv);
-            store_out<N>(f.w, f.pitch, f.n, i, j, false, div_by_reciprocal<N>(v, element<N>(f, j, j), rv));
-        }
-        __syncthreads(); // entry (i, j) is a term of the row's next dot
-    }
-}
-
 // Look-ahead part of a block's trailing update: after the panel [k0, k1), the entries (i, j), j <= i, of the
 // next panel's columns j in [k1, k2) and rows i in [k1, n) become D(a_ij; l_i, l_j; [k0, k1)) in place -- the
 // same one rounding of the same exact value as the update product gives them -- so that the next panel can
@@ -674,152 +656,42 @@ template <int N> __global__ void __launch_bounds__(256) zero_upper_kernel(u32* w
     if (j > i) store_out<N>(w, pitch, n, i, j, false, zero<N>(ST_OK));
 }
 
-// ---------------------------------------------------------------- triangular solves
-// Forward block [r0, r1) of L X = B, one wavefront per right-hand side.
-template <int N> __global__ void __launch_bounds__(64) solve_forward_kernel(SolveArgs a)
+// ---------------------------------------------------------------- triangular blocks
+// One block of a forward or backward solve, or of the rows below a Cholesky block, one wavefront per
+// right-hand side (row): the wave-parallel recurrence as far as it goes, then the general one.  What bounds it
+// is one wavefront's instruction count: at 256 bits a 32-row block took 163-167 us with the general recurrence
+// (an exact dot of the row's terms and a one-lane division per row).  With a digit per lane the solve of 512
+// unknowns and 64 right-hand sides went from 7.70 to 4.00 ms, the factorization of n = 512 from 12.3 to 10.9 ms.
+template <int N> __global__ void __launch_bounds__(64) tri_block_kernel(TriArgs g)
 {
-    __shared__ WaveLds<N> L;
+    constexpr std::size_t bytes = wd_fits<N>() && sizeof(TriLds<N>) > sizeof(WaveLds<N>) ? sizeof(TriLds<N>) : sizeof(WaveLds<N>);
+    __shared__ __attribute__((aligned(16))) unsigned char lds[bytes];
     const u32 c = blockIdx.x, lane = threadIdx.x;
-    const DotScratch sc{a.scratch + (u64)c * 2 * a.swords, a.swords, a.error};
-    const VecView xc{a.x, a.xpitch, (i64)a.r0 * a.nrhs + c, (i64)a.nrhs};
-    for (u32 i = a.r0; i < a.r1; ++i) {
-        const VecView li{a.f, a.fpitch, (i64)i * a.n + a.r0, 1};
-        const Num<N> v = wave_dot_sub<N>(load_out<N>(a.x, a.xpitch, (u64)i * a.nrhs + c), li, xc, i - a.r0, lane, L, sc);
+    u32 B = g.rows;
+    if (g.info) {
+        const int32_t p = g.info->pivot;
+        if (p >= 0) B = (u32)p - g.k0;
+    }
+    u32 i = 0;
+    if constexpr (wd_fits<N>())
+        if (B <= WD_ROWS) i = tri_block_fast<N>(g, c, B, lane, *reinterpret_cast<TriLds<N>*>(lds));
+    if (i >= B) return;
+    __syncthreads(); // the rows stored so far are terms of the next
+    WaveLds<N>& L = *reinterpret_cast<WaveLds<N>*>(lds);
+    const DotScratch sc{g.scratch + (u64)c * 2 * g.swords, g.swords, g.error};
+    const i64 xb = g.xbase + (i64)c * g.xc;
+    const VecView xv{g.x, g.xpitch, xb, g.xr};
+    for (; i < B; ++i) {
+        const VecView li{g.f, g.fpitch, g.fbase + (i64)i * g.fr, g.fk};
+        const u64 at = (u64)(xb + (i64)i * g.xr);
+        const Num<N> v = wave_dot_sub<N>(load_out<N>(g.x, g.xpitch, at), li, xv, i, lane, L, sc);
         if (lane == 0) {
             u32 rv[N + 1];
-            load_recip<N>(a.recip, a.rpitch, i, rv);
-            store_out<N>(a.x, a.xpitch, a.nrhs, i, c, false, div_by_reciprocal<N>(v, load_out<N>(a.f, a.fpitch, (u64)i * a.n + i), rv));
+            load_recip<N>(g.recip, g.rpitch, (u64)(g.rbase + (i64)i * g.rstep), rv);
+            const Num<N> l = load_out<N>(g.f, g.fpitch, (u64)(g.fbase + (i64)i * (g.fr + g.fk)));
+            store_out<N>(g.x, g.xpitch, 0, 0, (u32)at, false, div_by_reciprocal<N>(v, l, rv));
         }
         __syncthreads(); // x_i is a term of the next row's dot
-    }
-}
-
-// Backward block [r0, r1) of L^T X = B (column i of L as the vector), one wavefront per right-hand side.
-template <int N> __global__ void __launch_bounds__(64) solve_backward_kernel(SolveArgs a)
-{
-    __shared__ WaveLds<N> L;
-    const u32 c = blockIdx.x, lane = threadIdx.x;
-    const DotScratch sc{a.scratch + (u64)c * 2 * a.swords, a.swords, a.error};
-    for (u32 i = a.r1; i-- > a.r0;) {
-        Num<N> v = load_out<N>(a.x, a.xpitch, (u64)i * a.nrhs + c);
-        if (i + 1 < a.r1) {
-            const VecView col{a.f, a.fpitch, (i64)(i + 1) * a.n + i, (i64)a.n};
-            const VecView xc{a.x, a.xpitch, (i64)(i + 1) * a.nrhs + c, (i64)a.nrhs};
-            v = wave_dot_sub<N>(v, col, xc, a.r1 - i - 1, lane, L, sc);
-        }
-        if (lane == 0) {
-            u32 rv[N + 1];
-            load_recip<N>(a.recip, a.rpitch, i, rv);
-            store_out<N>(a.x, a.xpitch, a.nrhs, i, c, false, div_by_reciprocal<N>(v, load_out<N>(a.f, a.fpitch, (u64)i * a.n + i), rv));
-        }
-        __syncthreads();
-    }
-}
-
-// ---- in-block solves with the block staged in LDS
-// The in-block solves run one wavefront per right-hand side, a few waves on the whole GPU, so each row's
-// global loads (its terms, b_i, the reciprocal, l_ii, and the x_k just written) stand on the chain's
-// critical path.  These forms copy the block's part of L (the lower triangle, packed so that each row's
-// terms are contiguous: by rows for the forward pass, by columns for the backward pass), its x column and
-// its reciprocals into LDS once, then read only LDS in the recurrence; x_i goes to LDS for the later rows
-// and to global memory as the result.  Same arithmetic and order as the kernels above.
-constexpr u32 STAGED_ROWS = 32; // largest block the staged forms take
-
-// LDS words of the staged block of B rows: the packed triangle (N+3 planes of B(B+1)/2 entries), the x
-// column (N+3 planes of B entries) and the reciprocals (N+1 planes of B entries).
-template <int N> __host__ __device__ constexpr u32 staged_tri_pitch(u32 B) { return B * (B + 1) / 2; }
-template <int N> __host__ __device__ constexpr u64 staged_words(u32 B) { return (u64)(N + 3) * staged_tri_pitch<N>(B) + (u64)(N + 3) * B + (u64)(N + 1) * B; }
-
-// first index of column i of a column-packed lower triangle of B rows: sum over c < i of (B - c)
-__device__ __forceinline__ u32 tri_col_start(u32 B, u32 i) { return i * B - i * (i - 1) / 2; }
-
-template <int N> __device__ __forceinline__ void stage_copy(u32* dst, u64 dpitch, u64 di, const u32* src, u64 spitch, u64 si)
-{
-#pragma unroll
-    for (int w = 0; w < N + 3; ++w) dst[(u64)w * dpitch + di] = src[(u64)w * spitch + si];
-}
-
-// Copies the block's L triangle (by rows or by columns), x column and reciprocals into LDS.
-template <int N>
-__device__ __forceinline__ void stage_solve_block(const SolveArgs& a, u32 c, bool by_columns, u32* tri, u32* xs, u32* rs, u32 lane)
-{
-    const u32 B = a.r1 - a.r0, TP = staged_tri_pitch<N>(B);
-    for (u32 i = 0; i < B; ++i) {
-        if (by_columns) // column i: rows k = i .. B-1
-            for (u32 k = i + lane; k < B; k += WAVE)
-                stage_copy<N>(tri, TP, tri_col_start(B, i) + (k - i), a.f, a.fpitch, (u64)(a.r0 + k) * a.n + (a.r0 + i));
-        else // row i: columns k = 0 .. i
-            for (u32 k = lane; k <= i; k += WAVE)
-                stage_copy<N>(tri, TP, i * (i + 1) / 2 + k, a.f, a.fpitch, (u64)(a.r0 + i) * a.n + (a.r0 + k));
-    }
-    for (u32 i = lane; i < B; i += WAVE) {
-        stage_copy<N>(xs, B, i, a.x, a.xpitch, (u64)(a.r0 + i) * a.nrhs + c);
-#pragma unroll
-        for (int w = 0; w <= N; ++w) rs[(u64)w * B + i] = a.recip[(u64)w * a.rpitch + a.r0 + i];
-    }
-}
-
-template <int N> __device__ __forceinline__ void load_recip_lds(const u32* rs, u32 B, u32 i, u32 (&v)[N + 1])
-{
-#pragma unroll
-    for (int k = 0; k <= N; ++k) v[k] = rs[(u64)k * B + i];
-}
-
-// Forward block [r0, r1) of L X = B, r1 - r0 <= STAGED_ROWS, block staged in LDS (dynamic shared memory of
-// staged_words<N>(r1 - r0) words); one wavefront per right-hand side.
-template <int N> __global__ void __launch_bounds__(64) solve_forward_staged_kernel(SolveArgs a)
-{
-    __shared__ WaveLds<N> L;
-    extern __shared__ u32 stage[];
-    const u32 c = blockIdx.x, lane = threadIdx.x, B = a.r1 - a.r0, TP = staged_tri_pitch<N>(B);
-    u32* tri = stage;
-    u32* xs = tri + (u64)(N + 3) * TP;
-    u32* rs = xs + (u64)(N + 3) * B;
-    stage_solve_block<N>(a, c, false, tri, xs, rs, lane);
-    __syncthreads();
-    const DotScratch sc{a.scratch + (u64)c * 2 * a.swords, a.swords, a.error};
-    const VecView xv{xs, B, 0, 1};
-    for (u32 i = 0; i < B; ++i) {
-        const VecView li{tri, TP, (i64)(i * (i + 1) / 2), 1};
-        const Num<N> v = wave_dot_sub<N>(load_out<N>(xs, B, i), li, xv, i, lane, L, sc);
-        if (lane == 0) {
-            u32 rv[N + 1];
-            load_recip_lds<N>(rs, B, i, rv);
-            const Num<N> x = div_by_reciprocal<N>(v, load_out<N>(tri, TP, i * (i + 1) / 2 + i), rv);
-            store_out<N>(xs, B, 1, i, 0, false, x);
-            store_out<N>(a.x, a.xpitch, a.nrhs, a.r0 + i, c, false, x);
-        }
-        __syncthreads(); // x_i is a term of the next row's dot
-    }
-}
-
-// Backward block [r0, r1) of L^T X = B, staged as the forward form (the triangle packed by columns).
-template <int N> __global__ void __launch_bounds__(64) solve_backward_staged_kernel(SolveArgs a)
-{
-    __shared__ WaveLds<N> L;
-    extern __shared__ u32 stage[];
-    const u32 c = blockIdx.x, lane = threadIdx.x, B = a.r1 - a.r0, TP = staged_tri_pitch<N>(B);
-    u32* tri = stage;
-    u32* xs = tri + (u64)(N + 3) * TP;
-    u32* rs = xs + (u64)(N + 3) * B;
-    stage_solve_block<N>(a, c, true, tri, xs, rs, lane);
-    __syncthreads();
-    const DotScratch sc{a.scratch + (u64)c * 2 * a.swords, a.swords, a.error};
-    for (u32 i = B; i-- > 0;) {
-        Num<N> v = load_out<N>(xs, B, i);
-        if (i + 1 < B) {
-            const VecView col{tri, TP, (i64)tri_col_start(B, i) + 1, 1};
-            const VecView xv{xs, B, (i64)i + 1, 1};
-            v = wave_dot_sub<N>(v, col, xv, B - i - 1, lane, L, sc);
-        }
-        if (lane == 0) {
-            u32 rv[N + 1];
-            load_recip_lds<N>(rs, B, i, rv);
-            const Num<N> x = div_by_reciprocal<N>(v, load_out<N>(tri, TP, tri_col_start(B, i)), rv);
-            store_out<N>(xs, B, 1, i, 0, false, x);
-            store_out<N>(a.x, a.xpitch, a.nrhs, a.r0 + i, c, false, x);
-        }
-        __syncthreads();
     }
 }
 

@@ -20,8 +20,30 @@ struct FactorArgs {
     FactorInfo* info;
     uint32_t* scratch; // per thread: 2 * swords words
     uint64_t swords;
-    uint32_t* recip;   // reciprocals of the pivots l_jj (N+1 planes, entry j), written by the diagonal kernel
+    uint32_t* recip;   // reciprocals of the pivots l_jj (up to N+3 planes, entry j), written by the diagonal kernel
     uint64_t rpitch;
+};
+
+// A triangular block T x = b for many right-hand sides, in place: element (r, k), k <= r, of the block at plane
+// element fbase + r*fr + k*fk, element r of right-hand side c at xbase + r*xr + c*xc, the reciprocal of diagonal
+// entry r at rbase + r*rstep.  Forward and backward solves and the rows below a Cholesky block are this one
+// recurrence with other strides.
+struct TriArgs {
+    const uint32_t* f;
+    uint64_t fpitch;
+    int64_t fbase, fr, fk;
+    uint32_t* x;
+    uint64_t xpitch;
+    int64_t xbase, xr, xc;
+    const uint32_t* recip;
+    uint64_t rpitch;
+    int64_t rbase, rstep;
+    uint32_t rows, count;  // block rows, right-hand sides
+    uint32_t* scratch;     // per right-hand side: 2 * swords words
+    uint64_t swords;
+    int32_t* error;
+    const FactorInfo* info; // not null: only the rows before a failed pivot (row 0 is column k0)
+    uint32_t k0;
 };
 
 struct SolveArgs {
@@ -33,8 +55,6 @@ struct SolveArgs {
     uint32_t* scratch;
     uint64_t swords;
     int32_t* error;
-    const uint32_t* recip; // reciprocals of the diagonal l_ii (N+1 planes, entry i), from launch_reciprocals
-    uint64_t rpitch;
 };
 
 // Window words of the register path of the exact dot: 2N product words plus 24 words (768 bits) of
@@ -56,17 +76,18 @@ template <int N> hipError_t launch_chol_diag(const FactorArgs& f, uint32_t threa
 template <int N>
 hipError_t launch_factor_steps(const uint32_t* v, uint64_t pitch, uint32_t* scratch, uint64_t swords, int32_t* err, int reps, uint64_t* out,
                                uint32_t* sink, hipStream_t s);
-template <int N> hipError_t launch_chol_panel(const FactorArgs& f, hipStream_t s);
+// T x = b of one block for every right-hand side
+template <int N> hipError_t launch_tri_block(const TriArgs& g, hipStream_t s);
 // entries (i, j), j <= i, of columns [k1, k2) and rows [k1, n) updated by the block [k0, k1); at most
 // `waves` wavefronts (scratch slots)
 template <int N> hipError_t launch_chol_lookahead(const FactorArgs& f, uint32_t k2, uint32_t waves, hipStream_t s);
 template <int N> hipError_t launch_chol_invalid(uint32_t* w, uint64_t pitch, uint32_t n, uint32_t p, hipStream_t s);
 template <int N> hipError_t launch_zero_upper(uint32_t* w, uint64_t pitch, uint32_t n, hipStream_t s);
-template <int N> hipError_t launch_solve(int backward, const SolveArgs& a, hipStream_t s);
 // the off-block update of block [r0, r1) by exact dots (rows [r1, n) forward, [0, r0) backward); at most
 // `waves` wavefronts (scratch slots)
 template <int N> hipError_t launch_solve_update(int backward, const SolveArgs& a, uint32_t waves, hipStream_t s);
-// recip entry i = reciprocal of the mantissa of the diagonal element (i, i) of the n x n planes, i < n
+// recip entry i = reciprocal of the mantissa of the diagonal element (i, i) of the n x n planes, i < n (up to
+// N+3 planes)
 template <int N> hipError_t launch_reciprocals(const uint32_t* w, uint64_t pitch, uint32_t n, uint32_t* recip, uint64_t rpitch, hipStream_t s);
 
 } // namespace lf

@@ -18,10 +18,10 @@ template <int N> hipError_t launch_chol_diag(const FactorArgs& f, uint32_t threa
     return hipGetLastError();
 }
 
-template <int N> hipError_t launch_chol_panel(const FactorArgs& f, hipStream_t s)
+template <int N> hipError_t launch_tri_block(const TriArgs& g, hipStream_t s)
 {
-    if (f.k1 >= f.n) return hipSuccess;
-    hipLaunchKernelGGL((chol_panel_kernel<N>), dim3(f.n - f.k1), dim3(WAVE), 0, s, f);
+    if (!g.count || !g.rows) return hipSuccess;
+    hipLaunchKernelGGL((tri_block_kernel<N>), dim3(g.count), dim3(WAVE), 0, s, g);
     return hipGetLastError();
 }
 
@@ -46,24 +46,6 @@ template <int N> hipError_t launch_zero_upper(uint32_t* w, uint64_t pitch, uint3
     const uint64_t total = (uint64_t)n * n;
     if (!total) return hipSuccess;
     hipLaunchKernelGGL((zero_upper_kernel<N>), dim3((unsigned)((total + 255u) / 256u)), dim3(256), 0, s, w, pitch, n);
-    return hipGetLastError();
-}
-
-template <int N> hipError_t launch_solve(int backward, const SolveArgs& a, hipStream_t s)
-{
-    if (!a.nrhs || a.r1 <= a.r0) return hipSuccess;
-    const dim3 grid(a.nrhs), block(WAVE);
-    // blocks of up to STAGED_ROWS rows whose staged copy fits 64 KB of LDS beside the exact-dot rows run
-    // from LDS; larger blocks and wider values read global memory
-    const uint32_t B = a.r1 - a.r0;
-    const uint64_t dyn = staged_words<N>(B) * 4;
-    if (B <= STAGED_ROWS && dyn + sizeof(WaveLds<N>) <= (uint64_t(64) << 10)) {
-        if (backward) hipLaunchKernelGGL((solve_backward_staged_kernel<N>), grid, block, (unsigned)dyn, s, a);
-        else hipLaunchKernelGGL((solve_forward_staged_kernel<N>), grid, block, (unsigned)dyn, s, a);
-        return hipGetLastError();
-    }
-    if (backward) hipLaunchKernelGGL((solve_backward_kernel<N>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((solve_forward_kernel<N>), grid, block, 0, s, a);
     return hipGetLastError();
 }
 
@@ -98,11 +80,10 @@ hipError_t launch_factor_steps(const uint32_t* v, uint64_t pitch, uint32_t* scra
 
 template hipError_t launch_chol_diag<LF_WORDS>(const FactorArgs&, uint32_t, hipStream_t);
 template hipError_t launch_factor_steps<LF_WORDS>(const uint32_t*, uint64_t, uint32_t*, uint64_t, int32_t*, int, uint64_t*, uint32_t*, hipStream_t);
-template hipError_t launch_chol_panel<LF_WORDS>(const FactorArgs&, hipStream_t);
+template hipError_t launch_tri_block<LF_WORDS>(const TriArgs&, hipStream_t);
 template hipError_t launch_chol_lookahead<LF_WORDS>(const FactorArgs&, uint32_t, uint32_t, hipStream_t);
 template hipError_t launch_chol_invalid<LF_WORDS>(uint32_t*, uint64_t, uint32_t, uint32_t, hipStream_t);
 template hipError_t launch_zero_upper<LF_WORDS>(uint32_t*, uint64_t, uint32_t, hipStream_t);
-template hipError_t launch_solve<LF_WORDS>(int, const SolveArgs&, hipStream_t);
 template hipError_t launch_solve_update<LF_WORDS>(int, const SolveArgs&, uint32_t, hipStream_t);
 template hipError_t launch_reciprocals<LF_WORDS>(const uint32_t*, uint64_t, uint32_t, uint32_t*, uint64_t, hipStream_t);
 

@@ -1,0 +1,51 @@
+"""The digit-per-lane block kernels of the factorization and the solves (limbforge_amd/csrc/factor_wave.hpp) at
+their edges, bit for bit against the oracle: the smallest and widest precisions they take and the first one
+past them, a precision whose mantissa fills whole digits (416 bits), mantissas that are all ones or a power
+of two (rounding carries, exact sums), zero entries and right-hand sides, negative diagonals, exponent spreads
+inside, across and past the accumulators' columns, statuses, and blocks at and around 32 rows."""
+import numpy as np
+import pytest
+
+import lfcases
+
+pytestmark = pytest.mark.gpu
+
+BITS = [64, 96, 256, 416, 512, 640, 672]
+
+
+def special_mantissas(rng, x, bits):
+    """A fifth of the values all ones, a fifth powers of two, a fifth one unit above one."""
+    w = bits // 32
+    pick = rng.integers(0, 5, size=x.shape[0])
+    x[pick == 0, :w] = 0xFFFFFFFF
+    x[(pick == 1) | (pick == 2), :w] = 0
+    x[(pick == 1) | (pick == 2), w - 1] = 0x80000000
+    x[pick == 2, 0] |= 1
+    return x
+
+
+def triangle(rng, bits, n, span):
+    L = special_mantissas(rng, lfcases.random_records(rng, bits, n * n, span), bits)
+    L[rng.random(n * n) < 0.2] = lfcases.zero(bits)
+    d = np.arange(n) * (n + 1)
+    L[d] = special_mantissas(rng, lfcases.random_records(rng, bits, n, span // 2), bits)
+    return L
+
+
+@pytest.mark.parametrize("bits", BITS)
+@pytest.mark.parametrize("span", [0, 30, 200, 1500])
+def test_triangular_solves(capi, oracle, bits, span):
+    rng = np.random.default_rng(bits + 7 * span)
+    for n, nrhs, block in ((1, 1, 32), (31, 2, 32), (32, 3, 32), (33, 1, 32), (70, 5, 32), (40, 2, 7), (35, 2, 33)):
+        print(f"[gpu] solve bits={bits} span={span} n={n} nrhs={nrhs} block={block}", flush=True)
+        L = triangle(rng, bits, n, span)
+        B = special_mantissas(rng, lfcases.random_records(rng, bits, n * nrhs, span), bits)
+        B[rng.random(n * nrhs) < 0.2] = lfcases.zero(bits)
+        if n == 33:  # a status in the second block, a zero on the diagonal of the first
+            B[32 * nrhs, bits // 32 + 2] = 4
+            L[5 * (n + 1)] = lfcases.zero(bits)
+        for passes in (1, 2):
+            want = oracle.solve(bits, L, n, B, nrhs, block, passes)
+            got, _, _ = capi.solve(bits, passes, L, n, B, nrhs, block=block)
+            bad = np.nonzero((got != want).any(axis=1))[0]
+            assert bad.size == 0, f"n={n} passes={passes}: {bad.size} entries differ, first row {bad[0] // nrhs}"
