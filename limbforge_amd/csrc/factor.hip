@@ -3,7 +3,8 @@
 // src/linalg.mm:411-486, docs/numerics.md:674-748).
 //
 // The work matrix stays in limb planes on the device for the whole call.  Per column block [k0, k1):
-//   1. the diagonal block, column by column in one workgroup (pivot, sqrt, then div of the entries below);
+//   1. the diagonal block, column by column in one workgroup (chol_diag_wave_kernel, and chol_diag_kernel for
+//      what it leaves);
 //   2. the rows below it, one wavefront per row (tri_block_kernel);
 //   3. the trailing update a_ij = D(a_ij; l_i, l_j; [k0, k1)) for i >= j >= k1, in two parts as the
 //      reference splits it (linalg.mm:440-452): the next panel's columns [k1, k2) by the look-ahead kernel
@@ -243,7 +244,7 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
         }
     } hinfo;
     FACTOR_HIP(hipHostMalloc((void**)&hinfo.p, sizeof(lf::FactorInfo), hipHostMallocDefault), "hipHostMalloc (pivot)");
-    *hinfo.p = lf::FactorInfo{-1, 0, 0, 0};
+    *hinfo.p = lf::FactorInfo{-1, 0, 0, 0, 0};
     FACTOR_HIP(hipMemcpyAsync(dinfo.p, hinfo.p, sizeof(lf::FactorInfo), hipMemcpyHostToDevice, s), "upload pivot");
     // Look-ahead (the reference overlaps the next panel with the rest of the update on a second host thread,
     // linalg.mm:440-452): after the panel of block [k0, k1), the entries of the next panel's columns

@@ -531,6 +531,7 @@ __device__ Num<N> wave_dot_sub(const Num<N>& c, const VecView& x, const VecView&
 
 } // namespace lf
 #include "factor_wave.hpp"
+#include "factor_diag.hpp"
 namespace lf {
 
 // ---------------------------------------------------------------- Cholesky
@@ -573,8 +574,9 @@ template <int N> constexpr int diag_waves()
 // (lane 0) while the other waves form the numerators D(a_ij; l_i, l_j; [k0, j)) of the rows below, one
 // row per wave at a time, written in place (they read only columns before j); (B) one thread per row
 // divides its numerator by l_jj.  Stops at a failing pivot, before any entry of its column is written
-// (numerators of the rows below included: phase B is never reached).
-template <int N> __global__ void __launch_bounds__(diag_waves<N>() * WAVE) chol_diag_kernel(FactorArgs f)
+// (numerators of the rows below included: phase B is never reached).  With `resume` it starts at the first
+// column that chol_diag_wave_kernel left.
+template <int N> __global__ void __launch_bounds__(diag_waves<N>() * WAVE) chol_diag_kernel(FactorArgs f, u32 resume)
 {
     constexpr int DW = diag_waves<N>();
     __shared__ WaveLds<N> lds[DW];
@@ -582,7 +584,7 @@ template <int N> __global__ void __launch_bounds__(diag_waves<N>() * WAVE) chol_
     const u32 wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     WaveLds<N>& L = lds[wave];
     const DotScratch sc{f.scratch + (u64)wave * 2 * f.swords, f.swords, &f.info->error};
-    for (u32 j = f.k0; j < f.k1; ++j) {
+    for (u32 j = f.k0 + (resume ? (u32)f.info->resume : 0u); j < f.k1; ++j) {
         const VecView rj{f.w, f.pitch, (i64)j * f.n + f.k0, 1};
         if (wave == 0) {
             const Num<N> s = wave_dot_sub<N>(element<N>(f, j, j), rj, rj, j - f.k0, lane, L, sc);

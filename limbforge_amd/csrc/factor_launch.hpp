@@ -11,6 +11,7 @@ struct FactorInfo {
     int32_t sign;    // sign of the failing s_pp (0 for zero or a status)
     uint32_t status; // its status
     int32_t error;   // cluster scratch overflow (never expected)
+    int32_t resume;  // columns of the block that the wave-parallel diagonal kernel decided
 };
 
 struct FactorArgs {

@@ -14,7 +14,14 @@ template <int N> hipError_t launch_chol_diag(const FactorArgs& f, uint32_t threa
 {
     (void)threads;
     if (f.k1 <= f.k0) return hipSuccess;
-    hipLaunchKernelGGL((chol_diag_kernel<N>), dim3(1), dim3(diag_waves<N>() * WAVE), 0, s, f);
+    uint32_t resume = 0;
+    if constexpr (wd_fits<N>())
+        if (f.k1 - f.k0 <= WD_ROWS) { // what it leaves, usually nothing, is the general kernel's
+            hipLaunchKernelGGL((chol_diag_wave_kernel<N>), dim3(1), dim3(DIAG_WAVES * WAVE), 0, s, f);
+            if (hipError_t e = hipGetLastError()) return e;
+            resume = 1;
+        }
+    hipLaunchKernelGGL((chol_diag_kernel<N>), dim3(1), dim3(diag_waves<N>() * WAVE), 0, s, f, resume);
     return hipGetLastError();
 }
 

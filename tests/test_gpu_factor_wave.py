@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import lfcases
+from factor_cases import spd
 
 pytestmark = pytest.mark.gpu
 
@@ -49,3 +50,39 @@ def test_triangular_solves(capi, oracle, bits, span):
             got, _, _ = capi.solve(bits, passes, L, n, B, nrhs, block=block)
             bad = np.nonzero((got != want).any(axis=1))[0]
             assert bad.size == 0, f"n={n} passes={passes}: {bad.size} entries differ, first row {bad[0] // nrhs}"
+
+
+@pytest.mark.parametrize("bits", BITS)
+@pytest.mark.parametrize("kind", ["moderate", "graded", "wide", "banded", "spread"])
+def test_factorizations(capi, oracle, bits, kind):
+    """Blocks of 32, 31, 1 and 5 columns; zero entries with fill (banded), spreads past the columns (spread)."""
+    rng = np.random.default_rng(3 * bits + len(kind))
+    for n, block in ((1, 32), (2, 32), (31, 32), (65, 32), (33, 5)):
+        print(f"[gpu] cholesky bits={bits} {kind} n={n} block={block}", flush=True)
+        A = spd(oracle, rng, bits, n, kind)
+        want, piv, psign, pstat = oracle.cholesky(bits, A, n, block)
+        got, info = capi.cholesky(bits, A, n, block=block)
+        assert (info.pivot, info.pivot_sign, info.pivot_status) == (piv, psign, pstat)
+        bad = np.nonzero((got != want).any(axis=1))[0]
+        assert bad.size == 0, f"n={n} block={block}: {bad.size} entries differ, first ({bad[0] // n},{bad[0] % n})"
+
+
+@pytest.mark.parametrize("bits", [64, 256, 640])
+def test_squares_of_short_factors(capi, oracle, bits):
+    """A = L0 L0^T exactly, L0 of few-bit integers: every sum, root and quotient is exact."""
+    rng = np.random.default_rng(bits)
+    n, w = 34, bits // 32
+    L0 = np.tril(rng.integers(-7, 8, size=(n, n)))
+    L0[np.arange(n), np.arange(n)] = rng.integers(1, 9, size=n)
+    V = L0 @ L0.T
+    A = np.zeros((n * n, w + 3), np.uint32)
+    for k, v in enumerate(V.reshape(-1)):
+        if v:
+            e = int(abs(v)).bit_length() - 1
+            A[k, w - 1] = (int(abs(v)) << (31 - e)) & 0xFFFFFFFF
+            A[k, w] = e
+            A[k, w + 1] = lfcases.i32(1 if v > 0 else -1)
+    want, piv, _, _ = oracle.cholesky(bits, A, n, 32)
+    got, info = capi.cholesky(bits, A, n, block=32)
+    assert info.pivot == piv == n
+    assert (got == want).all()
