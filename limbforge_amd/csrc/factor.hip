@@ -66,9 +66,8 @@ struct OwnedStream {
 
 typedef hipError_t (*diag_fn)(const lf::FactorArgs&, uint32_t, hipStream_t);
 typedef hipError_t (*tri_fn)(const lf::TriArgs&, hipStream_t);
-typedef hipError_t (*lookahead_fn)(const lf::FactorArgs&, uint32_t, uint32_t, hipStream_t);
+typedef hipError_t (*update_fn)(const lf::UpdateArgs&, uint32_t, hipStream_t);
 typedef hipError_t (*invalid_fn)(uint32_t*, uint64_t, uint32_t, uint32_t, hipStream_t);
-typedef hipError_t (*solve_update_fn)(int, const lf::SolveArgs&, uint32_t, hipStream_t);
 typedef hipError_t (*recip_fn)(const uint32_t*, uint64_t, uint32_t, uint32_t*, uint64_t, hipStream_t);
 typedef hipError_t (*steps_fn)(const uint32_t*, uint64_t, uint32_t*, uint64_t, int32_t*, int, uint64_t*, uint32_t*, hipStream_t);
 struct FactorTables;
@@ -76,10 +75,9 @@ template <int N> void fill_factor(FactorTables& t);
 struct FactorTables {
     diag_fn diag[33] = {};
     tri_fn tri_block[33] = {};
-    lookahead_fn lookahead[33] = {};
+    update_fn update[33] = {};
     invalid_fn invalid[33] = {};
     hipError_t (*zero_upper[33])(uint32_t*, uint64_t, uint32_t, hipStream_t) = {};
-    solve_update_fn solve_update[33] = {};
     recip_fn reciprocals[33] = {};
     steps_fn steps[33] = {};
     FactorTables() { fill_factor<2>(*this); }
@@ -88,10 +86,9 @@ template <int N> void fill_factor(FactorTables& t)
 {
     t.diag[N] = lf::launch_chol_diag<N>;
     t.tri_block[N] = lf::launch_tri_block<N>;
-    t.lookahead[N] = lf::launch_chol_lookahead<N>;
+    t.update[N] = lf::launch_update<N>;
     t.invalid[N] = lf::launch_chol_invalid<N>;
     t.zero_upper[N] = lf::launch_zero_upper<N>;
-    t.solve_update[N] = lf::launch_solve_update<N>;
     t.reciprocals[N] = lf::launch_reciprocals<N>;
     t.steps[N] = lf::launch_factor_steps<N>;
     if constexpr (N < 32) fill_factor<N + 1>(t);
@@ -174,10 +171,12 @@ int update(int bits, const lf_linalg_options& o, bool syrk, const lf::MatView& l
 
 double since(Clock::time_point t) { return std::chrono::duration<double>(Clock::now() - t).count(); }
 
+// wavefronts (and scratch slots) of a look-ahead update: four for each of 256 tiles
+constexpr uint64_t LOOKAHEAD_WAVES = 1024;
 // wavefronts (and scratch slots) of a direct off-block solve update
 constexpr uint64_t SOLVE_UPDATE_WAVES = 2048;
 // Off-block solve updates of up to this many multiply-add terms (rows x right-hand sides x block) also run
-// as direct exact dots: on 2048 wavefronts 2^22 terms of 256 bits take about 50 us, less than one update
+// as direct exact dots: on 2048 wavefronts 2^20 terms of 256 bits take about 30 us, less than one update
 // GEMM's planning round trip (band analysis, line-table download, constants, about 0.4 ms of host time per
 // update at n = 512 with 64 right-hand sides).  Both forms round the same exact value once.
 constexpr double SOLVE_DIRECT_TERMS = 4194304.0;
@@ -226,7 +225,8 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
     // pivot record and per-thread cluster scratch (rows of a panel, or the diagonal block's threads)
     DevBuf dinfo, dscratch;
     const uint64_t swords = lf::factor_scratch_words(N, nb);
-    const uint64_t threads = std::max<uint64_t>(n, 256);
+    // one slot a row of a panel, and those of the look-ahead update's wavefronts
+    const uint64_t threads = std::max<uint64_t>(n, LOOKAHEAD_WAVES);
     if (2 * swords * threads * 4 > (uint64_t(32) << 30))
         return fail(LF_INVALID_ARGUMENT, "cholesky: the block is too large for the exact-dot scratch (use a smaller block)");
     FACTOR_HIP(dinfo.alloc(sizeof(lf::FactorInfo)), "hipMalloc (pivot)");
@@ -325,7 +325,11 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
         auto t = Clock::now();
         if (rest_pending) FACTOR_HIP(hipStreamWaitEvent(s, rest_done, 0), "hipStreamWaitEvent");
         FACTOR_HIP(hipEventRecord(l0, s), "hipEventRecord");
-        FACTOR_HIP(tables().lookahead[N](args(k0, k1), uint32_t(k2), waves, s), "look-ahead launch");
+        // the entries (i, j), j <= i, of columns [k1, k2) and rows [k1, n), in place
+        const lf::UpdateArgs ua{W, pitch, int64_t(k1 * n + k0), int64_t(n), 1, W, pitch, int64_t(k1 * n + k0), int64_t(n), 1, W, pitch,
+                                int64_t(k1 * n + k1), int64_t(n), 1, uint32_t(n - k1), uint32_t(k2 - k1), uint32_t(w), 1, (uint32_t*)dscratch.p, swords,
+                                &((lf::FactorInfo*)dinfo.p)->error};
+        FACTOR_HIP(tables().update[N](ua, waves, s), "look-ahead launch");
         FACTOR_HIP(hipEventRecord(l1, s), "hipEventRecord");
         // (2) the next panel on s
         const auto tp = Clock::now();
@@ -439,10 +443,14 @@ int lf_solve(int bits, int passes, const lf_operand* L, uint64_t n, const lf_ope
         const double terms = double(rows) * double(nrhs) * double(K);
         return fo.solve_host_macs >= 0 && (terms < fo.solve_host_macs || terms <= SOLVE_DIRECT_TERMS);
     };
+    // rows [r1, n) by row i of L going forward, rows [0, r0) by column i of L going backward
     auto dot_update = [&](int backward, uint64_t r0, uint64_t r1) {
-        lf::SolveArgs a{F, fpitch, Xp, xpitch, uint32_t(n), uint32_t(nrhs), uint32_t(r0), uint32_t(r1), (uint32_t*)dscratch.p, swords,
-                        (int32_t*)derr.p};
-        return timed([&] { return tables().solve_update[N](backward, a, uint32_t(slots), s); });
+        const uint64_t row0 = backward ? 0 : r1;
+        const lf::UpdateArgs ua{F, fpitch, backward ? int64_t(r0 * n) : int64_t(r1 * n + r0), backward ? 1 : int64_t(n), backward ? int64_t(n) : 1, Xp,
+                                xpitch, int64_t(r0 * nrhs), 1, int64_t(nrhs), Xp, xpitch, int64_t(row0 * nrhs), int64_t(nrhs), 1,
+                                uint32_t(backward ? r0 : n - r1), uint32_t(nrhs), uint32_t(r1 - r0), 0, (uint32_t*)dscratch.p, swords,
+                                (int32_t*)derr.p};
+        return timed([&] { return tables().update[N](ua, uint32_t(slots), s); });
     };
     if (passes & 1)
         for (uint64_t r0 = 0; r0 < n; r0 += nb) {

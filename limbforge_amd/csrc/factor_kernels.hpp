@@ -532,6 +532,7 @@ __device__ Num<N> wave_dot_sub(const Num<N>& c, const VecView& x, const VecView&
 } // namespace lf
 #include "factor_wave.hpp"
 #include "factor_diag.hpp"
+#include "factor_update.hpp"
 namespace lf {
 
 // ---------------------------------------------------------------- Cholesky
@@ -618,27 +619,6 @@ template <int N> __global__ void __launch_bounds__(diag_waves<N>() * WAVE) chol_
     }
 }
 
-// Look-ahead part of a block's trailing update: after the panel [k0, k1), the entries (i, j), j <= i, of the
-// next panel's columns j in [k1, k2) and rows i in [k1, n) become D(a_ij; l_i, l_j; [k0, k1)) in place -- the
-// same one rounding of the same exact value as the update product gives them -- so that the next panel can
-// start while the rest of the update (rows and columns from k2) runs on another stream.  One wavefront per
-// entry, grid-stride over the (n - k1) x (k2 - k1) rectangle; wavefront b uses scratch slot b.
-template <int N> __global__ void __launch_bounds__(64) chol_lookahead_kernel(FactorArgs f, u32 k2)
-{
-    __shared__ WaveLds<N> L;
-    const u32 lane = threadIdx.x, cols = k2 - f.k1;
-    const u64 entries = (u64)(f.n - f.k1) * cols;
-    const DotScratch sc{f.scratch + (u64)blockIdx.x * 2 * f.swords, f.swords, &f.info->error};
-    for (u64 e = blockIdx.x; e < entries; e += gridDim.x) {
-        const u32 i = f.k1 + (u32)(e / cols), j = f.k1 + (u32)(e % cols);
-        if (j > i) continue; // the whole wavefront skips the strict upper part
-        const VecView ri{f.w, f.pitch, (i64)i * f.n + f.k0, 1};
-        const VecView rj{f.w, f.pitch, (i64)j * f.n + f.k0, 1};
-        const Num<N> v = wave_dot_sub<N>(element<N>(f, i, j), ri, rj, f.k1 - f.k0, lane, L, sc);
-        if (lane == 0) store_out<N>(f.w, f.pitch, f.n, i, j, false, v);
-    }
-}
-
 // Entries (i, j) with i >= j >= p after a failing pivot p: zero with status invalid.  Thread per entry of
 // the trailing (n-p) x (n-p) square.
 template <int N> __global__ void __launch_bounds__(256) chol_invalid_kernel(u32* w, u64 pitch, u32 n, u32 p)
@@ -694,26 +674,6 @@ template <int N> __global__ void __launch_bounds__(64) tri_block_kernel(TriArgs 
             store_out<N>(g.x, g.xpitch, 0, 0, (u32)at, false, div_by_reciprocal<N>(v, l, rv));
         }
         __syncthreads(); // x_i is a term of the next row's dot
-    }
-}
-
-// Off-block update of a solve by the block [r0, r1), for updates too small to pay for the update GEMM's
-// planning: x_ic = D(x_ic; l, x_c; [r0, r1)) with l = row i of L (forward, rows i in [r1, n)) or column i of L
-// (backward, rows i in [0, r0)), one wavefront per entry, grid-stride over the rows x nrhs entries; wavefront
-// b uses scratch slot b.  The same one rounding of the same exact value as the update product.
-template <int N> __global__ void __launch_bounds__(64) solve_update_kernel(SolveArgs a, u32 backward)
-{
-    __shared__ WaveLds<N> L;
-    const u32 lane = threadIdx.x;
-    const u32 row0 = backward ? 0u : a.r1, rows = backward ? a.r0 : a.n - a.r1;
-    const u64 entries = (u64)rows * a.nrhs;
-    const DotScratch sc{a.scratch + (u64)blockIdx.x * 2 * a.swords, a.swords, a.error};
-    for (u64 e = blockIdx.x; e < entries; e += gridDim.x) {
-        const u32 i = row0 + (u32)(e / a.nrhs), c = (u32)(e % a.nrhs);
-        const VecView l = backward ? VecView{a.f, a.fpitch, (i64)a.r0 * a.n + i, (i64)a.n} : VecView{a.f, a.fpitch, (i64)i * a.n + a.r0, 1};
-        const VecView xc{a.x, a.xpitch, (i64)a.r0 * a.nrhs + c, (i64)a.nrhs};
-        const Num<N> v = wave_dot_sub<N>(load_out<N>(a.x, a.xpitch, (u64)i * a.nrhs + c), l, xc, a.r1 - a.r0, lane, L, sc);
-        if (lane == 0) store_out<N>(a.x, a.xpitch, a.nrhs, i, c, false, v);
     }
 }
 

@@ -47,13 +47,21 @@ struct TriArgs {
     uint32_t k0;
 };
 
-struct SolveArgs {
-    const uint32_t* f; // factor planes (n x n)
-    uint64_t fpitch;
-    uint32_t* x;       // right-hand sides / solution planes (n x nrhs)
+// Off-block update out_ic = D(out_ic; x_i, y_c; K) of rows x cols entries in place: element k of line x_i at
+// xbase + i*xr + k*xk, of line y_c at ybase + c*yc + k*yk, entry (i, c) at obase + i*orow + c*ocol; with `lower` the
+// entries c <= i alone.
+struct UpdateArgs {
+    const uint32_t* x;
     uint64_t xpitch;
-    uint32_t n, nrhs, r0, r1;
-    uint32_t* scratch;
+    int64_t xbase, xr, xk;
+    const uint32_t* y;
+    uint64_t ypitch;
+    int64_t ybase, yc, yk;
+    uint32_t* out;
+    uint64_t opitch;
+    int64_t obase, orow, ocol;
+    uint32_t rows, cols, K, lower;
+    uint32_t* scratch; // 2 * swords words per wavefront
     uint64_t swords;
     int32_t* error;
 };
@@ -79,14 +87,10 @@ hipError_t launch_factor_steps(const uint32_t* v, uint64_t pitch, uint32_t* scra
                                uint32_t* sink, hipStream_t s);
 // T x = b of one block for every right-hand side
 template <int N> hipError_t launch_tri_block(const TriArgs& g, hipStream_t s);
-// entries (i, j), j <= i, of columns [k1, k2) and rows [k1, n) updated by the block [k0, k1); at most
-// `waves` wavefronts (scratch slots)
-template <int N> hipError_t launch_chol_lookahead(const FactorArgs& f, uint32_t k2, uint32_t waves, hipStream_t s);
+// at most `waves` wavefronts (scratch slots)
+template <int N> hipError_t launch_update(const UpdateArgs& g, uint32_t waves, hipStream_t s);
 template <int N> hipError_t launch_chol_invalid(uint32_t* w, uint64_t pitch, uint32_t n, uint32_t p, hipStream_t s);
 template <int N> hipError_t launch_zero_upper(uint32_t* w, uint64_t pitch, uint32_t n, hipStream_t s);
-// the off-block update of block [r0, r1) by exact dots (rows [r1, n) forward, [0, r0) backward); at most
-// `waves` wavefronts (scratch slots)
-template <int N> hipError_t launch_solve_update(int backward, const SolveArgs& a, uint32_t waves, hipStream_t s);
 // recip entry i = reciprocal of the mantissa of the diagonal element (i, i) of the n x n planes, i < n (up to
 // N+3 planes)
 template <int N> hipError_t launch_reciprocals(const uint32_t* w, uint64_t pitch, uint32_t n, uint32_t* recip, uint64_t rpitch, hipStream_t s);

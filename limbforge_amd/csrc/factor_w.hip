@@ -32,11 +32,17 @@ template <int N> hipError_t launch_tri_block(const TriArgs& g, hipStream_t s)
     return hipGetLastError();
 }
 
-template <int N> hipError_t launch_chol_lookahead(const FactorArgs& f, uint32_t k2, uint32_t waves, hipStream_t s)
+template <int N> hipError_t launch_update(const UpdateArgs& g, uint32_t waves, hipStream_t s)
 {
-    if (f.k1 >= f.n || k2 <= f.k1 || !waves) return hipSuccess;
-    const uint64_t entries = (uint64_t)(f.n - f.k1) * (k2 - f.k1);
-    hipLaunchKernelGGL((chol_lookahead_kernel<N>), dim3((unsigned)std::min<uint64_t>(entries, waves)), dim3(WAVE), 0, s, f, k2);
+    if (!g.rows || !g.cols || !waves) return hipSuccess;
+    if constexpr (wd_fits<N>())
+        if (g.K <= WD_ROWS && waves >= UPD_WAVES) {
+            const uint32_t tc = upd_cols(g.cols), tr = upd_rows(tc);
+            const uint64_t tiles = (uint64_t)((g.rows + tr - 1) / tr) * ((g.cols + tc - 1) / tc);
+            hipLaunchKernelGGL((update_wave_kernel<N>), dim3((unsigned)std::min<uint64_t>(tiles, waves / UPD_WAVES)), dim3(64 * UPD_WAVES), 0, s, g);
+            return hipGetLastError();
+        }
+    hipLaunchKernelGGL((update_kernel<N>), dim3((unsigned)std::min<uint64_t>((uint64_t)g.rows * g.cols, waves)), dim3(WAVE), 0, s, g);
     return hipGetLastError();
 }
 
@@ -53,16 +59,6 @@ template <int N> hipError_t launch_zero_upper(uint32_t* w, uint64_t pitch, uint3
     const uint64_t total = (uint64_t)n * n;
     if (!total) return hipSuccess;
     hipLaunchKernelGGL((zero_upper_kernel<N>), dim3((unsigned)((total + 255u) / 256u)), dim3(256), 0, s, w, pitch, n);
-    return hipGetLastError();
-}
-
-template <int N> hipError_t launch_solve_update(int backward, const SolveArgs& a, uint32_t waves, hipStream_t s)
-{
-    const uint64_t rows = backward ? a.r0 : a.n - a.r1;
-    if (!a.nrhs || !rows || a.r1 <= a.r0 || !waves) return hipSuccess;
-    const uint64_t entries = rows * a.nrhs;
-    hipLaunchKernelGGL((solve_update_kernel<N>), dim3((unsigned)std::min<uint64_t>(entries, waves)), dim3(WAVE), 0, s, a,
-                       backward ? 1u : 0u);
     return hipGetLastError();
 }
 
@@ -88,10 +84,9 @@ hipError_t launch_factor_steps(const uint32_t* v, uint64_t pitch, uint32_t* scra
 template hipError_t launch_chol_diag<LF_WORDS>(const FactorArgs&, uint32_t, hipStream_t);
 template hipError_t launch_factor_steps<LF_WORDS>(const uint32_t*, uint64_t, uint32_t*, uint64_t, int32_t*, int, uint64_t*, uint32_t*, hipStream_t);
 template hipError_t launch_tri_block<LF_WORDS>(const TriArgs&, hipStream_t);
-template hipError_t launch_chol_lookahead<LF_WORDS>(const FactorArgs&, uint32_t, uint32_t, hipStream_t);
+template hipError_t launch_update<LF_WORDS>(const UpdateArgs&, uint32_t, hipStream_t);
 template hipError_t launch_chol_invalid<LF_WORDS>(uint32_t*, uint64_t, uint32_t, uint32_t, hipStream_t);
 template hipError_t launch_zero_upper<LF_WORDS>(uint32_t*, uint64_t, uint32_t, hipStream_t);
-template hipError_t launch_solve_update<LF_WORDS>(int, const SolveArgs&, uint32_t, hipStream_t);
 template hipError_t launch_reciprocals<LF_WORDS>(const uint32_t*, uint64_t, uint32_t, uint32_t*, uint64_t, hipStream_t);
 
 } // namespace lf
