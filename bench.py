@@ -238,13 +238,14 @@ def gemm_section(reps: int, oracle_samples: int, cpu_budget: float, peak_tps: fl
         check = {"rows": len(rows), "outputs": len(rows) * n, "mismatches": int((got != want).any(axis=1).sum())}
     # roofline of the dominant kernel, the int8-MFMA residue product: 4 int8 products (d1 d1, d1 d0, d0 d1,
     # d0 d0) of 2 ops each per modulus, extended row, extended column and K step, as launched (padded K)
-    rr = reports["residue"]
+    # (of the band_bits = 512 run, whose one band per line is also the plan that the default options run here)
+    rr = reports["residue_band512"]
     kp = max(64, (n + 63) // 64 * 64)
     ops = 8 * rr.moduli * rr.gemm_rows * rr.gemm_cols * kp
-    prod_s = res["residue"]["stages"]["product_ms"] * 1e-3
+    prod_s = res["residue_band512"]["stages"]["product_ms"] * 1e-3
     roof = {"bound": "mfma", "achieved": round(ops / prod_s / 1e12, 2), "peak": MFMA_INT8_PEAK / 1e12, "unit": "Tops/s (int8)",
             "frac": round(ops / prod_s / MFMA_INT8_PEAK, 4), "traffic": None, "kernel": "product_kernel (v_mfma_i32_32x32x32_i8)",
-            "kernel_ms": res["residue"]["stages"]["product_ms"], "int8_ops": int(ops)}
+            "kernel_ms": res["residue_band512"]["stages"]["product_ms"], "int8_ops": int(ops)}
     limb_wp = n * n * n * (bits // 32) ** 2
     limb_s = res["limb"]["device_ms"] * 1e-3
     limb_roof = {"bound": "valu", "achieved": round(limb_wp / limb_s / 1e12, 3), "unit": "Tword-products/s",
@@ -563,7 +564,9 @@ def cholesky_section(oracle_check: bool):
     ratio, _, _ = capi.run_host(bits, "div", absval(r), scale)
     res["scaled_residual"] = max(abs(to_float(q, bits)) for q in ratio)
     log(f"[bench] cholesky: {res}")
-    # roofline of the SYRK's int8-MFMA residue product (lower-triangle tiles only)
+    # roofline of the SYRK's int8-MFMA residue product (lower-triangle tiles only), of a run whose lines are one band
+    # each by option (the default options join the few lines of two bands)
+    srep = capi.syrk(bits, A, rows, n, lower_only=False, options=capi.LinalgOptions.default(band_bits=512))[1]
     kp = (rows + 63) // 64 * 64
     tiles = (srep.gemm_rows + 127) // 128
     ops = 8 * srep.moduli * 128 * 128 * (tiles * (tiles + 1) // 2) * kp

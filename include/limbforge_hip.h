@@ -193,7 +193,10 @@ typedef struct lf_linalg_pair {
 /* LinalgReport (linalg.hpp:33-45): band histograms per side ([b] = lines with exactly b bands; index 0:
  * zero or status lines; band_slots = max_bands + 1 entries, at most 65), fallback lines and outputs,
  * band pairs (first 64), extended GEMM sizes, moduli and int8 GEMMs (three per modulus), stage times
- * (host analysis, uploads, device time, assembly, and the device time per kernel stage). */
+ * (host analysis, uploads, device time, assembly, and the device time per kernel stage).  Bands, pairs,
+ * sizes and moduli are those of the reference's rule (greedy bands of band_bits).  Where it costs less, the
+ * product runs with each line's bands joined into one band from its lowest exponent: more moduli, no band pairs,
+ * the same outputs; the times are of what ran. */
 typedef struct lf_linalg_report {
     uint64_t m, n, k;
     uint32_t band_slots;

@@ -12,7 +12,6 @@
 #include "gemm_kernels.hpp"
 #include "gemm_launch.hpp"
 #include "gemm_plan.hpp"
-#include "residue_reduce.hpp"
 #include "host_copy.hpp"
 
 #include <algorithm>
@@ -29,9 +28,6 @@
 namespace lf {
 
 // ------------------------------------------------------------------ int8 MFMA residue product
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef int v16i __attribute__((ext_vector_type(16)));
-
 constexpr int PT = 128;       // output tile per workgroup (rows and columns)
 constexpr int PK = 32;        // K per MFMA step
 constexpr u32 XCDS = 8;       // MI355X: 8 XCDs, workgroups dealt to them round-robin by linear id
@@ -254,8 +250,7 @@ uint32_t inverse_mod(uint64_t a, uint64_t m) // a^-1 mod m (gcd 1)
 }
 
 // ------------------------------------------------------------------ band analysis on the device
-// The reference's per-line analysis (linalg.mm:82-111), one wavefront per line reading the line's exponent,
-// sign and status planes: status OR, largest and smallest exponent of a nonzero status-free entry, the class
+// The reference's per-line analysis (linalg.mm:82-111) from the lines' exponent, sign and status planes: status OR, largest and smallest exponent of a nonzero status-free entry, the class
 // (0 bands, 1 zero or status line, 2 exact fallback) and the greedy bands [hi - G, hi] taken from the largest
 // exponent down (lo: the smallest exponent inside), one pass over the line per band.  Lines with more than
 // max_bands bands or a spread above max_spread are class 2; the first GEMM_MAX_BANDS bands are stored and nb
@@ -265,47 +260,61 @@ using lf::MatView;
 using lf::u32;
 using lf::u64;
 using lf::GEMM_MAX_BANDS;
+using lf::DIGIT_TABLE_BYTES;
+using lf::PT;
 
-struct AnalyzeArgs {
+struct AnalyzeSide {
     MatView v;
+    uint32_t nlines, blocks;
+    uint32_t by_line; // lines adjacent in memory: a workgroup takes 16 lines, else one wavefront a line
+    GemmLine* out;
+    GemmLine* host; // the same table in pinned host memory
+};
+struct AnalyzeArgs {
+    AnalyzeSide side[2];
     uint32_t field_plane; // N: exponent plane (sign N + 1, status N + 2)
-    uint32_t nlines, K;
+    uint32_t K;
     int32_t G, max_bands, max_spread;
     uint32_t force;
-    GemmLine* out;
 };
 
-__device__ __forceinline__ int wave_max(int x)
+constexpr u32 ANALYZE_THREADS = 1024, ANALYZE_LINES = 16;
+
+// Reductions over the threads of one line: the 64 lanes of its wavefront, or lanes l, l + 16, l + 32, l + 48 of
+// every wavefront of the workgroup (through red, 16 values a wavefront), with every thread getting the result.
+template <bool BY_LINE, class F> __device__ __forceinline__ int line_reduce(int x, int (*red)[ANALYZE_LINES], F pick)
 {
+    const u32 lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
 #pragma unroll
-    for (int o = 32; o; o >>= 1) x = max(x, __shfl_xor(x, o));
-    return x;
-}
-__device__ __forceinline__ int wave_min(int x)
-{
+    for (int o = 32; o >= (BY_LINE ? 16 : 1); o >>= 1) x = pick(x, __shfl_xor(x, o));
+    if constexpr (BY_LINE) {
+        if (lane < ANALYZE_LINES) red[wave][lane] = x;
+        __syncthreads();
+        x = red[0][lane % ANALYZE_LINES];
 #pragma unroll
-    for (int o = 32; o; o >>= 1) x = min(x, __shfl_xor(x, o));
-    return x;
-}
-__device__ __forceinline__ u32 wave_or(u32 x)
-{
-#pragma unroll
-    for (int o = 32; o; o >>= 1) x |= (u32)__shfl_xor((int)x, o);
+        for (u32 w = 1; w < ANALYZE_THREADS / 64u; ++w) x = pick(x, red[w][lane % ANALYZE_LINES]);
+        __syncthreads();
+    }
     return x;
 }
 
-__global__ void __launch_bounds__(256) analyze_kernel(AnalyzeArgs a)
+// One line's record, its threads striding over the line's K entries: first status and exponent range, then one
+// pass per band.  BY_LINE: the workgroup's 16 lines go through the same passes together.
+template <bool BY_LINE> __device__ __forceinline__ void analyze_line(const AnalyzeArgs& a, const AnalyzeSide& S, u32 line, bool live, u32 first,
+                                                                     u32 step, bool leader, GemmLine& L, int (*red)[ANALYZE_LINES])
 {
-    const u32 lane = threadIdx.x & 63u, line = blockIdx.x * 4u + (threadIdx.x >> 6);
-    if (line >= a.nlines) return; // whole wavefronts leave together
-    const u32* ep = a.v.planes + (u64)a.field_plane * a.v.pitch;
-    const u32* sp = ep + a.v.pitch;
-    const u32* tp = sp + a.v.pitch;
-    const u64 base = (u64)line * a.v.ls;
+    const u32* ep = S.v.planes + (u64)a.field_plane * S.v.pitch;
+    const u32* sp = ep + S.v.pitch;
+    const u32* tp = sp + S.v.pitch;
+    const u64 base = (u64)line * S.v.ls;
+    const u32 K = live ? a.K : 0u;
+    const auto mx = [](int x, int y) { return max(x, y); };
+    const auto mn = [](int x, int y) { return min(x, y); };
     u32 status = 0;
     int top = INT_MIN, bottom = INT_MAX;
-    for (u32 k = lane; k < a.K; k += 64u) {
-        const u64 i = base + (u64)k * a.v.ks;
+#pragma unroll 4
+    for (u32 k = first; k < K; k += step) {
+        const u64 i = base + (u64)k * S.v.ks;
         const int e = (int)ep[i], sg = (int)sp[i];
         const u32 st = tp[i];
         status |= st;
@@ -314,62 +323,95 @@ __global__ void __launch_bounds__(256) analyze_kernel(AnalyzeArgs a)
             bottom = min(bottom, e);
         }
     }
-    status = wave_or(status);
-    top = wave_max(top);
-    bottom = wave_min(bottom);
-    GemmLine L;
-    L.cls = 1;
-    L.nb = 0;
-    L.low = 0;
-    L.status = status;
+    status = (u32)line_reduce<BY_LINE>((int)status, red, [](int x, int y) { return x | y; });
+    top = line_reduce<BY_LINE>(top, red, mx);
+    bottom = line_reduce<BY_LINE>(bottom, red, mn);
     const bool any = top != INT_MIN;
-    L.top = any ? top : 0;
-    L.bottom = any ? bottom : 0;
+    int cls = 1, nb = 0, low = 0, hi = top;
+    bool more = false;
+    if (leader)
 #pragma unroll
-    for (int b = 0; b < GEMM_MAX_BANDS; ++b) L.member[b] = L.lo[b] = L.hi[b] = 0;
-    if (!status && any) {
-        if (a.force) L.cls = 2;
+        for (int b = 0; b < GEMM_MAX_BANDS; ++b) L.member[b] = L.lo[b] = L.hi[b] = 0;
+    if (live && !status && any) {
+        if (a.force) cls = 2;
         else if (a.max_bands >= 1 && (long)top - bottom <= a.G) {
-            L.cls = 0;
-            L.nb = 1;
-            L.lo[0] = bottom;
-            L.hi[0] = top;
-            L.low = bottom;
-        } else if ((long)top - bottom > a.max_spread) {
-            L.cls = 2;
-        } else {
-            int hi = top, nb = 0;
-            bool fallback = false;
-            while (true) {
-                int lo = hi, next = INT_MIN;
-                for (u32 k = lane; k < a.K; k += 64u) {
-                    const u64 i = base + (u64)k * a.v.ks;
-                    const int e = (int)ep[i], sg = (int)sp[i];
-                    const u32 st = tp[i];
-                    if (st || !sg || e > hi) continue;
-                    if ((long)e >= (long)hi - a.G) lo = min(lo, e);
-                    else next = max(next, e);
-                }
-                lo = wave_min(lo);
-                next = wave_max(next);
-                if (nb < GEMM_MAX_BANDS) {
-                    L.lo[nb] = lo;
-                    L.hi[nb] = hi;
-                }
-                ++nb;
-                L.low = lo;
-                if (nb > a.max_bands) {
-                    fallback = true;
-                    break;
-                }
-                if (next == INT_MIN) break;
-                hi = next;
+            cls = 0;
+            nb = 1;
+            low = bottom;
+            if (leader) {
+                L.lo[0] = bottom;
+                L.hi[0] = top;
             }
-            L.cls = fallback ? 2 : 0;
-            L.nb = fallback ? 0 : nb;
-        }
+        } else if ((long)top - bottom > a.max_spread) cls = 2;
+        else more = true;
     }
-    if (lane == 0) a.out[line] = L;
+    while (BY_LINE ? __syncthreads_or(more) != 0 : more) {
+        int lo = hi, next = INT_MIN;
+        if (more)
+#pragma unroll 4
+            for (u32 k = first; k < K; k += step) {
+                const u64 i = base + (u64)k * S.v.ks;
+                const int e = (int)ep[i], sg = (int)sp[i];
+                const u32 st = tp[i];
+                if (st || !sg || e > hi) continue;
+                if ((long)e >= (long)hi - a.G) lo = min(lo, e);
+                else next = max(next, e);
+            }
+        lo = line_reduce<BY_LINE>(lo, red, mn);
+        next = line_reduce<BY_LINE>(next, red, mx);
+        if (!more) continue;
+        if (leader && nb < GEMM_MAX_BANDS) {
+            L.lo[nb] = lo;
+            L.hi[nb] = hi;
+        }
+        ++nb;
+        low = lo;
+        if (nb > a.max_bands) {
+            cls = 2;
+            nb = 0;
+            more = false;
+        } else if (next == INT_MIN) {
+            cls = 0;
+            more = false;
+        } else
+            hi = next;
+    }
+    if (leader) {
+        L.cls = cls;
+        L.nb = nb;
+        L.low = low;
+        L.status = status;
+        L.top = any ? top : 0;
+        L.bottom = any ? bottom : 0;
+        L.member[0] = (int)line; // its extended row while every line is one band
+    }
+}
+
+// Both sides of a product in one launch; the records go to the device table and to the host's.  What bounds it is
+// the latency of its loads: 16 lines and 64 rows of them at a time where lines are adjacent (a wavefront per
+// line there read one word per 64 bytes: 56 us for 512 columns of 2048 entries).
+__global__ void __launch_bounds__(ANALYZE_THREADS) analyze_kernel(AnalyzeArgs a)
+{
+    __shared__ int red[ANALYZE_THREADS / 64][ANALYZE_LINES];
+    __shared__ GemmLine rec[ANALYZE_LINES];
+    const bool second = blockIdx.x >= a.side[0].blocks;
+    const AnalyzeSide S = second ? a.side[1] : a.side[0];
+    const u32 line0 = (blockIdx.x - (second ? a.side[0].blocks : 0u)) * ANALYZE_LINES;
+    const u32 t = threadIdx.x;
+    if (S.by_line) {
+        const u32 l = t % ANALYZE_LINES;
+        analyze_line<true>(a, S, line0 + l, line0 + l < S.nlines, t / ANALYZE_LINES, ANALYZE_THREADS / ANALYZE_LINES, t < ANALYZE_LINES, rec[l], red);
+    } else {
+        const u32 l = t / 64u;
+        analyze_line<false>(a, S, line0 + l, line0 + l < S.nlines, t % 64u, 64u, t % 64u == 0, rec[l], red);
+    }
+    __syncthreads();
+    const u32 lines = min(ANALYZE_LINES, S.nlines - line0), words = sizeof(GemmLine) / 4;
+    for (u32 w = t; w < lines * words; w += ANALYZE_THREADS) {
+        const u32 v = reinterpret_cast<const u32*>(rec)[w];
+        reinterpret_cast<u32*>(S.out + line0)[w] = v;
+        reinterpret_cast<u32*>(S.host + line0)[w] = v;
+    }
 }
 
 // Primes <= 65279, descending: balanced residues then split into two int8 digits (linalg.mm:38-40).
@@ -393,52 +435,29 @@ const std::vector<uint32_t>& primes()
 
 using lf::Product;
 
+// One side of a product: its line table (in pinned host memory) and what the report says of it.
 struct Side {
-    std::vector<GemmLine> lines;
-    std::vector<std::vector<std::pair<long, long>>> bands;
+    GemmLine* lines = nullptr;
+    std::size_t count = 0;
     std::vector<uint64_t> histogram;
     uint64_t fallback = 0;
-    std::vector<std::vector<int>> band_members; // band b -> lines having a band b (in line order)
 };
 
-// The analysis of one side on the device: one analyze_kernel launch over the side's lines, the line table
-// back to the host (the only data the planner reads), then the band histogram and fallback count.
-int analyze_side(const MatView& v, int N, std::size_t lines, std::size_t K, const lf_linalg_options& o, bool force, GemmLine* dev,
-                 hipStream_t stream, Side& s)
+void read_side(Side& s, int max_bands)
 {
-    s.lines.assign(lines, GemmLine{});
-    s.bands.assign(lines, {});
-    if (lines) {
-        AnalyzeArgs a{v, uint32_t(N), uint32_t(lines), uint32_t(K), o.band_bits, o.max_bands, o.max_spread, force ? 1u : 0u, dev};
-        hipLaunchKernelGGL(analyze_kernel, dim3(unsigned((lines + 3) / 4)), dim3(256), 0, stream, a);
-        if (hipError_t e = hipGetLastError()) return fail(LF_RUNTIME_ERROR, std::string("analysis launch: ") + hipGetErrorString(e));
-        if (hipError_t e = hipMemcpyAsync(s.lines.data(), dev, sizeof(GemmLine) * lines, hipMemcpyDeviceToHost, stream))
-            return fail(LF_RUNTIME_ERROR, std::string("download line table: ") + hipGetErrorString(e));
-        if (hipError_t e = hipStreamSynchronize(stream))
-            return fail(LF_RUNTIME_ERROR, std::string("device execution (analysis): ") + hipGetErrorString(e));
+    s.histogram.assign(std::size_t(std::max(max_bands, 0)) + 1, 0);
+    for (std::size_t i = 0; i < s.count; ++i) {
+        const GemmLine& L = s.lines[i];
+        if (L.cls == 2) ++s.fallback;
+        else ++s.histogram[L.cls == 1 ? 0 : L.nb];
     }
-    s.histogram.assign(std::size_t(std::max(o.max_bands, 0)) + 1, 0);
-    for (std::size_t i = 0; i < lines; ++i) {
-        GemmLine& L = s.lines[i];
-        if (L.cls == 1) {
-            ++s.histogram[0];
-            continue;
-        }
-        if (L.cls == 2) {
-            ++s.fallback;
-            continue;
-        }
-        ++s.histogram[L.nb];
-        for (int b = 0; b < L.nb && b < GEMM_MAX_BANDS; ++b) s.bands[i].push_back({L.lo[b], L.hi[b]});
-    }
-    return LF_OK;
 }
 
 // GPU-path capacity: lines whose bands this build's rebuild kernels cannot hold take the exact-dot path
 // (same results; the report counts them as fallback lines).
 void route_capacity(Side& s, int wx_class)
 {
-    for (std::size_t i = 0; i < s.lines.size(); ++i) {
+    for (std::size_t i = 0; i < s.count; ++i) {
         GemmLine& L = s.lines[i];
         if (L.cls != 0) continue;
         const bool too_many = L.nb > GEMM_MAX_BANDS;
@@ -447,7 +466,6 @@ void route_capacity(Side& s, int wx_class)
             L.cls = 2;
             ++s.fallback;
             --s.histogram[L.nb];
-            s.bands[i].clear();
         }
     }
 }
@@ -535,6 +553,240 @@ struct PoolBuf {
     }
 };
 
+// The line tables' pinned host memory, kept per host thread and device and grown on demand (a product waits for
+// its stream before it returns, so the next one may overwrite it).
+struct PinnedTable {
+    GemmLine* p = nullptr;
+    std::size_t lines = 0;
+    ~PinnedTable()
+    {
+        if (p) (void)hipHostFree(p);
+    }
+};
+hipError_t pinned_table(std::size_t lines, GemmLine** out)
+{
+    thread_local PinnedTable tables[16];
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev)) return e;
+    PinnedTable& t = tables[dev & 15];
+    if (t.lines < lines) {
+        if (t.p) (void)hipHostFree(t.p);
+        t.p = nullptr;
+        t.lines = 0;
+        if (hipError_t e = hipHostMalloc((void**)&t.p, lines * sizeof(GemmLine), hipHostMallocDefault)) return e;
+        t.lines = lines;
+    }
+    *out = t.p;
+    return hipSuccess;
+}
+
+// ------------------------------------------------------------------ constants of the residue path
+// Modulus counts up to the widest CRT class: bits and double log2 sums of the products of the first L primes.
+constexpr unsigned MAX_L = 208;
+struct ModulusSums {
+    double have[MAX_L + 1];
+    int bits[MAX_L + 1];
+    ModulusSums()
+    {
+        Big M = big_from(1);
+        have[0] = 0;
+        bits[0] = M.bits();
+        for (unsigned q = 0; q < MAX_L; ++q) {
+            have[q + 1] = have[q] + std::log2(double(primes()[q]));
+            big_mul_small(M, primes()[q]);
+            bits[q + 1] = M.bits();
+        }
+    }
+};
+// The fewest moduli for an integer of `need` bits: the reference's double sum, then the same bound exactly (M is
+// odd and `need` an integer, so M > 2^need means more than `need` bits), which only guards against the sum's
+// rounding.  0: more than MAX_L.
+unsigned modulus_count(double need, int* bits)
+{
+    static const ModulusSums sums;
+    unsigned L = 0;
+    while (L <= MAX_L && sums.have[L] <= need) ++L;
+    while (L <= MAX_L && sums.bits[L] <= int(need)) ++L;
+    if (L > MAX_L) return 0;
+    *bits = sums.bits[L];
+    return L;
+}
+
+// Device tables kept per host thread and device: the digit table of all moduli (once), and the CRT constants of
+// the (moduli, words) sizes used last, at most CRT_SETS of them (each below 100 KB).
+struct DigitTable {
+    const int8_t* table;
+    const int32_t* offset[DIGIT_TABLE_BYTES / 32 + 1]; // by byte length / 32
+    const uint32_t* moduli;
+    const float* inverse;
+};
+struct CrtSet {
+    unsigned L = 0;
+    int WX = 0;
+    int shift = 0;
+    const int32_t* fold;
+    const uint32_t* crt;
+    const uint32_t* bound;
+};
+constexpr std::size_t CRT_SETS = 16;
+struct ConstantCache {
+    void* digits_mem = nullptr;
+    DigitTable digits{};
+    struct Entry {
+        CrtSet set;
+        void* mem = nullptr;
+        uint64_t used = 0;
+    };
+    std::vector<Entry> sets;
+    uint64_t clock = 0;
+    ~ConstantCache()
+    {
+        if (digits_mem) (void)hipFree(digits_mem);
+        for (auto& e : sets)
+            if (e.mem) (void)hipFree(e.mem);
+    }
+};
+ConstantCache& constant_cache(int dev)
+{
+    thread_local ConstantCache caches[16];
+    return caches[dev & 15];
+}
+
+// Uploads `words` into new device memory, complete on return.
+hipError_t upload_words(const std::vector<uint32_t>& words, void** mem)
+{
+    if (hipError_t e = hipMalloc(mem, words.size() * 4)) return e;
+    if (hipError_t e = hipMemcpy(*mem, words.data(), words.size() * 4, hipMemcpyHostToDevice)) {
+        (void)hipFree(*mem);
+        *mem = nullptr;
+        return e;
+    }
+    return hipSuccess;
+}
+
+hipError_t digit_table(const DigitTable** out)
+{
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev)) return e;
+    ConstantCache& c = constant_cache(dev);
+    if (!c.digits_mem) {
+        constexpr unsigned W = DIGIT_TABLE_BYTES, S = W / 32 + 1;
+        std::vector<uint32_t> w(MAX_L * 2 * W / 4 + S * MAX_L + 2 * MAX_L, 0);
+        int8_t* tab = reinterpret_cast<int8_t*>(w.data());
+        uint32_t *off = w.data() + MAX_L * 2 * W / 4, *mod = off + S * MAX_L, *inv = mod + MAX_L;
+        for (unsigned q = 0; q < MAX_L; ++q) {
+            const uint32_t m = primes()[q];
+            uint64_t p = 1, sum = 0;
+            for (unsigned h = 0; h < W; ++h) {
+                if (h % 32 == 0) off[h / 32 * MAX_L + q] = uint32_t(128 * sum % m);
+                const int v = p > m / 2 ? int(p) - int(m) : int(p), d0 = ((v + 128) & 255) - 128;
+                tab[(q * 2) * W + h] = int8_t((v - d0) / 256);
+                tab[(q * 2 + 1) * W + h] = int8_t(d0);
+                sum += p;
+                p = (p << 8) % m;
+            }
+            off[(S - 1) * MAX_L + q] = uint32_t(128 * sum % m);
+            mod[q] = m;
+            const float f = 1.0f / float(m);
+            std::memcpy(&inv[q], &f, 4);
+        }
+        if (hipError_t e = upload_words(w, &c.digits_mem)) return e;
+        const uint32_t* d = (const uint32_t*)c.digits_mem;
+        c.digits.table = (const int8_t*)d;
+        for (unsigned k = 0; k < S; ++k) c.digits.offset[k] = (const int32_t*)(d + MAX_L * 2 * W / 4 + k * MAX_L);
+        c.digits.moduli = d + MAX_L * 2 * W / 4 + S * MAX_L;
+        c.digits.inverse = (const float*)(c.digits.moduli + MAX_L);
+    }
+    *out = &c.digits;
+    return hipSuccess;
+}
+
+// fold[L][3] | crt[L][WX] | bound[2][WX] for the first L primes and WX CRT words
+hipError_t crt_constants(unsigned L, int WX, CrtSet* out)
+{
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev)) return e;
+    ConstantCache& c = constant_cache(dev);
+    for (auto& e : c.sets)
+        if (e.set.L == L && e.set.WX == WX) {
+            e.used = ++c.clock;
+            *out = e.set;
+            return hipSuccess;
+        }
+    Big M = big_from(1);
+    for (unsigned q = 0; q < L; ++q) big_mul_small(M, primes()[q]);
+    CrtSet set;
+    set.L = L;
+    set.WX = WX;
+    set.shift = 32 * (WX - 1) - M.bits();
+    std::vector<uint32_t> w, crt;
+    for (unsigned q = 0; q < L; ++q) {
+        const uint32_t m = primes()[q];
+        const Big Mq = big_div_small(M, m);
+        // the product kernel's digit weights 65536 y, 256 y, y (mod m, balanced), y = (M/m)^-1 mod m
+        const uint64_t y = inverse_mod(big_mod_small(Mq, m), m);
+        for (uint64_t d : {uint64_t(65536), uint64_t(256), uint64_t(1)}) {
+            const int64_t k = int64_t(d * y % m);
+            w.push_back(uint32_t(int32_t(k > int64_t(m / 2) ? k - int64_t(m) : k)));
+        }
+        const std::vector<uint32_t> words = big_shifted(Mq, set.shift, WX);
+        crt.insert(crt.end(), words.begin(), words.end());
+    }
+    const std::size_t o_crt = w.size(), o_bound = o_crt + crt.size();
+    w.insert(w.end(), crt.begin(), crt.end());
+    const std::vector<uint32_t> Ms = big_shifted(M, set.shift, WX);
+    w.insert(w.end(), Ms.begin(), Ms.end());
+    for (int i = 0; i < WX; ++i) w.push_back((Ms[i] >> 1) | (i + 1 < WX ? Ms[i + 1] << 31 : 0u));
+    ConstantCache::Entry* slot = nullptr;
+    if (c.sets.size() < CRT_SETS) {
+        c.sets.emplace_back();
+        slot = &c.sets.back();
+    } else {
+        slot = &*std::min_element(c.sets.begin(), c.sets.end(), [](const auto& x, const auto& y) { return x.used < y.used; });
+        (void)hipFree(slot->mem); // the products that used it have finished
+        *slot = {};
+    }
+    if (hipError_t e = upload_words(w, &slot->mem)) return e;
+    const uint32_t* d = (const uint32_t*)slot->mem;
+    set.fold = (const int32_t*)d;
+    set.crt = d + o_crt;
+    set.bound = d + o_bound;
+    slot->set = set;
+    slot->used = ++c.clock;
+    *out = set;
+    return hipSuccess;
+}
+
+// ------------------------------------------------------------------ the plan of a residue product
+// How the class 0 lines run: by their bands, or joined, every line one band from its lowest exponent.  Joined lines
+// need more moduli and CRT words, and save the extra rows and band pairs: on the 512-bit 512^3 product with three
+// bands a line (73 moduli, nine pairs an output, against 123 moduli) 1.62 ms by bands, 0.43 ms joined.
+struct Plan {
+    bool joined = false;
+    unsigned L = 0;
+    int wx_class = 0, width = 0; // widest band: bits an entry is shifted by
+    double cost = 0;
+};
+// Bits an exact product of band integers needs, and the CRT class that holds M (2: none compiled).
+bool plan_moduli(Plan& p, int bits, int logk)
+{
+    int mbits = 0;
+    p.L = modulus_count(2.0 * bits + 2 * p.width + logk + 2, &mbits);
+    const int N = bits / 32;
+    p.wx_class = !p.L ? 2 : mbits + 1 <= 32 * (lf::rebuild_words(N, 0) - 1) ? 0 : mbits + 1 <= 32 * (lf::rebuild_words(N, 1) - 1) ? 1 : 2;
+    return p.wx_class < 2;
+}
+std::size_t digit_bytes(int N, int width) { return (std::size_t(4 * N) + (width + 7) / 8 + 31) / 32 * 32; }
+// Nanoseconds of the three large stages, from their measured rates on an MI355X: 2.8 per 32-deep step of a 128 x 128
+// product tile, 16 CRT multiply-adds per picosecond-thousand and 0.06 per staged band pair and output, 0.7 per
+// thousand residues.  It only has to rank two plans of one product, which differ by their moduli and rows.
+double plan_cost(const Plan& p, int N, std::size_t rows, std::size_t cols, std::size_t lines, std::size_t K, double pairs, bool syrk)
+{
+    const double tr = double((rows + PT - 1) / PT), tc = double((cols + PT - 1) / PT), tiles = syrk ? tr * (tr + 1) / 2 : tr * tc;
+    const double steps = double((K + 63) / 64 * 2), WX = lf::rebuild_words(N, p.wx_class);
+    return 2.8 * tiles * steps * p.L + pairs * (6.2e-5 * p.L * WX + (p.joined ? 0.0 : 0.06)) + 7e-4 * double(lines) * double(K) * p.L;
+}
+
 #define GEMM_HIP(call, where)                                                                                          \
     do {                                                                                                               \
         hipError_t e_ = (call);                                                                                        \
@@ -542,6 +794,7 @@ struct PoolBuf {
     } while (0)
 
 typedef hipError_t (*digits_fn)(const lf::DigitsArgs&, hipStream_t);
+typedef hipError_t (*round_fn)(int, const lf::RoundArgs&, hipStream_t);
 typedef hipError_t (*rebuild_fn)(int, const lf::RebuildArgs&, hipStream_t);
 typedef hipError_t (*dot_fn)(int, const lf::DotArgs&, hipStream_t);
 typedef hipError_t (*csize_fn)(const lf::DotArgs&, uint32_t*, hipStream_t);
@@ -550,6 +803,7 @@ struct GemmTables;
 template <int N> void fill_gemm(GemmTables& t);
 struct GemmTables {
     digits_fn digits[33] = {};
+    round_fn round[33] = {};
     rebuild_fn rebuild[33] = {};
     dot_fn dot[33] = {};
     csize_fn cluster_size[33] = {};
@@ -559,6 +813,7 @@ struct GemmTables {
 template <int N> void fill_gemm(GemmTables& t)
 {
     t.digits[N] = lf::launch_digits<N>;
+    t.round[N] = lf::launch_round<N>;
     t.rebuild[N] = lf::launch_rebuild<N>;
     t.dot[N] = lf::launch_dot<N>;
     t.cluster_size[N] = lf::launch_cluster_size<N>;
@@ -586,174 +841,196 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
     }
     auto t0 = Clock::now();
     const bool force = P.opt.force_fallback || P.K > MAX_K || P.opt.method == 1;
-    // line tables: written by the analysis on the device, completed with the member lists on the host
-    PoolBuf dl{0}, dr{1};
-    GEMM_HIP(dl.alloc(sizeof(GemmLine) * std::max<std::size_t>(P.m, 1)), "hipMalloc (lines)");
-    if (!P.syrk) GEMM_HIP(dr.alloc(sizeof(GemmLine) * std::max<std::size_t>(P.n, 1)), "hipMalloc (lines)");
-    Side ls, rs_own;
-    if (int r = analyze_side(P.left, N, P.m, P.K, P.opt, force, (GemmLine*)dl.p, P.stream, ls)) return r;
-    if (!P.syrk)
-        if (int r = analyze_side(P.right, N, P.n, P.K, P.opt, force, (GemmLine*)dr.p, P.stream, rs_own)) return r;
-    Side& rs = P.syrk ? ls : rs_own;
-    // modulus count from the widest band of both sides (linalg.mm:341-345)
-    int pmax = 0;
-    for (const Side* s : {&ls, &rs})
-        for (std::size_t i = 0; i < s->lines.size(); ++i)
-            if (s->lines[i].cls == 0)
-                for (int b = 0; b < s->lines[i].nb && b < GEMM_MAX_BANDS; ++b) pmax = std::max(pmax, s->lines[i].hi[b] - s->lines[i].lo[b]);
-    const int logk = ceil_log2(P.K);
-    const double need = 2.0 * P.bits + 2 * pmax + logk + 2;
-    double have = 0;
-    unsigned L = 0;
-    while (have <= need) have += std::log2(double(primes()[L++]));
-    // the same bound checked exactly: M > 2^need, i.e. M has more than `need` bits (M is odd and `need` an
-    // integer); the double sum above decides L as the reference does, this only guards against its rounding
-    Big M = big_from(1);
-    for (unsigned q = 0; q < L; ++q) big_mul_small(M, primes()[q]);
-    while (M.bits() <= int(need)) {
-        big_mul_small(M, primes()[L]);
-        ++L;
+    // line tables: written by the analysis on the device and into pinned host memory in one launch, completed with
+    // the member lists on the host where lines are not their own extended rows
+    const std::size_t nlines = P.m + (P.syrk ? 0 : P.n);
+    PoolBuf dtab{0};
+    GEMM_HIP(dtab.alloc(sizeof(GemmLine) * std::max<std::size_t>(nlines, 1)), "hipMalloc (lines)");
+    GemmLine* htab = nullptr;
+    GEMM_HIP(pinned_table(std::max<std::size_t>(nlines, 1), &htab), "hipHostMalloc (lines)");
+    const GemmLine* dleft = (const GemmLine*)dtab.p;
+    const GemmLine* dright = P.syrk ? dleft : dleft + P.m;
+    {
+        AnalyzeArgs a{};
+        a.field_plane = uint32_t(N);
+        a.K = uint32_t(P.K);
+        a.G = P.opt.band_bits;
+        a.max_bands = P.opt.max_bands;
+        a.max_spread = P.opt.max_spread;
+        a.force = force ? 1u : 0u;
+        uint32_t blocks = 0;
+        for (int k = 0; k < (P.syrk ? 1 : 2); ++k) {
+            AnalyzeSide& S = a.side[k];
+            S.v = k ? P.right : P.left;
+            S.nlines = uint32_t(k ? P.n : P.m);
+            S.blocks = (S.nlines + ANALYZE_LINES - 1) / ANALYZE_LINES;
+            S.by_line = S.v.ls == 1 && S.v.ks != 1;
+            S.out = (GemmLine*)dtab.p + (k ? P.m : 0);
+            S.host = htab + (k ? P.m : 0);
+            blocks += S.blocks;
+        }
+        if (blocks) {
+            hipLaunchKernelGGL(analyze_kernel, dim3(blocks), dim3(ANALYZE_THREADS), 0, P.stream, a);
+            GEMM_HIP(hipGetLastError(), "analysis launch");
+            GEMM_HIP(hipStreamSynchronize(P.stream), "device execution (analysis)");
+        }
     }
-    const int mbits = M.bits();
-    int wx_class = mbits + 1 <= 32 * (lf::rebuild_words(N, 0) - 1) ? 0 : mbits + 1 <= 32 * (lf::rebuild_words(N, 1) - 1) ? 1 : 2;
-    if (wx_class == 2) { // beyond the compiled CRT classes: every band line takes the exact-dot path
+    Side ls, rs_own;
+    ls.lines = htab;
+    ls.count = P.m;
+    read_side(ls, P.opt.max_bands);
+    if (!P.syrk) {
+        rs_own.lines = htab + P.m;
+        rs_own.count = P.n;
+        read_side(rs_own, P.opt.max_bands);
+    }
+    Side& rs = P.syrk ? ls : rs_own;
+    const int logk = ceil_log2(P.K);
+    // the band plan: modulus count from the widest band of both sides (linalg.mm:341-345)
+    Plan bands;
+    for (const Side* s : {&ls, &rs})
+        for (std::size_t i = 0; i < s->count; ++i)
+            if (s->lines[i].cls == 0)
+                for (int b = 0; b < s->lines[i].nb && b < GEMM_MAX_BANDS; ++b) bands.width = std::max(bands.width, s->lines[i].hi[b] - s->lines[i].lo[b]);
+    if (!plan_moduli(bands, P.bits, logk)) { // beyond the compiled CRT classes: every band line takes the exact-dot path
         for (Side* s : {&ls, &rs})
-            for (auto& Ln : s->lines)
+            for (std::size_t i = 0; i < s->count; ++i) {
+                GemmLine& Ln = s->lines[i];
                 if (Ln.cls == 0) {
                     --s->histogram[Ln.nb];
                     Ln.cls = 2;
                     ++s->fallback;
                 }
-        wx_class = 0;
+            }
+        bands.wx_class = 0;
     }
-    route_capacity(ls, wx_class);
-    if (!P.syrk) route_capacity(rs, wx_class);
-    // extended operands: band-major member lists (linalg.mm:326-330)
-    std::size_t Me = 0, Ne = 0;
-    auto assign_members = [](Side& s) {
+    route_capacity(ls, bands.wx_class);
+    if (!P.syrk) route_capacity(rs, bands.wx_class);
+    // lines by class and bands: extended rows, and what the outputs are
+    struct Count {
+        std::size_t rows = 0, lines0 = 0, single = 0, trivial = 0, dots = 0;
+        int widest = 0, most = 0; // widest line, most bands
+    };
+    auto count_side = [](const Side& s) {
+        Count c;
+        for (std::size_t i = 0; i < s.count; ++i) {
+            const GemmLine& Ln = s.lines[i];
+            if (Ln.cls == 0) {
+                ++c.lines0;
+                c.rows += std::size_t(Ln.nb);
+                c.single += Ln.nb == 1;
+                c.widest = std::max(c.widest, Ln.top - Ln.bottom);
+                c.most = std::max(c.most, Ln.nb);
+            } else if (Ln.cls == 1) ++c.trivial;
+            else ++c.dots;
+        }
+        return c;
+    };
+    const Count cl = count_side(ls), cr = P.syrk ? cl : count_side(rs);
+    const bool any_pair = cl.lines0 && cr.lines0;
+    const std::size_t rep_rows = cl.rows, rep_cols = cr.rows;
+    // the plan that runs
+    Plan plan = bands;
+    bool single = cl.single == cl.lines0 && cr.single == cr.lines0; // every line is one band
+    if (any_pair && !single) {
+        Plan join;
+        join.joined = true;
+        join.width = std::max(cl.widest, cr.widest);
+        if (plan_moduli(join, P.bits, logk) && digit_bytes(N, join.width) <= DIGIT_TABLE_BYTES) {
+            const double share = P.syrk ? 0.5 : 1.0; // outputs of the lower triangle
+            const double out = share * double(cl.lines0) * double(cr.lines0);
+            bands.cost = plan_cost(bands, N, cl.rows, cr.rows, nlines, P.K, share * double(cl.rows) * double(cr.rows), P.syrk);
+            join.cost = plan_cost(join, N, cl.lines0, cr.lines0, nlines, P.K, out, P.syrk);
+            if (join.cost < bands.cost) {
+                plan = join;
+                single = true;
+            }
+        }
+    }
+    const unsigned L = plan.L;
+    // extended operands: band-major member lists (linalg.mm:326-330); a side whose lines are all one band in the
+    // device's table is its own list
+    bool upload = false;
+    auto assign_members = [&](Side& s, const Count& c) {
+        if (c.lines0 == s.count && single && !(plan.joined && P.subtract)) return c.lines0;
+        upload = upload || s.count;
         std::size_t next = 0;
+        if (plan.joined)
+            for (std::size_t i = 0; i < s.count; ++i)
+                if (s.lines[i].cls == 0) {
+                    GemmLine& Ln = s.lines[i];
+                    Ln.nb = 1;
+                    Ln.lo[0] = Ln.low = Ln.bottom;
+                    Ln.hi[0] = Ln.top;
+                }
         for (int b = 0; b < GEMM_MAX_BANDS; ++b)
-            for (auto& Ln : s.lines)
-                if (Ln.cls == 0 && Ln.nb > b) Ln.member[b] = int(next++);
+            for (std::size_t i = 0; i < s.count; ++i)
+                if (s.lines[i].cls == 0 && s.lines[i].nb > b) s.lines[i].member[b] = int(next++);
         return next;
     };
-    Me = assign_members(ls);
-    Ne = P.syrk ? Me : assign_members(rs);
-    bool any_pair = false;
-    for (auto& a : ls.lines)
-        if (a.cls == 0) {
-            for (auto& b : rs.lines)
-                if (b.cls == 0) {
-                    any_pair = true;
-                    break;
-                }
-            break;
-        }
     if (rep) {
         rep->band_slots = uint32_t(std::min<std::size_t>(ls.histogram.size(), 65));
         for (std::size_t b = 0; b < ls.histogram.size() && b < 65; ++b) rep->left_bands[b] = ls.histogram[b];
         for (std::size_t b = 0; b < rs.histogram.size() && b < 65; ++b) rep->right_bands[b] = rs.histogram[b];
         rep->left_fallback = ls.fallback;
         rep->right_fallback = rs.fallback;
+        uint32_t np = 0;
+        if (any_pair)
+            for (int b = 0; b < cl.most; ++b)
+                for (int c = 0; c < (P.syrk ? b + 1 : cr.most) && np < 64; ++c) {
+                    uint32_t rows = 0, cols = 0;
+                    for (std::size_t i = 0; i < ls.count; ++i) rows += ls.lines[i].cls == 0 && ls.lines[i].nb > b;
+                    for (std::size_t i = 0; i < rs.count; ++i) cols += rs.lines[i].cls == 0 && rs.lines[i].nb > c;
+                    rep->pairs[np++] = {uint32_t(b), uint32_t(c), rows, cols, bands.L};
+                }
+        rep->npairs = np;
         rep->analysis_seconds = since(t0);
     }
-    t0 = Clock::now();
-    // line tables with the member lists
-    GEMM_HIP(hipMemcpyAsync(dl.p, ls.lines.data(), sizeof(GemmLine) * P.m, hipMemcpyHostToDevice, P.stream), "upload lines");
-    const GemmLine* dright = (const GemmLine*)dl.p;
-    if (!P.syrk) {
-        GEMM_HIP(hipMemcpyAsync(dr.p, rs.lines.data(), sizeof(GemmLine) * P.n, hipMemcpyHostToDevice, P.stream), "upload lines");
-        dright = (const GemmLine*)dr.p;
-    }
-    // outputs for the exact-dot kernels, by window class
+    // outputs for the exact-dot kernels, by window class; the others are counted from the lines
     std::vector<uint32_t> lists[3];
     uint64_t trivial = 0, gpu_out = 0, multi = 0;
-    for (std::size_t i = 0; i < P.m; ++i)
-        for (std::size_t j = 0; j < (P.syrk ? i + 1 : P.n); ++j) {
-            const GemmLine &a = ls.lines[i], &b = rs.lines[j];
-            if (a.cls == 1 || b.cls == 1) {
-                ++trivial;
-                continue;
+    if (cl.dots || cr.dots) {
+        for (std::size_t i = 0; i < P.m; ++i)
+            for (std::size_t j = 0; j < (P.syrk ? i + 1 : P.n); ++j) {
+                const GemmLine &a = ls.lines[i], &b = rs.lines[j];
+                if (a.cls == 1 || b.cls == 1) {
+                    ++trivial;
+                    continue;
+                }
+                if (a.cls == 0 && b.cls == 0) {
+                    ++gpu_out;
+                    multi += a.nb > 1 || b.nb > 1;
+                    continue;
+                }
+                const long span = (long(a.top) + b.top) - (long(a.bottom) + b.bottom) + 64L * N + logk + 3;
+                const int cls = span <= 32L * lf::dot_window_words(0) ? 0 : span <= 32L * lf::dot_window_words(1) ? 1 : 2;
+                lists[cls].push_back(uint32_t(i));
+                lists[cls].push_back(uint32_t(j));
             }
-            if (a.cls == 0 && b.cls == 0) {
-                ++gpu_out;
-                multi += a.nb > 1 || b.nb > 1;
-                continue;
-            }
-            const long span = (long(a.top) + b.top) - (long(a.bottom) + b.bottom) + 64L * N + logk + 3;
-            const int cls = span <= 32L * lf::dot_window_words(0) ? 0 : span <= 32L * lf::dot_window_words(1) ? 1 : 2;
-            lists[cls].push_back(uint32_t(i));
-            lists[cls].push_back(uint32_t(j));
-        }
+    } else {
+        const auto pairs_of = [&](uint64_t a, uint64_t b) { return P.syrk ? a * (a + 1) / 2 : a * b; };
+        gpu_out = pairs_of(cl.lines0, cr.lines0);
+        multi = gpu_out - pairs_of(cl.single, cr.single);
+        trivial = pairs_of(P.m, P.n) - gpu_out;
+    }
     const uint64_t fallback_outputs = (lists[0].size() + lists[1].size() + lists[2].size()) / 2;
+    const std::size_t Me = assign_members(ls, cl), Ne = P.syrk ? Me : assign_members(rs, cr);
+    t0 = Clock::now();
+    if (upload) GEMM_HIP(hipMemcpyAsync(dtab.p, htab, sizeof(GemmLine) * nlines, hipMemcpyHostToDevice, P.stream), "upload lines");
     // residue path
     const std::size_t Kp = std::max<std::size_t>((std::max<std::size_t>(P.K, 1) + 63) / 64 * 64, 64);
     const std::size_t Mp = (Me + PT - 1) / PT * PT, Np = (Ne + PT - 1) / PT * PT; // product tiles
-    PoolBuf dconst{2}, dig_l1{3}, dig_l0{4}, dig_r1{5}, dig_r0{6}, dres{7}, dlist[3] = {{8}, {9}, {10}}, derr{11};
+    PoolBuf dig_l1{3}, dig_l0{4}, dig_r1{5}, dig_r0{6}, dres{7}, dlist[3] = {{8}, {9}, {10}};
     // events bounding the stages: start, digits done, products done, rebuild done, exact dots done
     hipEvent_t* ev = nullptr;
     GEMM_HIP(stage_events(&ev), "hipEventCreate");
     hipEvent_t e0 = ev[0], e1 = ev[4];
-    const int WX = lf::rebuild_words(N, wx_class);
-    const int G = P.opt.band_bits;
-    // constants: moduli | reduce[L][2] | chunk_pow[L][64] | shift_pow[L][G+1] | fold[L][3] | crt[L][WX] | bound[2][WX]
-    std::vector<uint32_t> cst;
-    std::size_t o_mod = 0, o_rec = 0, o_chunk = 0, o_shift = 0, o_fold = 0, o_crt = 0, o_bound = 0;
-    int tshift = 0;
+    const int WX = lf::rebuild_words(N, plan.wx_class);
+    const DigitTable* dt = nullptr;
+    CrtSet crt{};
     if (any_pair) {
-        o_mod = cst.size();
-        for (unsigned q = 0; q < L; ++q) cst.push_back(primes()[q]);
-        o_rec = cst.size();
-        for (unsigned q = 0; q < L; ++q) {
-            const uint32_t m = primes()[q];
-            const float inv = 1.0f / float(m);
-            uint32_t bits;
-            std::memcpy(&bits, &inv, 4);
-            const int64_t c32 = int64_t((uint64_t(1) << 32) % m);
-            cst.push_back(bits);
-            cst.push_back(uint32_t(int32_t(c32 > int64_t(m / 2) ? c32 - int64_t(m) : c32)));
-        }
-        o_chunk = cst.size();
-        for (unsigned q = 0; q < L; ++q) {
-            const uint32_t m = primes()[q];
-            uint64_t p = 1;
-            for (int h = 0; h < 64; ++h) {
-                cst.push_back(uint32_t(p));
-                p = (p << 16) % m;
-            }
-        }
-        o_shift = cst.size();
-        for (unsigned q = 0; q < L; ++q) {
-            const uint32_t m = primes()[q];
-            uint64_t p = 1;
-            for (int s = 0; s <= G; ++s) {
-                cst.push_back(uint32_t(p));
-                p = (p << 1) % m;
-            }
-        }
-        o_fold = cst.size();
-        tshift = 32 * (WX - 1) - mbits;
-        std::vector<std::vector<uint32_t>> crt(L);
-        for (unsigned q = 0; q < L; ++q) {
-            const uint32_t m = primes()[q];
-            Big Mq = big_div_small(M, m);
-            // the product kernel's digit weights 65536 y, 256 y, y (mod m, balanced), y = (M/m)^-1 mod m
-            const uint64_t y = inverse_mod(big_mod_small(Mq, m), m);
-            for (uint64_t w : {uint64_t(65536), uint64_t(256), uint64_t(1)}) {
-                const int64_t k = int64_t(w * y % m);
-                cst.push_back(uint32_t(int32_t(k > int64_t(m / 2) ? k - int64_t(m) : k)));
-            }
-            crt[q] = big_shifted(Mq, tshift, WX);
-        }
-        o_crt = cst.size();
-        for (unsigned q = 0; q < L; ++q) cst.insert(cst.end(), crt[q].begin(), crt[q].end());
-        o_bound = cst.size();
-        std::vector<uint32_t> Ms = big_shifted(M, tshift, WX), H(WX, 0);
-        for (int w = 0; w < WX; ++w) H[w] = (Ms[w] >> 1) | (w + 1 < WX ? Ms[w + 1] << 31 : 0u);
-        cst.insert(cst.end(), Ms.begin(), Ms.end());
-        cst.insert(cst.end(), H.begin(), H.end());
-        GEMM_HIP(dconst.alloc(cst.size() * 4), "hipMalloc (constants)");
-        GEMM_HIP(hipMemcpyAsync(dconst.p, cst.data(), cst.size() * 4, hipMemcpyHostToDevice, P.stream), "upload constants");
+        GEMM_HIP(digit_table(&dt), "digit table");
+        GEMM_HIP(crt_constants(L, WX, &crt), "CRT constants");
         const std::size_t lplane = Mp * Kp, rplane = Np * Kp;
         GEMM_HIP(dig_l1.alloc(L * lplane), "hipMalloc (digits)");
         GEMM_HIP(dig_l0.alloc(L * lplane), "hipMalloc (digits)");
@@ -768,50 +1045,36 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
             GEMM_HIP(dlist[c].alloc(lists[c].size() * 4), "hipMalloc (outputs)");
             GEMM_HIP(hipMemcpyAsync(dlist[c].p, lists[c].data(), lists[c].size() * 4, hipMemcpyHostToDevice, P.stream), "upload outputs");
         }
-    GEMM_HIP(derr.alloc(4), "hipMalloc");
-    GEMM_HIP(hipMemsetAsync(derr.p, 0, 4, P.stream), "hipMemsetAsync");
     if (rep) rep->upload_seconds = since(t0);
     t0 = Clock::now();
     GEMM_HIP(hipEventRecord(e0, P.stream), "hipEventRecord");
-    const uint32_t* C32 = (const uint32_t*)dconst.p;
     if (any_pair) {
-        // the digits kernel writes every byte of the lines' rows; the padding rows [Me, Mp) of each
-        // modulus plane are cleared here
-        auto clear_tail = [&](void* base, std::size_t rows, std::size_t rows_p) -> hipError_t {
-            if (rows_p == rows) return hipSuccess;
-            return hipMemset2DAsync((int8_t*)base + rows * Kp, rows_p * Kp, 0, (rows_p - rows) * Kp, L, P.stream);
-        };
-        GEMM_HIP(clear_tail(dig_l1.p, Me, Mp), "hipMemset2DAsync");
-        GEMM_HIP(clear_tail(dig_l0.p, Me, Mp), "hipMemset2DAsync");
-        if (!P.syrk) {
-            GEMM_HIP(clear_tail(dig_r1.p, Ne, Np), "hipMemset2DAsync");
-            GEMM_HIP(clear_tail(dig_r0.p, Ne, Np), "hipMemset2DAsync");
-        }
+        // the digits kernel writes every byte of the lines' rows; the padding rows past them only feed residues
+        // that nothing reads
         lf::DigitsArgs d{};
         d.L = L;
         d.Kp = uint32_t(Kp);
         d.K = uint32_t(P.K);
-        d.moduli = C32 + o_mod;
-        d.reduce = C32 + o_rec;
-        d.chunk_pow = C32 + o_chunk;
-        d.shift_pow = C32 + o_shift;
-        d.shift_max = uint32_t(G);
-        d.v = P.left;
-        d.lines = (const GemmLine*)dl.p;
-        d.nlines = uint32_t(P.m);
-        d.rows_p = uint32_t(Mp);
-        d.d1 = (int8_t*)dig_l1.p;
-        d.d0 = (int8_t*)dig_l0.p;
-        GEMM_HIP(gemm_tables().digits[N](d, P.stream), "digits launch");
-        if (!P.syrk) {
-            d.v = P.right;
-            d.lines = dright;
-            d.nlines = uint32_t(P.n);
-            d.rows_p = uint32_t(Np);
-            d.d1 = (int8_t*)dig_r1.p;
-            d.d0 = (int8_t*)dig_r0.p;
-            GEMM_HIP(gemm_tables().digits[N](d, P.stream), "digits launch");
+        d.joined = plan.joined;
+        d.bytes = uint32_t(digit_bytes(N, plan.width));
+        d.table = dt->table;
+        d.offset = dt->offset[d.bytes / 32];
+        d.moduli = dt->moduli;
+        d.inverse = dt->inverse;
+        for (int k = 0; k < (P.syrk ? 1 : 2); ++k) {
+            lf::DigitsSide& S = d.side[k];
+            S.v = k ? P.right : P.left;
+            S.lines = k ? dright : dleft;
+            S.nlines = uint32_t(k ? P.n : P.m);
+            S.rows_p = uint32_t(k ? Np : Mp);
+            S.d1 = (int8_t*)(k ? dig_r1.p : dig_l1.p);
+            S.d0 = (int8_t*)(k ? dig_r0.p : dig_l0.p);
+            S.by_line = S.v.ls == 1 && S.v.ks != 1;
+            S.tk = S.by_line ? 32u : Kp >= 256 ? 256u : Kp >= 128 ? 128u : 64u;
+            const uint64_t blocks = (S.nlines + 256u / S.tk - 1) / (256u / S.tk) * ((Kp + S.tk - 1) / S.tk);
+            S.blocks = uint32_t(blocks);
         }
+        GEMM_HIP(gemm_tables().digits[N](d, P.stream), "digits launch");
         GEMM_HIP(hipEventRecord(ev[1], P.stream), "hipEventRecord");
         lf::ProductArgs pa{};
         pa.a1 = (const int8_t*)dig_l1.p;
@@ -823,23 +1086,42 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
         pa.Np = uint32_t(Np);
         pa.Kp = uint32_t(Kp);
         pa.L = L;
-        pa.moduli = C32 + o_mod;
-        pa.fold = (const int32_t*)(C32 + o_fold);
+        pa.moduli = dt->moduli;
+        pa.fold = crt.fold;
         pa.lower = P.syrk;
         GEMM_HIP(lf::launch_product(pa, P.stream), "product launch");
     } else
         GEMM_HIP(hipEventRecord(ev[1], P.stream), "hipEventRecord");
     GEMM_HIP(hipEventRecord(ev[2], P.stream), "hipEventRecord");
-    {
+    if (single && !P.subtract) {
+        lf::RoundArgs r{};
+        r.res = (const uint16_t*)dres.p;
+        r.Mp = uint32_t(Mp);
+        r.Np = uint32_t(Np);
+        r.L = any_pair ? L : 0;
+        r.crt = crt.crt;
+        r.bound = crt.bound;
+        r.t = crt.shift;
+        r.left = dleft;
+        r.right = dright;
+        r.m = uint32_t(P.m);
+        r.n = uint32_t(P.n);
+        r.out = (uint32_t*)P.C.planes;
+        r.out_pitch = P.C.pitch;
+        r.out_stride = P.out_stride ? P.out_stride : P.n;
+        r.syrk = P.syrk;
+        r.lower_only = P.lower_only;
+        GEMM_HIP(gemm_tables().round[N](plan.wx_class, r, P.stream), "rebuild launch");
+    } else {
         lf::RebuildArgs r{};
         r.res = (const uint16_t*)dres.p;
         r.Mp = uint32_t(Mp);
         r.Np = uint32_t(Np);
         r.L = any_pair ? L : 0;
-        r.crt = C32 + o_crt;
-        r.bound = C32 + o_bound;
-        r.t = tshift;
-        r.left = (const GemmLine*)dl.p;
+        r.crt = crt.crt;
+        r.bound = crt.bound;
+        r.t = crt.shift;
+        r.left = dleft;
         r.right = dright;
         r.m = uint32_t(P.m);
         r.n = uint32_t(P.n);
@@ -850,11 +1132,8 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
         r.lower_only = P.lower_only;
         r.subtract = P.subtract;
         // band pairs per output and the stage of the pair CRTs, in row chunks of at most 1 GiB
-        uint32_t pi = 0, pj = 0;
-        for (auto& Ln : ls.lines) pi = std::max<uint32_t>(pi, Ln.cls == 0 ? uint32_t(Ln.nb) : 0u);
-        for (auto& Ln : rs.lines) pj = std::max<uint32_t>(pj, Ln.cls == 0 ? uint32_t(Ln.nb) : 0u);
-        r.pj = std::max<uint32_t>(pj, 1);
-        r.pairs = any_pair ? pi * pj : 0;
+        r.pj = single ? 1u : std::max<uint32_t>(uint32_t(cr.most), 1);
+        r.pairs = any_pair ? (single ? 1u : uint32_t(cl.most)) * r.pj : 0;
         const uint64_t per_row = uint64_t(r.pairs) * P.n * (WX + 1) * 4;
         const uint64_t chunk = per_row ? std::max<uint64_t>(1, (uint64_t(1) << 30) / per_row) : P.m;
         PoolBuf dstage{12};
@@ -863,7 +1142,7 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
         for (uint64_t row0 = 0; row0 < P.m; row0 += chunk) {
             r.row0 = uint32_t(row0);
             r.rows = uint32_t(std::min<uint64_t>(chunk, P.m - row0));
-            GEMM_HIP(gemm_tables().rebuild[N](wx_class, r, P.stream), "rebuild launch");
+            GEMM_HIP(gemm_tables().rebuild[N](plan.wx_class, r, P.stream), "rebuild launch");
         }
     }
     GEMM_HIP(hipEventRecord(ev[3], P.stream), "hipEventRecord");
@@ -872,7 +1151,7 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
         lf::DotArgs x{};
         x.left = P.left;
         x.right = P.right;
-        x.lrows = (const GemmLine*)dl.p;
+        x.lrows = dleft;
         x.rcols = dright;
         x.list = (const uint32_t*)dlist[c].p;
         x.count = uint32_t(lists[c].size() / 2);
@@ -887,7 +1166,6 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
         x.lower_only = P.lower_only;
         x.subtract = P.subtract;
         x.mirror = P.syrk && !P.lower_only;
-        x.error = (int32_t*)derr.p;
         if (c < 2) {
             GEMM_HIP(gemm_tables().dot[N](c, x, P.stream), "exact dot launch");
             continue;
@@ -926,44 +1204,26 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
         }
     }
     GEMM_HIP(hipEventRecord(e1, P.stream), "hipEventRecord");
-    int32_t err = 0;
-    GEMM_HIP(hipMemcpyAsync(&err, derr.p, 4, hipMemcpyDeviceToHost, P.stream), "download status");
     GEMM_HIP(hipStreamSynchronize(P.stream), "device execution (linalg)");
     float ms = 0, stage_ms[4] = {};
     GEMM_HIP(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
     for (int q = 0; q < 4; ++q) GEMM_HIP(hipEventElapsedTime(&stage_ms[q], ev[q], ev[q + 1]), "hipEventElapsedTime");
     if (device_ms) *device_ms = ms;
-    if (err) return fail(LF_RUNTIME_ERROR, "exact dot: internal window overflow");
     if (rep) {
         rep->gpu_seconds = ms * 1e-3;
         rep->digits_seconds = stage_ms[0] * 1e-3;
         rep->product_seconds = stage_ms[1] * 1e-3;
         rep->rebuild_seconds = stage_ms[2] * 1e-3;
         rep->dot_seconds = stage_ms[3] * 1e-3;
-        rep->gemm_rows = Me;
-        rep->gemm_cols = Ne;
-        rep->moduli = any_pair ? L : 0;
-        rep->int8_gemms = any_pair ? 3ull * L : 0;
+        rep->gemm_rows = rep_rows;
+        rep->gemm_cols = rep_cols;
+        rep->moduli = any_pair ? bands.L : 0;
+        rep->int8_gemms = any_pair ? 3ull * bands.L : 0;
         rep->gpu_outputs = gpu_out;
         rep->multi_band_outputs = multi;
         rep->fallback_outputs = fallback_outputs;
         rep->trivial_outputs = trivial;
-        rep->crt_words = any_pair ? uint32_t(WX) : 0;
-        uint32_t np = 0;
-        if (any_pair) {
-            int lb = 0, rb = 0;
-            for (auto& Ln : ls.lines) lb = std::max(lb, Ln.cls == 0 ? Ln.nb : 0);
-            for (auto& Ln : rs.lines) rb = std::max(rb, Ln.cls == 0 ? Ln.nb : 0);
-            for (int b = 0; b < lb; ++b)
-                for (int c = 0; c < (P.syrk ? b + 1 : rb); ++c) {
-                    if (np >= 64) break;
-                    uint32_t rows = 0, cols = 0;
-                    for (auto& Ln : ls.lines) rows += Ln.cls == 0 && Ln.nb > b;
-                    for (auto& Ln : rs.lines) cols += Ln.cls == 0 && Ln.nb > c;
-                    rep->pairs[np++] = {uint32_t(b), uint32_t(c), rows, cols, L};
-                }
-        }
-        rep->npairs = np;
+        rep->crt_words = any_pair ? uint32_t(lf::rebuild_words(N, bands.wx_class)) : 0;
         rep->assembly_seconds = since(t0);
     }
     return LF_OK;

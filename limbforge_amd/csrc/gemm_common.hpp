@@ -34,18 +34,28 @@ struct MatView {
     uint64_t ls, ks;
 };
 
-struct DigitsArgs {
+// Bytes of a modulus's digit table row: entries' shifted mantissas reach at most this many bytes.
+constexpr uint32_t DIGIT_TABLE_BYTES = 256;
+
+struct DigitsSide {
     MatView v;
     const GemmLine* lines;
-    uint32_t nlines, K, Kp, rows_p; // rows_p: extended rows (padded) of this side
-    uint32_t L;
-    const uint32_t* moduli;   // [L]
-    const uint32_t* reduce;   // [L][2]: the bits of 1.0f / m (correctly rounded), balanced 2^32 mod m
-    const uint32_t* chunk_pow; // [L][64]: 2^(16h) mod m for the 16-bit mantissa chunks
-    const uint32_t* shift_pow; // [L][G+1]: 2^s mod m
-    uint32_t shift_max;        // G
-    int8_t* d1;                // [L][rows_p][Kp]
+    uint32_t nlines, rows_p; // rows_p: extended rows (padded) of this side
+    int8_t* d1;              // [L][rows_p][Kp]
     int8_t* d0;
+    uint32_t blocks;         // workgroups of this side
+    uint32_t tk, by_line;    // entries of one line per workgroup (of 256); 1: consecutive threads take consecutive lines
+};
+
+struct DigitsArgs {
+    DigitsSide side[2];
+    uint32_t K, Kp, L;
+    uint32_t joined;         // every line is one band from its lowest exponent
+    uint32_t bytes;          // bytes of a shifted mantissa, a multiple of 32, at most DIGIT_TABLE_BYTES
+    const int8_t* table;     // [moduli][2][DIGIT_TABLE_BYTES]: high and low int8 digit of balanced 2^(8h) mod m
+    const int32_t* offset;   // [moduli]: 128 sum_{h < bytes} 2^(8h) mod m
+    const uint32_t* moduli;
+    const float* inverse;    // 1.0f / m
 };
 
 struct ProductArgs {
@@ -79,6 +89,21 @@ struct RebuildArgs {
     uint32_t row0, rows, pairs, pj;
 };
 
+// Outputs of a product with one band per line: CRT and rounding in one pass (no update form).
+struct RoundArgs {
+    const uint16_t* res;
+    uint32_t Mp, Np, L;
+    const uint32_t* crt;
+    const uint32_t* bound;
+    int32_t t;
+    const GemmLine* left;
+    const GemmLine* right;
+    uint32_t m, n;
+    uint32_t* out;
+    uint64_t out_pitch, out_stride;
+    uint32_t syrk, lower_only;
+};
+
 // Exact dot products of fallback outputs (and the plain limb GEMM): one lane per listed output.
 struct DotArgs {
     MatView left, right;      // element (line, k)
@@ -90,7 +115,6 @@ struct DotArgs {
     uint32_t* out;
     uint64_t out_pitch, out_stride;
     uint32_t syrk, lower_only, subtract, mirror;
-    int32_t* error;           // set when an output needs more than the compiled window
 };
 
 } // namespace lf

@@ -1,14 +1,15 @@
 // gemm_kernels.hpp — kernels of the exact dense products C = RN(op(A) B) and RN(C - op(A) B).
 //
 // Residue path (the reference's algorithm, src/linalg.metal:24-152, rebuilt for CDNA4):
-//   digits_kernel   each entry's exact band integer X = m * 2^(e-lo) reduced modulo every prime (16-bit
-//                   chunk x (2^16h mod m) dot products, then the band shift), balanced residue
-//                   v in (-m/2, m/2], split into int8 digits v = 256 d1 + d0 (linalg.metal:24-39)
+//   digits_kernel   each entry's exact band integer X = m * 2^(e-lo) reduced modulo every prime (its bytes times
+//                   2^(8h) mod m on v_mfma_i32_32x32x32_i8), balanced residue v in [-m/2, m/2], split into
+//                   int8 digits v = 256 d1 + d0 (linalg.metal:24-39)
 //   product_kernel  per modulus and 128x128 tile: G11 = D1 D1', G00 = D0 D0', Gmid = D1 D0' + D0 D1' on
 //                   v_mfma_i32_32x32x32_i8 with int32 accumulation from LDS-staged tiles, then
 //                   y = (65536 G11 + 256 Gmid + G00) (M/m)^-1 mod m written as uint16 (linalg.metal:66-96
 //                   writes the residue itself; the CRT factor rides on the digit weights here)
-//   crt_pairs_kernel, rebuild_kernel  one lane per output: for each band pair, the exact integer by direct
+//   crt_round_kernel  one band per line: one lane per output, CRT and rounding
+//   crt_pairs_kernel, rebuild_kernel  several bands, and updates; one lane per output: for each band pair, the exact integer by direct
 //                   CRT X' = sum_q y_q (M/m_q) 2^t (independent 64-bit column sums, no carry chains),
 //                   reduced mod M' and mapped to the symmetric range,
 //                   then one rounding, or exact accumulation over the band pairs then one rounding
@@ -23,18 +24,27 @@
 
 namespace lf {
 
-// a global table read through the constant address space (uniform loads become scalar loads)
-typedef __attribute__((address_space(4))) const u32 CU32;
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
 
-// ---------------------------------------------------------------- digits
-// One workgroup per (line, 256 consecutive k of [0, Kp)): thread t finds the band of entry k0 + t and its
-// 16-bit mantissa chunks once, then for 16 moduli at a time forms the residue of the entry's extended
-// value (linalg.metal:24-65: chunks times 2^(16h) mod m, times 2^shift mod m, sign, balanced, split into
-// d1 * 256 + d0) and leaves the two digit bytes in LDS; the workgroup then writes every band row of the
-// line for those 256 columns as 16-byte chunks, zero where the entry is not a member of that band (or is
-// zero, carries a status, or lies past K).  Every byte of a line's rows is written, so only the padding
-// rows past the last line need clearing on the host side.
-constexpr u32 DIG_QB = 16; // moduli per LDS batch
+// Residue digits of both operands.  An entry's exact integer X = mantissa << (exponent - band lo) is a string
+// of bytes x_h, and X mod m = sum_h x_h (2^(8h) mod m): a matrix product of entries by moduli with at most 256
+// terms.  It runs on v_mfma_i32_32x32x32_i8: the bytes less 128 as int8 (the 128s come back as one constant a
+// modulus), the powers as two int8 digits, so that two int32 sums give T = 256 s1 + s0 + offset, |T| < 2^30, and
+// one FP32 quotient estimate reduces T to the balanced residue.  A workgroup takes 256 entries (tk consecutive
+// k of 256 / tk lines; where lines are adjacent in memory consecutive threads take consecutive lines, so that
+// loads coalesce), places their shifted bytes in LDS, and for 32 moduli at a time leaves the digit bytes in
+// LDS and writes every band row of its lines as 16-byte chunks, zero where the entry is not a member of that
+// band (or is zero, carries a status, or lies past K).  Rows past the last line are left as they are: no
+// kernel reads the residues they give.
+// What bounds it is the reduction of each residue (about 20 instructions): the two reductions by 16-bit chunks
+// and a table of shift powers that this replaces took 32 multiply-adds of 16-bit chunks and as much again.
+constexpr u32 DIG_QB = 32;                      // moduli per LDS batch
+constexpr u32 DIG_STAGE_ROW = 2 * 256 + 16;     // bytes of a modulus's stage row: both digits of 256 entries
+// a shifted mantissa's LDS row: an odd number of 16-byte chunks, so that the 16 lanes of a fragment read hit
+// distinct banks
+__host__ __device__ constexpr u32 digits_row_bytes(u32 bytes) { return bytes + 16; }
+__host__ __device__ constexpr u64 digits_lds_bytes(u32 bytes) { return (u64)256 * digits_row_bytes(bytes) + DIG_QB * DIG_STAGE_ROW + 256 + 64; }
 
 __device__ __forceinline__ u32 byte_eq_mask(u32 x, u32 b4)
 {
@@ -46,96 +56,124 @@ __device__ __forceinline__ u32 byte_eq_mask(u32 x, u32 b4)
 
 template <int N> __global__ void __launch_bounds__(256) digits_kernel(DigitsArgs g)
 {
-    __shared__ __attribute__((aligned(16))) int8_t stage[DIG_QB][2][256];
-    __shared__ __attribute__((aligned(16))) uint8_t bandof[256];
-    const u32 kblocks = (g.Kp + 255u) / 256u;
-    const u32 line = blockIdx.x / kblocks;
-    const u32 k0 = (blockIdx.x - line * kblocks) * 256u;
-    if (line >= g.nlines) return;
-    const GemmLine* L = g.lines + line;
-    if (L->cls != 0) return; // no rows (uniform over the workgroup)
-    const u32 t = threadIdx.x, k = k0 + t;
-    const int nb = L->nb;
-    u32 band = 0xffu;
-    int shift = 0, s = 0;
-    u32 c[2 * N];
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const u32 rowb = digits_row_bytes(g.bytes);
+    unsigned char* stage = lds + 256u * rowb;
+    unsigned char* bandof = stage + DIG_QB * DIG_STAGE_ROW;
+    u32* signs = reinterpret_cast<u32*>(bandof + 256); // bit e % 32 of word e / 32: entry e is negative
+    const bool second = blockIdx.x >= g.side[0].blocks;
+    const DigitsSide S = second ? g.side[1] : g.side[0];
+    const u32 blk = blockIdx.x - (second ? g.side[0].blocks : 0u);
+    const u32 tk = S.tk, tl = 256u / tk, kblocks = (g.Kp + tk - 1) / tk;
+    const u32 line0 = (blk / kblocks) * tl, k0 = (blk % kblocks) * tk;
+    const u32 t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    for (u32 i = t; i < 256u * rowb / 16u; i += 256u) reinterpret_cast<uint4*>(lds)[i] = make_uint4(0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u);
+    if (t < 8) signs[t] = 0;
+    __syncthreads();
+    {
+        const u32 tline = S.by_line ? t % tl : t / tk, tkk = S.by_line ? t / tl : t % tk, e = tline * tk + tkk;
+        const u32 line = line0 + tline, k = k0 + tkk;
+        u32 band = 0xffu;
+        if (line < S.nlines && k < g.K && S.lines[line].cls == 0) {
+            const GemmLine* L = S.lines + line;
+            const u64 idx = (u64)line * S.v.ls + (u64)k * S.v.ks;
+            const u32* P = S.v.planes;
+            const u64 pitch = S.v.pitch;
+            const u32 st = P[(u64)(N + 2) * pitch + idx];
+            const int s = (int)P[(u64)(N + 1) * pitch + idx];
+            if (!st && s) {
+                const int ex = (int)P[(u64)N * pitch + idx];
+                u32 shift = 0;
+                if (g.joined) {
+                    band = 0;
+                    shift = (u32)(ex - L->low);
+                } else
+                    for (int b = 0; b < L->nb; ++b)
+                        if (ex >= L->lo[b] && ex <= L->hi[b]) {
+                            band = (u32)b;
+                            shift = (u32)(ex - L->lo[b]);
+                        }
+                // the band's width bounds the shift, and the planner sized the row for the widest band
+                if (band != 0xffu && shift / 8u + 4u * N + 4u <= rowb) {
+                    const u32 ws = shift >> 5, b = shift & 31u;
+                    u32* row = reinterpret_cast<u32*>(lds + e * rowb) + ws;
+                    u32 lo = 0;
 #pragma unroll
-    for (int h = 0; h < 2 * N; ++h) c[h] = 0;
-    if (k < g.K) {
-        const u64 idx = (u64)line * g.v.ls + (u64)k * g.v.ks;
-        const u32* P = g.v.planes;
-        const u64 pitch = g.v.pitch;
-        const u32 st = P[(u64)(N + 2) * pitch + idx];
-        s = (int)P[(u64)(N + 1) * pitch + idx];
-        if (!st && s) {
-            const int e = (int)P[(u64)N * pitch + idx];
-            for (int b = 0; b < nb; ++b)
-                if (e >= L->lo[b] && e <= L->hi[b]) {
-                    band = (u32)b;
-                    shift = e - L->lo[b];
+                    for (int w = 0; w < N; ++w) {
+                        const u32 x = P[(u64)w * pitch + idx];
+                        row[w] = (b ? __builtin_amdgcn_alignbit(x, lo, 32u - b) : x) ^ 0x80808080u;
+                        lo = x;
+                    }
+                    if (b) row[N] = (lo >> (32u - b)) ^ 0x80808080u;
+                    if (s < 0) atomicOr(&signs[e >> 5], 1u << (e & 31u));
                 }
-            if (band != 0xffu)
-#pragma unroll
-                for (int w = 0; w < N; ++w) {
-                    const u32 x = P[(u64)w * pitch + idx];
-                    c[2 * w] = x & 0xffffu;
-                    c[2 * w + 1] = x >> 16;
-                }
+            }
         }
+        bandof[e] = (unsigned char)band;
     }
-    bandof[t] = (uint8_t)band;
-    const u64 plane = (u64)g.rows_p * g.Kp;
-    // the modulus tables are read through the constant address space: uniform loads from it are scalar
-    // loads (through a generic pointer the compiler must assume the digit stores below may alias them, and
-    // loads every table row into every lane)
-    const CU32* cpow = (const CU32*)g.chunk_pow;
-    const CU32* mods = (const CU32*)g.moduli;
-    const CU32* red = (const CU32*)g.reduce;
+    __syncthreads();
+    // waves 0-3: entries 64 wave + 32 h + (lane % 32); bytes 32 step + 16 (lane / 32) of each
+    const u32 steps = g.bytes / 32u, r = lane & 31u, kh = lane >> 5;
+    const u32 sg[2] = {signs[2u * wave], signs[2u * wave + 1u]};
     for (u32 qb = 0; qb < g.L; qb += DIG_QB) {
-        const u32 nq = g.L - qb < DIG_QB ? g.L - qb : DIG_QB;
-        // every lane runs the same modulus loop (an entry outside every band has all chunks zero and
-        // yields zero digits); the next modulus's table row is loaded while this one is reduced
-        u32 cp[2 * N], cpn[2 * N], sp = g.shift_pow[qb * (g.shift_max + 1) + (u32)shift];
+        const u32 q = qb + r < g.L ? qb + r : g.L - 1; // lanes past the last modulus repeat it
+        const int8_t* tab = g.table + (u64)q * 2 * DIGIT_TABLE_BYTES + 16u * kh;
+        v16i s1[2] = {}, s0[2] = {};
+        for (u32 st = 0; st < steps; ++st) {
+            const v4i b1 = *(const v4i*)(tab + 32u * st), b0 = *(const v4i*)(tab + DIGIT_TABLE_BYTES + 32u * st);
 #pragma unroll
-        for (int h = 0; h < 2 * N; ++h) cp[h] = cpow[qb * 64u + h];
-        for (u32 qi = 0; qi < nq; ++qi) {
-            const u32 q = qb + qi, qn = qi + 1 < nq ? q + 1 : q;
-#pragma unroll
-            for (int h = 0; h < 2 * N; ++h) cpn[h] = cpow[qn * 64u + h];
-            const u32 spn = g.shift_pow[qn * (g.shift_max + 1) + (u32)shift];
-            const int m = (int)mods[q], c32 = (int)red[2 * q + 1];
-            const float inv = __uint_as_float(red[2 * q]);
-            u64 acc = 0;
-#pragma unroll
-            for (int h = 0; h < 2 * N; ++h) acc += (u64)c[h] * cp[h];
-            // acc < 2N 2^32 and r sp < 2^32: both within the 2^47 of residue_of (residue_reduce.hpp)
-            u32 r = residue_of((int64_t)acc, m, inv, c32);
-            r = residue_of((int64_t)(u32)__umul24(r, sp), m, inv, c32); // (__umul24 is declared int)
-            int v = (int)r;
-            if (s < 0) v = v ? m - v : 0;
-            if (v > (m >> 1)) v -= m;
-            const int d0 = ((v + 128) & 255) - 128;
-            const int d1 = (v - d0) / 256;
-            stage[qi][0][t] = (int8_t)d1;
-            stage[qi][1][t] = (int8_t)d0;
-#pragma unroll
-            for (int h = 0; h < 2 * N; ++h) cp[h] = cpn[h];
-            sp = spn;
+            for (int h = 0; h < 2; ++h) {
+                const v4i a = *(const v4i*)(lds + (64u * wave + 32u * h + r) * rowb + 32u * st + 16u * kh);
+                s1[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b1, s1[h], 0, 0, 0);
+                s0[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b0, s0[h], 0, 0, 0);
+            }
         }
+        const int m = (int)g.moduli[q], half = m >> 1, off = g.offset[q];
+        const float inv = g.inverse[q];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i4 = 0; i4 < 4; ++i4) {
+                // accumulator element 4 i4 + i: entry row 8 i4 + 4 (lane / 32) + i, modulus column lane % 32
+                u32 w1 = 0, w0 = 0;
+                const u32 e = 8u * i4 + 4u * kh;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int T = s1[h][4 * i4 + i] * 256 + s0[h][4 * i4 + i] + off;
+                    int v = T - residue_mul24((int)__builtin_rintf((float)T * inv), m);
+                    v -= v > half ? m : 0;
+                    v += v < -half ? m : 0;
+                    const int neg = -(int)((sg[h] >> (e + i)) & 1u);
+                    v = (v ^ neg) - neg;
+                    const int d0 = (v << 24) >> 24, d1 = (v - d0) >> 8;
+                    w0 |= ((u32)d0 & 0xffu) << (8 * i);
+                    w1 |= ((u32)d1 & 0xffu) << (8 * i);
+                }
+                unsigned char* at = stage + r * DIG_STAGE_ROW + 64u * wave + 32u * h + e;
+                *reinterpret_cast<u32*>(at) = w1;
+                *reinterpret_cast<u32*>(at + 256) = w0;
+            }
         __syncthreads();
-        // chunk j: 16 columns (c16) of band row b of plane pl of modulus qb + qi
-        const u32 chunks = nq * 2u * (u32)nb * 16u;
-        for (u32 j = t; j < chunks; j += 256u) {
-            const u32 c16 = j & 15u, rest = j >> 4, b = rest % (u32)nb, r2 = rest / (u32)nb, pl = r2 & 1u, qi = r2 >> 1;
-            const u32 kk = k0 + 16u * c16;
-            if (kk >= g.Kp) continue;
-            const uint4 dv = *reinterpret_cast<const uint4*>(&stage[qi][pl][16u * c16]);
-            const uint4 bv = *reinterpret_cast<const uint4*>(&bandof[16u * c16]);
-            const u32 b4 = b * 0x01010101u;
-            const uint4 out = make_uint4(dv.x & byte_eq_mask(bv.x, b4), dv.y & byte_eq_mask(bv.y, b4), dv.z & byte_eq_mask(bv.z, b4),
-                                         dv.w & byte_eq_mask(bv.w, b4));
-            int8_t* dst = (pl ? g.d0 : g.d1) + (u64)(qb + qi) * plane + (u64)L->member[b] * g.Kp + kk;
-            *reinterpret_cast<uint4*>(dst) = out;
+        // chunk j: 16 entries (c16) of digit plane pl of modulus qb + qi, written to every band row of their line
+        const u32 nq = g.L - qb < DIG_QB ? g.L - qb : DIG_QB;
+        for (u32 j = t; j < nq * 32u; j += 256u) {
+            const u32 c16 = j & 15u, pl = (j >> 4) & 1u, qi = j >> 5;
+            const u32 line = line0 + 16u * c16 / tk, kk = k0 + 16u * c16 % tk;
+            if (line >= S.nlines || kk >= g.Kp || S.lines[line].cls != 0) continue;
+            const GemmLine* L = S.lines + line;
+            const uint4 dv = *reinterpret_cast<const uint4*>(stage + qi * DIG_STAGE_ROW + 256u * pl + 16u * c16);
+            int8_t* plane = (pl ? S.d0 : S.d1) + (u64)(qb + qi) * S.rows_p * g.Kp + kk;
+            if (g.joined || L->nb == 1) {
+                *reinterpret_cast<uint4*>(plane + (u64)L->member[0] * g.Kp) = dv;
+                continue;
+            }
+            const uint4 bv = *reinterpret_cast<const uint4*>(bandof + 16u * c16);
+            for (int b = 0; b < L->nb; ++b) {
+                const u32 b4 = (u32)b * 0x01010101u;
+                *reinterpret_cast<uint4*>(plane + (u64)L->member[b] * g.Kp) =
+                    make_uint4(dv.x & byte_eq_mask(bv.x, b4), dv.y & byte_eq_mask(bv.y, b4), dv.z & byte_eq_mask(bv.z, b4),
+                               dv.w & byte_eq_mask(bv.w, b4));
+            }
         }
         __syncthreads();
     }
@@ -149,8 +187,8 @@ template <int N> __global__ void __launch_bounds__(256) digits_kernel(DigitsArgs
 // factor still applied here): 67-word rows 300 us scalar against 173 us staged; 39-word rows 500 us scalar
 // against 531 us staged.
 constexpr int CRT_LDS_MIN_WX = 48;
-template <int WX>
-__device__ __forceinline__ int crt_rebuild(const RebuildArgs& g, const u32* tab, u32 row, u32 col, u32 (&X)[WX])
+template <int WX, class Args>
+__device__ __forceinline__ int crt_rebuild(const Args& g, const u32* tab, u32 row, u32 col, u32 (&X)[WX])
 {
     // tab (LDS, when WX >= CRT_LDS_MIN_WX): the L rows of WX CRT words
     constexpr bool STAGED = WX >= CRT_LDS_MIN_WX;
@@ -325,6 +363,41 @@ template <int WX> __device__ __forceinline__ int read_stage(const RebuildArgs& g
 #pragma unroll
     for (int w = 0; w < WX; ++w) X[w] = src[w * wstride];
     return (int)src[WX * wstride];
+}
+
+// One pass from the residues to the rounded output where every line is one band: nothing is staged between the
+// CRT and the rounding.  One lane an output, outputs of one row a workgroup: 256 where the CRT words are staged
+// in LDS for the workgroup, else 64, so that a small product spreads over the GPU.
+constexpr u32 round_block(int wx) { return wx >= CRT_LDS_MIN_WX ? 256u : 64u; }
+template <int N, int WX> __global__ void __launch_bounds__(round_block(WX)) crt_round_kernel(RoundArgs g)
+{
+    constexpr int WXP = (WX + 3) & ~3;
+    constexpr u32 ROUND_BLOCK = round_block(WX);
+    extern __shared__ __attribute__((aligned(16))) u32 tab[];
+    const u32 nblocks = (g.n + ROUND_BLOCK - 1) / ROUND_BLOCK;
+    const u32 i = blockIdx.x / nblocks, j0 = (blockIdx.x % nblocks) * ROUND_BLOCK, j = j0 + threadIdx.x;
+    if (g.syrk && j0 > i) return; // the whole workgroup lies above the diagonal
+    if constexpr (WX >= CRT_LDS_MIN_WX) {
+        for (u32 k = threadIdx.x; k < g.L * WXP; k += ROUND_BLOCK) {
+            const u32 q = k / WXP, w = k % WXP;
+            tab[k] = w < (u32)WX ? g.crt[q * WX + w] : 0u;
+        }
+        __syncthreads();
+    }
+    if (j >= g.n || (g.syrk && j > i)) return;
+    const bool mirror = g.syrk && !g.lower_only;
+    const GemmLine* Li = g.left + i;
+    const GemmLine* Lj = g.right + j;
+    if (Li->cls == 1 || Lj->cls == 1) { // zero or status line
+        store_out<N>(g.out, g.out_pitch, g.out_stride, i, j, mirror, zero<N>(Li->status | Lj->status));
+        return;
+    }
+    if (Li->cls != 0 || Lj->cls != 0) return; // exact dot kernels
+    u32 X[WX];
+    // a SYRK's members are in line order, so the row's is the larger: the product's lower triangle
+    const int sg = crt_rebuild<WX>(g, tab, (u32)Li->member[0], (u32)Lj->member[0], X);
+    const i64 scale = (i64)Li->low + Lj->low - 2 * (32 * N - 1) - g.t;
+    store_out<N>(g.out, g.out_pitch, g.out_stride, i, j, mirror, pack<N, WX>(X, scale, sg, ST_OK));
 }
 
 // WX: CRT integer words (M' normalised to bit 32(WX-1)-1); ACC: multi-band accumulator words (kept in LDS,

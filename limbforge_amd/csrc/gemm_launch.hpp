@@ -13,6 +13,7 @@ constexpr int rebuild_words(int N, int cls) { return cls == 0 ? 2 * N + 7 : 2 * 
 constexpr int dot_window_words(int cls) { return cls == 0 ? 64 : 128; }
 
 template <int N> hipError_t launch_digits(const DigitsArgs& g, hipStream_t s);
+template <int N> hipError_t launch_round(int wx_class, const RoundArgs& g, hipStream_t s);
 template <int N> hipError_t launch_rebuild(int wx_class, const RebuildArgs& g, hipStream_t s);
 template <int N> hipError_t launch_dot(int window_class, const DotArgs& g, hipStream_t s);
 template <int N> hipError_t launch_cluster_size(const DotArgs& g, uint32_t* words, hipStream_t s);

@@ -10,10 +10,32 @@ namespace lf {
 
 template <int N> hipError_t launch_digits(const DigitsArgs& g, hipStream_t s)
 {
-    if (!g.K || !g.nlines || !g.L) return hipSuccess;
-    if (g.Kp % 16u) return hipErrorInvalidValue; // rows are written in 16-byte chunks
-    hipLaunchKernelGGL((digits_kernel<N>), dim3(((g.Kp + 255u) / 256u) * g.nlines), dim3(256), 0, s, g);
+    const u32 blocks = g.side[0].blocks + g.side[1].blocks;
+    if (!g.K || !blocks || !g.L) return hipSuccess;
+    if (g.Kp % 32u || g.bytes % 32u || g.bytes > DIGIT_TABLE_BYTES) return hipErrorInvalidValue;
+    const u64 lds = digits_lds_bytes(g.bytes);
+    if (lds > (u64(64) << 10))
+        if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&digits_kernel<N>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
+            return e;
+    hipLaunchKernelGGL((digits_kernel<N>), dim3(blocks), dim3(256), lds, s, g);
     return hipGetLastError();
+}
+
+template <int N, int WX> hipError_t launch_round_wx(const RoundArgs& g, hipStream_t s)
+{
+    const u64 lds = crt_table_bytes(g.L, WX);
+    if (lds > (u64(64) << 10))
+        if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&crt_round_kernel<N, WX>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
+            return e;
+    constexpr u32 RB = round_block(WX);
+    hipLaunchKernelGGL((crt_round_kernel<N, WX>), dim3(((g.n + RB - 1) / RB) * g.m), dim3(RB), lds, s, g);
+    return hipGetLastError();
+}
+
+template <int N> hipError_t launch_round(int wx_class, const RoundArgs& g, hipStream_t s)
+{
+    if (!g.m || !g.n) return hipSuccess;
+    return wx_class == 0 ? launch_round_wx<N, rebuild_words(N, 0)>(g, s) : launch_round_wx<N, rebuild_words(N, 1)>(g, s);
 }
 
 template <int N> hipError_t launch_rebuild(int wx_class, const RebuildArgs& g, hipStream_t s)
@@ -57,6 +79,7 @@ hipError_t launch_cluster_sum(const DotArgs& g, const uint32_t* words, const uin
 }
 
 template hipError_t launch_digits<LF_WORDS>(const DigitsArgs&, hipStream_t);
+template hipError_t launch_round<LF_WORDS>(int, const RoundArgs&, hipStream_t);
 template hipError_t launch_rebuild<LF_WORDS>(int, const RebuildArgs&, hipStream_t);
 template hipError_t launch_dot<LF_WORDS>(int, const DotArgs&, hipStream_t);
 template hipError_t launch_cluster_size<LF_WORDS>(const DotArgs&, uint32_t*, hipStream_t);
