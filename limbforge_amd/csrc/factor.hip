@@ -229,13 +229,14 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
     const uint64_t threads = std::max<uint64_t>(n, LOOKAHEAD_WAVES);
     if (2 * swords * threads * 4 > (uint64_t(32) << 30))
         return fail(LF_INVALID_ARGUMENT, "cholesky: the block is too large for the exact-dot scratch (use a smaller block)");
-    FACTOR_HIP(dinfo.alloc(sizeof(lf::FactorInfo)), "hipMalloc (pivot)");
+    FACTOR_HIP(dinfo.alloc(sizeof(lf::FactorInfo) + 4), "hipMalloc (pivot)");
     FACTOR_HIP(dscratch.alloc(2 * swords * threads * 4), "hipMalloc (scratch)");
     // reciprocals of the pivots (up to N+3 planes of n entries), for the divisions of the rows below each block
     DevBuf drecip;
     const uint64_t rpitch = (n + 63) / 64 * 64;
     FACTOR_HIP(drecip.alloc((N + 3) * rpitch * 4), "hipMalloc (reciprocals)");
-    // the pivot record comes back through pinned memory, so that reading it does not wait on the stream
+    // a failed pivot is written to pinned memory by the kernel that finds it; the host reads the record after the
+    // block's event, with no copy on the stream
     struct PinnedInfo {
         lf::FactorInfo* p = nullptr;
         ~PinnedInfo()
@@ -244,8 +245,10 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
         }
     } hinfo;
     FACTOR_HIP(hipHostMalloc((void**)&hinfo.p, sizeof(lf::FactorInfo), hipHostMallocDefault), "hipHostMalloc (pivot)");
-    *hinfo.p = lf::FactorInfo{-1, 0, 0, 0, 0};
+    *hinfo.p = lf::FactorInfo{-1, 0, 0, 0};
+    int32_t* derror = (int32_t*)((lf::FactorInfo*)dinfo.p + 1);
     FACTOR_HIP(hipMemcpyAsync(dinfo.p, hinfo.p, sizeof(lf::FactorInfo), hipMemcpyHostToDevice, s), "upload pivot");
+    FACTOR_HIP(hipMemsetAsync(derror, 0, 4, s), "hipMemsetAsync");
     // Look-ahead (the reference overlaps the next panel with the rest of the update on a second host thread,
     // linalg.mm:440-452): after the panel of block [k0, k1), the entries of the next panel's columns
     // [k1, k2) are updated by a look-ahead kernel on stream s, the next panel follows on s, and the rest of
@@ -253,92 +256,75 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
     // still gets one rounding of the same exact value per block, so the bits are those of the serial order.
     OwnedStream upd;
     FACTOR_HIP(hipStreamCreateWithFlags(&upd.s, hipStreamNonBlocking), "hipStreamCreate");
-    hipEvent_t ev[6];
-    for (auto& e : ev) e = nullptr;
+    // events: the start and end of each block's kernels on s (the even and the odd block), the rest of an update
+    hipEvent_t ev[5] = {};
     struct EventsGuard {
         hipEvent_t* e;
         ~EventsGuard()
         {
-            for (int i = 0; i < 6; ++i)
+            for (int i = 0; i < 5; ++i)
                 if (e[i]) (void)hipEventDestroy(e[i]);
         }
     } guard{ev};
     for (auto& e : ev) FACTOR_HIP(hipEventCreate(&e), "hipEventCreate");
-    hipEvent_t &p0 = ev[0], &p1 = ev[1], &panel_done = ev[2], &rest_done = ev[3], &l0 = ev[4], &l1 = ev[5];
+    hipEvent_t *begun = ev, *done = ev + 2, &rest_done = ev[4];
     const uint32_t waves = uint32_t(threads);
     bool rest_pending = false;
-    auto args = [&](uint64_t a, uint64_t b) {
-        return lf::FactorArgs{W, pitch, n32, uint32_t(a), uint32_t(b), (lf::FactorInfo*)dinfo.p, (uint32_t*)dscratch.p, swords,
-                              (uint32_t*)drecip.p, rpitch};
-    };
-    // the panel of block [a, b) on s, its pivot record on its way to the host, panel_done recorded
-    auto panel = [&](uint64_t a, uint64_t b) -> int {
-        const lf::FactorArgs f = args(a, b);
-        FACTOR_HIP(hipEventRecord(p0, s), "hipEventRecord");
+    // the panel of block number q, [a, b), on s, done[q & 1] recorded
+    auto panel = [&](uint64_t q, uint64_t a, uint64_t b) -> int {
+        const lf::FactorArgs f{W, pitch, n32, uint32_t(a), uint32_t(b), (lf::FactorInfo*)dinfo.p, hinfo.p, derror, (uint32_t*)dscratch.p, swords,
+                               (uint32_t*)drecip.p, rpitch};
         FACTOR_HIP(tables().diag[N](f, uint32_t(std::min<uint64_t>(256, (b - a + 63) / 64 * 64)), s), "panel launch");
         // the rows below: row i is the right-hand side of L_block l_i = a_i
         const lf::TriArgs t{W, pitch, int64_t(a * n + a), int64_t(n), 1, W, pitch, int64_t(b * n + a), 1, int64_t(n), (const uint32_t*)drecip.p,
-                            rpitch, int64_t(a), 1, uint32_t(b - a), uint32_t(n - b), (uint32_t*)dscratch.p, swords, &f.info->error, f.info,
-                            uint32_t(a)};
+                            rpitch, int64_t(a), 1, uint32_t(b - a), uint32_t(n - b), (uint32_t*)dscratch.p, swords, derror, f.info, uint32_t(a)};
         FACTOR_HIP(tables().tri_block[N](t, s), "panel launch");
-        FACTOR_HIP(hipEventRecord(p1, s), "hipEventRecord");
-        FACTOR_HIP(hipMemcpyAsync(hinfo.p, dinfo.p, sizeof(lf::FactorInfo), hipMemcpyDeviceToHost, s), "download pivot");
-        FACTOR_HIP(hipEventRecord(panel_done, s), "hipEventRecord");
+        FACTOR_HIP(hipEventRecord(done[q & 1], s), "hipEventRecord");
         return LF_OK;
     };
-    // waits for the panel just enqueued; LF_OK and `failed` set when its pivot failed
-    auto finish_panel = [&](Clock::time_point t, bool& failed) -> int {
-        FACTOR_HIP(hipEventSynchronize(panel_done), "device execution (panel)");
+    // waits for block q's panel; LF_OK and `failed` set when its pivot failed
+    auto finish_panel = [&](uint64_t q, Clock::time_point t, bool& failed) -> int {
+        FACTOR_HIP(hipEventSynchronize(done[q & 1]), "device execution (panel)");
         float ms = 0;
-        FACTOR_HIP(hipEventElapsedTime(&ms, p0, p1), "hipEventElapsedTime");
+        FACTOR_HIP(hipEventElapsedTime(&ms, begun[q & 1], done[q & 1]), "hipEventElapsedTime");
         ci.timing_gpu_seconds += ms * 1e-3;
         ci.panel_seconds += since(t);
         ++ci.blocks;
-        if (hinfo.p->error) return fail(LF_LOGIC_ERROR, "cholesky: exact-dot scratch overflow");
-        failed = hinfo.p->pivot >= 0;
-        if (failed) {
-            ci.pivot = uint64_t(hinfo.p->pivot);
-            ci.pivot_sign = hinfo.p->sign;
-            ci.pivot_status = hinfo.p->status;
-            if (rest_pending) FACTOR_HIP(hipStreamWaitEvent(s, rest_done, 0), "hipStreamWaitEvent");
-            FACTOR_HIP(tables().invalid[N](W, pitch, n32, uint32_t(hinfo.p->pivot), s), "invalid launch");
-            FACTOR_HIP(hipStreamSynchronize(s), "device execution");
-        }
+        const int32_t pivot = ((volatile lf::FactorInfo*)hinfo.p)->pivot;
+        failed = pivot >= 0 && uint64_t(pivot) < std::min<uint64_t>(n, (q + 1) * nb);
         return LF_OK;
     };
-    {
-        const auto t = Clock::now();
-        if (int r = panel(0, std::min(n, nb))) return r;
-        bool failed = false;
-        if (int r = finish_panel(t, failed)) return r;
-        if (failed) {
-            ci.timing_wall_seconds = since(start);
-            if (info) *info = ci;
-            return LF_OK;
-        }
-    }
-    for (uint64_t k0 = 0; k0 < n;) {
+    // A block's pivot is looked at after the next block's kernels are on the streams, so that s does not wait for the
+    // host: past a failed pivot those kernels leave the panels alone, and what they update is marked invalid here.
+    auto t = Clock::now();
+    FACTOR_HIP(hipEventRecord(begun[0], s), "hipEventRecord");
+    if (int r = panel(0, 0, std::min(n, nb))) return r;
+    bool failed = false;
+    uint64_t q = 0; // the block whose panel is on s and not yet looked at
+    for (uint64_t k0 = 0;; k0 += nb, ++q) {
         const uint64_t k1 = std::min(n, k0 + nb), w = k1 - k0;
-        if (k1 >= n) break;
-        const uint64_t k2 = std::min(n, k1 + nb);
-        // (1) the next panel's columns, after the previous block's rest of the update
-        auto t = Clock::now();
-        if (rest_pending) FACTOR_HIP(hipStreamWaitEvent(s, rest_done, 0), "hipStreamWaitEvent");
-        FACTOR_HIP(hipEventRecord(l0, s), "hipEventRecord");
-        // the entries (i, j), j <= i, of columns [k1, k2) and rows [k1, n), in place
-        const lf::UpdateArgs ua{W, pitch, int64_t(k1 * n + k0), int64_t(n), 1, W, pitch, int64_t(k1 * n + k0), int64_t(n), 1, W, pitch,
-                                int64_t(k1 * n + k1), int64_t(n), 1, uint32_t(n - k1), uint32_t(k2 - k1), uint32_t(w), 1, (uint32_t*)dscratch.p, swords,
-                                &((lf::FactorInfo*)dinfo.p)->error};
-        FACTOR_HIP(tables().update[N](ua, waves, s), "look-ahead launch");
-        FACTOR_HIP(hipEventRecord(l1, s), "hipEventRecord");
-        // (2) the next panel on s
-        const auto tp = Clock::now();
-        if (int r = panel(k1, k2)) return r;
-        // (3) the rest of this block's update on the second stream, after this block's panel (the look-ahead
-        // and the next panel write only columns [k1, k2), which this part neither reads nor writes)
+        if (k1 < n) {
+            const uint64_t k2 = std::min(n, k1 + nb);
+            // (1) the next panel's columns, after the previous block's rest of the update
+            if (rest_pending) FACTOR_HIP(hipStreamWaitEvent(s, rest_done, 0), "hipStreamWaitEvent");
+            FACTOR_HIP(hipEventRecord(begun[(q + 1) & 1], s), "hipEventRecord");
+            // the entries (i, j), j <= i, of columns [k1, k2) and rows [k1, n), in place
+            const lf::UpdateArgs ua{W, pitch, int64_t(k1 * n + k0), int64_t(n), 1, W, pitch, int64_t(k1 * n + k0), int64_t(n), 1, W, pitch,
+                                    int64_t(k1 * n + k1), int64_t(n), 1, uint32_t(n - k1), uint32_t(k2 - k1), uint32_t(w), 1,
+                                    (uint32_t*)dscratch.p, swords, derror};
+            FACTOR_HIP(tables().update[N](ua, waves, s), "look-ahead launch");
+            // (2) the next panel on s
+            if (int r = panel(q + 1, k1, k2)) return r;
+        }
+        const auto tn = Clock::now();
+        // (3) this block's pivot
+        if (int r = finish_panel(q, t, failed)) return r;
+        if (failed || k1 >= n) break;
+        t = tn;
+        // (4) the rest of this block's update on the second stream, after this block's panel (the look-ahead and the
+        // next panel write only columns [k1, k2), which this part neither reads nor writes)
         rest_pending = false;
-        if (k2 < n) {
-            FACTOR_HIP(hipStreamWaitEvent(upd.s, l0, 0), "hipStreamWaitEvent");
+        if (const uint64_t k2 = std::min(n, k1 + nb); k2 < n) {
             const lf::MatView v{W + (k2 * n + k0), pitch, n, 1};
             float ms = 0;
             if (int r = update(bits, lo, true, v, v, n - k2, n - k2, w, W + (k2 * n + k2), pitch, n, upd.s, ms)) return r;
@@ -347,18 +333,20 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
             ci.timing_gpu_seconds += ms * 1e-3;
             ++ci.gpu_updates;
         }
-        ci.update_seconds += since(t);
-        {
-            float ms = 0;
-            FACTOR_HIP(hipEventSynchronize(l1), "device execution (look-ahead)");
-            FACTOR_HIP(hipEventElapsedTime(&ms, l0, l1), "hipEventElapsedTime");
-            ci.timing_gpu_seconds += ms * 1e-3;
-        }
-        // (4) the next panel's pivot
-        bool failed = false;
-        if (int r = finish_panel(tp, failed)) return r;
-        if (failed) break;
-        k0 = k1;
+        ci.update_seconds += since(tn);
+    }
+    if (failed) {
+        const lf::FactorInfo i = *hinfo.p;
+        ci.pivot = uint64_t(i.pivot);
+        ci.pivot_sign = i.sign;
+        ci.pivot_status = i.status;
+        FACTOR_HIP(tables().invalid[N](W, pitch, n32, uint32_t(i.pivot), s), "invalid launch");
+    }
+    {
+        int32_t error = 0;
+        FACTOR_HIP(hipMemcpyAsync(&error, derror, 4, hipMemcpyDeviceToHost, s), "download status");
+        FACTOR_HIP(hipStreamSynchronize(s), "device execution");
+        if (error) return fail(LF_LOGIC_ERROR, "cholesky: exact-dot scratch overflow");
     }
     if (rest_pending) FACTOR_HIP(hipStreamSynchronize(upd.s), "device execution (update)");
     ci.timing_wall_seconds = since(start);
@@ -406,8 +394,8 @@ int lf_solve(int bits, int passes, const lf_operand* L, uint64_t n, const lf_ope
     FACTOR_HIP(drecip.alloc((N + 3) * rpitch * 4), "hipMalloc (reciprocals)");
     FACTOR_HIP(tables().reciprocals[N](F, fpitch, uint32_t(n), (uint32_t*)drecip.p, rpitch, s), "reciprocals launch");
     double gpu = 0;
-    // device time: an event pair around every in-block kernel and direct update, read after the last
-    // synchronization (the update GEMM reports its own kernels' time)
+    // device time, where it is asked for: an event pair around each run of in-block kernels and direct updates, read
+    // after the last synchronization (the update GEMM reports its own kernels' time)
     struct Events {
         std::vector<hipEvent_t> e;
         ~Events()
@@ -415,16 +403,16 @@ int lf_solve(int bits, int passes, const lf_operand* L, uint64_t n, const lf_ope
             for (auto x : e) (void)hipEventDestroy(x);
         }
     } events;
+    auto mark = [&](bool begin) -> hipError_t {
+        if (!gpu_seconds || begin != (events.e.size() % 2 == 0)) return hipSuccess; // (already in, or out of, a run)
+        hipEvent_t x = nullptr;
+        if (hipError_t e = hipEventCreate(&x)) return e;
+        events.e.push_back(x);
+        return hipEventRecord(x, s);
+    };
     auto timed = [&](auto&& launch) -> hipError_t {
-        hipEvent_t a = nullptr, b = nullptr;
-        hipError_t e = hipEventCreate(&a);
-        if (e != hipSuccess) return e;
-        events.e.push_back(a);
-        if ((e = hipEventCreate(&b)) != hipSuccess) return e;
-        events.e.push_back(b);
-        if ((e = hipEventRecord(a, s)) != hipSuccess) return e;
-        if ((e = launch()) != hipSuccess) return e;
-        return hipEventRecord(b, s);
+        if (hipError_t e = mark(true)) return e;
+        return launch();
     };
     // row r of the block is row r0 + r of L going forward, and row r1 - 1 - r of L^T (column of L) going backward
     auto block_solve = [&](int backward, uint64_t r0, uint64_t r1) {
@@ -462,6 +450,7 @@ int lf_solve(int bits, int passes, const lf_operand* L, uint64_t n, const lf_ope
                 FACTOR_HIP(dot_update(0, r0, r1), "solve update launch");
                 continue;
             }
+            FACTOR_HIP(mark(false), "hipEventRecord");
             const lf::MatView left{F + (r1 * n + r0), fpitch, n, 1}, right{Xp + r0 * nrhs, xpitch, 1, nrhs};
             if (int r = update(bits, lo, false, left, right, n - r1, nrhs, K, Xp + r1 * nrhs, xpitch, nrhs, s, ms)) return r;
             gpu += ms * 1e-3;
@@ -476,10 +465,12 @@ int lf_solve(int bits, int passes, const lf_operand* L, uint64_t n, const lf_ope
                 FACTOR_HIP(dot_update(1, r0, r1), "solve update launch");
                 continue;
             }
+            FACTOR_HIP(mark(false), "hipEventRecord");
             const lf::MatView left{F + r0 * n, fpitch, 1, n}, right{Xp + r0 * nrhs, xpitch, 1, nrhs};
             if (int r = update(bits, lo, false, left, right, r0, nrhs, K, Xp, xpitch, nrhs, s, ms)) return r;
             gpu += ms * 1e-3;
         }
+    FACTOR_HIP(mark(false), "hipEventRecord");
     int32_t err = 0;
     FACTOR_HIP(hipMemcpyAsync(&err, derr.p, 4, hipMemcpyDeviceToHost, s), "download status");
     FACTOR_HIP(hipStreamSynchronize(s), "device execution (solve)");

@@ -237,7 +237,7 @@ __device__ __forceinline__ int wave_or(int v)
 
 // The value of lane l - 1 in lane l (0 in lane 0): a DPP wave shift right by one lane (wave_shr:1), at ALU
 // latency where a shuffle goes through LDS.  Every lane of the wave must be active.
-__device__ __forceinline__ u32 wave_from_previous_lane(u32 v) { return (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xF, 0xF, false); }
+__device__ __forceinline__ u32 wave_from_previous_lane(u32 v) { return (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x138, 0xF, 0xF, true); }
 
 // Maximum (MAX) or minimum of a 32-bit value over the 64 lanes of the wave, in every lane: DPP row shifts by
 // 1, 2, 4 and 8 leave each row's reduction in its lane 15, the row broadcasts of lanes 15 and 31 carry it to
@@ -584,16 +584,19 @@ template <int N> __global__ void __launch_bounds__(diag_waves<N>() * WAVE) chol_
     __shared__ int stop;
     const u32 wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     WaveLds<N>& L = lds[wave];
-    const DotScratch sc{f.scratch + (u64)wave * 2 * f.swords, f.swords, &f.info->error};
+    const DotScratch sc{f.scratch + (u64)wave * 2 * f.swords, f.swords, f.error};
+    if (f.info->pivot >= 0) return; // a block before this one failed
     for (u32 j = f.k0 + (resume ? (u32)f.info->resume : 0u); j < f.k1; ++j) {
         const VecView rj{f.w, f.pitch, (i64)j * f.n + f.k0, 1};
         if (wave == 0) {
             const Num<N> s = wave_dot_sub<N>(element<N>(f, j, j), rj, rj, j - f.k0, lane, L, sc);
             if (lane == 0) {
                 if (s.st || s.s <= 0) {
-                    f.info->pivot = (int32_t)j;
-                    f.info->sign = s.st ? 0 : s.s;
-                    f.info->status = s.st;
+                    const FactorInfo i{(int32_t)j, s.st ? 0 : s.s, s.st, 0};
+                    f.info->sign = i.sign;
+                    f.info->status = i.status;
+                    f.info->pivot = i.pivot;
+                    *f.host = i;
                     stop = 1;
                 } else {
                     store_out<N>(f.w, f.pitch, f.n, j, j, false, sqrt<N>(s));
@@ -644,26 +647,29 @@ template <int N> __global__ void __launch_bounds__(256) zero_upper_kernel(u32* w
 // is one wavefront's instruction count: at 256 bits a 32-row block took 163-167 us with the general recurrence
 // (an exact dot of the row's terms and a one-lane division per row).  With a digit per lane the solve of 512
 // unknowns and 64 right-hand sides went from 7.70 to 4.00 ms, the factorization of n = 512 from 12.3 to 10.9 ms.
-template <int N> __global__ void __launch_bounds__(64) tri_block_kernel(TriArgs g)
+template <int N> constexpr u32 tri_waves() { return wd_fits<N>() ? TRI_WAVES : 1; }
+template <int N> __global__ void __launch_bounds__(64 * tri_waves<N>()) tri_block_kernel(TriArgs g)
 {
-    constexpr std::size_t bytes = wd_fits<N>() && sizeof(TriLds<N>) > sizeof(WaveLds<N>) ? sizeof(TriLds<N>) : sizeof(WaveLds<N>);
+    constexpr std::size_t bytes = wd_fits<N>() ? sizeof(TriLds<N>) : sizeof(WaveLds<N>);
     __shared__ __attribute__((aligned(16))) unsigned char lds[bytes];
-    const u32 c = blockIdx.x, lane = threadIdx.x;
+    const u32 wave = threadIdx.x / 64u, lane = threadIdx.x % 64u, c = blockIdx.x * tri_waves<N>() + wave;
     u32 B = g.rows;
     if (g.info) {
         const int32_t p = g.info->pivot;
-        if (p >= 0) B = (u32)p - g.k0;
+        if (p >= 0) B = (u32)p > g.k0 ? (u32)p - g.k0 : 0u; // (nothing where an earlier block failed)
     }
     u32 i = 0;
     if constexpr (wd_fits<N>())
-        if (B <= WD_ROWS) i = tri_block_fast<N>(g, c, B, lane, *reinterpret_cast<TriLds<N>*>(lds));
-    if (i >= B) return;
-    __syncthreads(); // the rows stored so far are terms of the next
-    WaveLds<N>& L = *reinterpret_cast<WaveLds<N>*>(lds);
+        if (B <= WD_ROWS) i = tri_block_fast<N>(g, c, B, wave, lane, *reinterpret_cast<TriLds<N>*>(lds));
+    if (i >= B || c >= g.count) return;
+    // the general recurrence, in the LDS of this wavefront's accumulators; its own stores are terms of later rows
+    static_assert(!wd_fits<N>() || sizeof(WaveLds<N>) <= sizeof(i64) * WD_ROWS * (WD_COLS + 1), "the exact dot's rows fit the accumulators");
+    WaveLds<N>& L = *reinterpret_cast<WaveLds<N>*>(lds + wave * sizeof(i64) * WD_ROWS * (WD_COLS + 1));
     const DotScratch sc{g.scratch + (u64)c * 2 * g.swords, g.swords, g.error};
     const i64 xb = g.xbase + (i64)c * g.xc;
     const VecView xv{g.x, g.xpitch, xb, g.xr};
     for (; i < B; ++i) {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         const VecView li{g.f, g.fpitch, g.fbase + (i64)i * g.fr, g.fk};
         const u64 at = (u64)(xb + (i64)i * g.xr);
         const Num<N> v = wave_dot_sub<N>(load_out<N>(g.x, g.xpitch, at), li, xv, i, lane, L, sc);
@@ -673,7 +679,6 @@ template <int N> __global__ void __launch_bounds__(64) tri_block_kernel(TriArgs 
             const Num<N> l = load_out<N>(g.f, g.fpitch, (u64)(g.fbase + (i64)i * (g.fr + g.fk)));
             store_out<N>(g.x, g.xpitch, 0, 0, (u32)at, false, div_by_reciprocal<N>(v, l, rv));
         }
-        __syncthreads(); // x_i is a term of the next row's dot
     }
 }
 

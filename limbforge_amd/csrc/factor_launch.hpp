@@ -10,7 +10,6 @@ struct FactorInfo {
     int32_t pivot;   // first failing column, -1 while none
     int32_t sign;    // sign of the failing s_pp (0 for zero or a status)
     uint32_t status; // its status
-    int32_t error;   // cluster scratch overflow (never expected)
     int32_t resume;  // columns of the block that the wave-parallel diagonal kernel decided
 };
 
@@ -19,6 +18,8 @@ struct FactorArgs {
     uint64_t pitch;
     uint32_t n, k0, k1;
     FactorInfo* info;
+    FactorInfo* host;  // a failed pivot's record in pinned host memory (read only after the block's event)
+    int32_t* error;    // cluster scratch overflow (never expected)
     uint32_t* scratch; // per thread: 2 * swords words
     uint64_t swords;
     uint32_t* recip;   // reciprocals of the pivots l_jj (up to N+3 planes, entry j), written by the diagonal kernel

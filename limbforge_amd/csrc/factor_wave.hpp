@@ -38,7 +38,7 @@ constexpr int WD_TOP = 61;
 template <int N> constexpr int recip_words() { return wd_fits<N>() ? N + 3 : N + 1; }
 
 // The value of lane l + 1 in lane l (0 in lane 63): DPP wave_shl:1.  Every lane must be active.
-__device__ __forceinline__ u32 wave_from_next_lane(u32 v) { return (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xF, 0xF, false); }
+__device__ __forceinline__ u32 wave_from_next_lane(u32 v) { return (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x130, 0xF, 0xF, true); }
 
 __device__ __forceinline__ u32 wd_read(u32 v, int lane) { return (u32)__builtin_amdgcn_readlane((int)v, lane); }
 
@@ -133,11 +133,11 @@ template <int N> __device__ __forceinline__ bool wd_round(i64 S, i64 alpha, u32 
     return r.e <= EMAX && r.e >= -(i64)EMAX;
 }
 
-// RN(a / b) from the reciprocal R = floor((2^P - 1) / B), P = 64N + 64, of b's mantissa, given as Rs[i] =
-// digit lane - i of R (0 outside it); be, bs: b's exponent and sign.  With V = A R the quotient 2^P A / B lies
-// in [V, V + 2^(32N)]: its top 32N + 1 bits are V's unless the rounding bit is 0 and every bit between it
-// and 2^(32N) is 1 (24 of them are looked at: about one division in 2^24 takes the general routine).  A
-// quotient of two 32N-bit mantissas is never halfway between two others, so a set rounding bit rounds up.
+// RN(a / b) from the reciprocal R of b's mantissa, 2^P / B to within 2^30 units, P = 64N + 64, given as Rs[i] =
+// digit lane - i of R (0 outside it); be, bs: b's exponent and sign.  V = A R is 2^P A / B to within 2^(32N + 30),
+// and the quotient's last place is 2^(32N + 64) or more: the rounding bit tells, unless it and the 23 bits below it
+// are 0111...1 or 1000...0 (about one division in 2^23 takes the general routine).  A quotient of two 32N-bit
+// mantissas is never halfway between two others, so a set rounding bit rounds up.
 template <int N>
 __device__ __forceinline__ bool wd_divide(const WaveNum& a, const u32 (&Rs)[wd_mant<N>()], i64 be, int bs, u32 lane, WaveNum& q)
 {
@@ -154,7 +154,7 @@ __device__ __forceinline__ bool wd_divide(const WaveNum& a, const u32 (&Rs)[wd_m
     q.e = a.e - be - (ge ? 0 : 1);
     q.s = a.s * bs;
     const u32 g = wd_below(V, sigma);
-    if (g == 0x7fffffu) return false;
+    if (g == 0x7fffffu || g == 0x800000u) return false;
     if (g >> 23) q.m = wd_increment<N>(q.m, q.e, lane);
     return q.e <= EMAX && q.e >= -(i64)EMAX;
 }
@@ -184,11 +184,15 @@ template <int N> __device__ __forceinline__ u32 wd_word(u32 m, u32 lane)
     return (u32)(v >> s);
 }
 
-// Stores a wave number at plane element `at` (lane w writes plane w).
+// Plane `lane` of a wave number's record (lanes below N + 3), and the record stored at plane element `at`.
+template <int N> __device__ __forceinline__ u32 wd_record_word(const WaveNum& x, u32 lane)
+{
+    const u32 v = wd_word<N>(x.m, lane);
+    return lane == (u32)N ? (u32)(int)x.e : lane == (u32)N + 1 ? (u32)x.s : lane == (u32)N + 2 ? 0u : v;
+}
 template <int N> __device__ __forceinline__ void wd_store(u32* planes, u64 pitch, u64 at, const WaveNum& x, u32 lane)
 {
-    u32 v = wd_word<N>(x.m, lane);
-    v = lane == (u32)N ? (u32)(int)x.e : lane == (u32)N + 1 ? (u32)x.s : lane == (u32)N + 2 ? 0u : v;
+    const u32 v = wd_record_word<N>(x, lane);
     if (lane < (u32)N + 3) planes[(u64)lane * pitch + at] = v;
 }
 
@@ -228,18 +232,20 @@ template <int N, int M> __device__ __forceinline__ void reciprocal_words(const u
 }
 
 // ------------------------------------------------------------------ triangular blocks
-// LDS of one wavefront's block: the rows' accumulators (an odd number of 64-bit columns a row, so that lanes
-// adding at the same column of their rows hit distinct banks), the signed grid digits of the strict lower
-// triangle packed by columns with their origins (zero entries: WD_ZERO), and the reciprocals of the diagonal
-// between zeros, so that lane c reads digit c - i without a bound.
+// LDS of a block: the signed grid digits of the strict lower triangle packed by columns with their origins (zero
+// entries: WD_ZERO), the reciprocals of the diagonal between zeros, so that lane c reads digit c - i without a
+// bound, and for each wavefront, which runs one right-hand side, its rows' accumulators (an odd number of 64-bit
+// columns a row, so that lanes adding at the same column of their rows hit distinct banks).
 constexpr u32 WD_ROWS = 32;
 constexpr int WD_TRI = WD_ROWS * (WD_ROWS - 1) / 2;
 constexpr int WD_ZERO = 0x7fffffff;
+constexpr u32 TRI_WAVES = 4;
 template <int N> struct TriLds {
-    i64 acc[WD_ROWS][WD_COLS + 1];
+    i64 acc[TRI_WAVES][WD_ROWS][WD_COLS + 1];
     int digit[wd_grid<N>()][WD_TRI];
     int origin[WD_TRI];
     u32 recip[WD_ROWS][wd_mant<N>() - 1 + WD_COLS];
+    int odd; // a status in the block, or a zero on its diagonal
 };
 
 // first index of column k of the strict lower triangle: rows k + 1 .. WD_ROWS - 1
@@ -264,27 +270,30 @@ template <int GD, int H> __device__ __forceinline__ void wd_accumulate(i64* at, 
 }
 
 // The recurrence x_r = (b_r - sum_{k<r} l_rk x_k) / l_rr over the rows of a block of up to 32 rows, one
-// rounding of the exact sum and one of the quotient per row, for right-hand side c on one wavefront.
-// Returns the rows done: all of them, or the first one that needs the general routines (a status, a zero
-// divisor, terms spread past the accumulator's columns, a quotient too close to a rounding boundary).
-template <int N> __device__ __forceinline__ u32 tri_block_fast(const TriArgs& g, u32 c, u32 B, u32 lane, TriLds<N>& L)
+// rounding of the exact sum and one of the quotient per row, for right-hand side c on one wavefront of the
+// workgroup.  Returns the rows done: all of them, or the first one that needs the general routines (a status, a
+// zero divisor, terms spread past the accumulator's columns, a quotient too close to a rounding boundary).
+// The block is staged by the whole workgroup: its loads' latency, 16 rounds of them for one wavefront, was about
+// a quarter of the kernel.
+template <int N> __device__ __forceinline__ u32 tri_block_fast(const TriArgs& g, u32 c, u32 B, u32 wave, u32 lane, TriLds<N>& L)
 {
     constexpr int D = wd_mant<N>(), GD = wd_grid<N>(), RD = wd_recip<N>(), H = (GD + 1) / 2;
-    const u32 row = lane & 31u, half = lane >> 5;
+    const u32 t = 64u * wave + lane, row = lane & 31u, half = lane >> 5;
+    const bool mine = c < g.count;
     const u64 xb = (u64)(g.xbase + (i64)c * g.xc);
     {
-        int4* z = reinterpret_cast<int4*>(&L.acc[0][0]);
+        int4* z = reinterpret_cast<int4*>(&L.acc[0][0][0]);
         static_assert(sizeof(L.acc) % 16 == 0, "whole 16-byte chunks");
-        for (u32 k = lane; k < sizeof(L.acc) / 16; k += 64u) z[k] = make_int4(0, 0, 0, 0);
+        for (u32 k = t; k < sizeof(L.acc) / 16; k += 64u * TRI_WAVES) z[k] = make_int4(0, 0, 0, 0);
         u32* r = &L.recip[0][0];
-        for (u32 k = lane; k < sizeof(L.recip) / 4; k += 64u) r[k] = 0u;
+        for (u32 k = t; k < sizeof(L.recip) / 4; k += 64u * TRI_WAVES) r[k] = 0u;
+        if (t == 0) L.odd = 0;
     }
-    wave_sync();
-    bool odd = false; // a status, or a zero on the diagonal
-    for (u32 k = half; k < B; k += 2u)
+    __syncthreads();
+    for (u32 k = t >> 5; k < B; k += 2u * TRI_WAVES)
         if (row > k && row < B) {
             const Num<N> l = load_out<N>(g.f, g.fpitch, (u64)(g.fbase + (i64)row * g.fr + (i64)k * g.fk));
-            odd = odd || l.st != 0;
+            if (l.st) L.odd = 1;
             int d[GD], o;
             lane_to_grid<N>(l, d, o);
             const u32 at = wd_col_start(k) + (row - k - 1);
@@ -294,46 +303,51 @@ template <int N> __device__ __forceinline__ u32 tri_block_fast(const TriArgs& g,
         }
     int le = 0, ls = 0, alpha = 0;
     bool placed = false; // alpha is set: the row has an addend or a term
+    bool odd = false;
     if (lane < B) {
         const u64 at = (u64)(g.fbase + (i64)lane * (g.fr + g.fk));
         le = (int)g.f[(u64)N * g.fpitch + at];
         ls = (int)g.f[(u64)(N + 1) * g.fpitch + at];
-        odd = odd || g.f[(u64)(N + 2) * g.fpitch + at] != 0 || ls == 0;
-        u32 v[N + 3], e[RD + 1];
+        odd = g.f[(u64)(N + 2) * g.fpitch + at] != 0 || ls == 0;
+        if (wave == TRI_WAVES - 1) {
+            u32 v[N + 3];
 #pragma unroll
-        for (int k = 0; k < N + 3; ++k) v[k] = g.recip[(u64)k * g.rpitch + (u64)(g.rbase + (i64)lane * g.rstep)];
+            for (int k = 0; k < N + 3; ++k) v[k] = g.recip[(u64)k * g.rpitch + (u64)(g.rbase + (i64)lane * g.rstep)];
 #pragma unroll
-        for (int j = 0; j < RD; ++j) {
-            const int bit = WD_BITS * j, wi = bit / 32, s = bit % 32;
-            u32 t = wi < N + 3 ? v[wi] >> s : 0u;
-            if (s > 32 - WD_BITS && wi + 1 < N + 3) t |= v[wi + 1] << (32 - s);
-            e[j] = t & WD_MASK;
+            for (int j = 0; j < RD; ++j) {
+                const int bit = WD_BITS * j, wi = bit / 32, s = bit % 32;
+                u32 e = wi < N + 3 ? v[wi] >> s : 0u;
+                if (s > 32 - WD_BITS && wi + 1 < N + 3) e |= v[wi + 1] << (32 - s);
+                L.recip[lane][D - 1 + j] = e & WD_MASK;
+            }
         }
+        if (mine) {
+            const Num<N> b = load_out<N>(g.x, g.xpitch, xb + (u64)((i64)lane * g.xr));
+            odd = odd || b.st != 0;
+            if (b.s) {
+                int d[GD], o;
+                lane_to_grid<N>(b, d, o);
+                alpha = o + GD - 1 - wd_center<N>();
+                placed = true;
 #pragma unroll
-        for (int j = 0; j < RD; ++j) L.recip[lane][D - 1 + j] = e[j];
-        const Num<N> b = load_out<N>(g.x, g.xpitch, xb + (u64)((i64)lane * g.xr));
-        odd = odd || b.st != 0;
-        if (b.s) {
-            int d[GD], o;
-            lane_to_grid<N>(b, d, o);
-            alpha = o + GD - 1 - wd_center<N>();
-            placed = true;
-#pragma unroll
-            for (int j = 0; j < GD; ++j) L.acc[lane][wd_center<N>() - (GD - 1) + j] = b.s < 0 ? -(i64)d[j] : (i64)d[j];
+                for (int j = 0; j < GD; ++j) L.acc[wave][lane][wd_center<N>() - (GD - 1) + j] = b.s < 0 ? -(i64)d[j] : (i64)d[j];
+            }
         }
     }
-    if (__ballot(odd)) return 0;
+    __syncthreads();
+    if (!mine) return B;
+    if (L.odd || __ballot(odd)) return 0;
     // both lanes of a row carry its origin
     alpha = __shfl(alpha, (int)row);
     placed = __shfl((int)placed, (int)row) != 0;
-    wave_sync();
+    i64(&acc)[WD_ROWS][WD_COLS + 1] = L.acc[wave];
     u64 outside = 0; // rows with a term outside their columns
     for (u32 i = 0; i < B; ++i) {
         if ((outside >> i) & 1u) return i;
         u32 Rs[D];
 #pragma unroll
         for (int k = 0; k < D; ++k) Rs[k] = L.recip[i][D - 1 + (int)lane - k];
-        const i64 S = L.acc[i][lane];
+        const i64 S = acc[i][lane];
         WaveNum v, x;
         if (!wd_round<N>(S, (i64)(int)wd_read((u32)alpha, (int)i), lane, v)) return i;
         if (!wd_divide<N>(v, Rs, (i64)(int)wd_read((u32)le, (int)i), (int)wd_read((u32)ls, (int)i), lane, x)) return i;
@@ -360,7 +374,7 @@ template <int N> __device__ __forceinline__ u32 tri_block_fast(const TriArgs& g,
                 int ld[GD];
 #pragma unroll
                 for (int j = 0; j < GD; ++j) ld[j] = L.digit[j][at];
-                wd_accumulate<GD, H>(&L.acc[row][o + H * (int)half], xd, ld);
+                wd_accumulate<GD, H>(&acc[row][o + H * (int)half], xd, ld);
             }
         }
         outside |= __ballot(bad);
