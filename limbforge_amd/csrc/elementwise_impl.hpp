@@ -5,6 +5,7 @@
 #pragma once
 #include "lf_internal.hpp"
 #include "coop_core.hpp"
+#include "div_core.hpp"
 #include "dot2_core.hpp"
 #include "limb_core.hpp"
 
@@ -51,6 +52,14 @@ __device__ __forceinline__ u32 operand_index(u32 i, u32 stride, u32 period)
     return period ? j % period : j;
 }
 
+// i as a value that the compiler cannot relate to i: the operands of the rare quotient that cd_div leaves
+// undecided are loaded again through it, instead of being kept in registers beside the recurrence.
+__device__ __forceinline__ u32 reload_index(u32 i)
+{
+    asm volatile("" : "+v"(i));
+    return i;
+}
+
 template <int N, int OP> __global__ void __launch_bounds__(256) elementwise_kernel(ElemArgs g)
 {
     const u32 i = blockIdx.x * 256u + threadIdx.x;
@@ -62,7 +71,14 @@ template <int N, int OP> __global__ void __launch_bounds__(256) elementwise_kern
         Cpx<N> z;
         if constexpr (OP == OP_CADD) z = cadd<N>(x, y);
         else if constexpr (OP == OP_CMUL) z = cmul<N>(x, y);
-        else if constexpr (OP == OP_CDIV) z = cdiv<N>(x, y);
+        else if constexpr (OP == OP_CDIV) {
+            // the composed division (cdiv): both parts divide by |y|^2
+            const Num<N> d = add<N>(mul<N>(y.re, y.re), mul<N>(y.im, y.im));
+            const Num<N> re = add<N>(mul<N>(x.re, y.re), mul<N>(x.im, y.im)), im = sub<N>(mul<N>(x.im, y.re), mul<N>(x.re, y.im));
+            const Divisor<N> v = cd_divisor<N>(d.w);
+            const bool a = cd_div<N>(re, d, v, z.re), b = cd_div<N>(im, d, v, z.im);
+            if (!(a && b)) z = cdiv<N>(load_cpx<N>(g.a, g.pa, reload_index(i)), load_cpx<N>(g.b, g.pb, reload_index(jb)));
+        }
         else {
             const Cpx<N> w = load_cpx<N>(g.c, g.pc, operand_index(i, g.c_stride, g.c_period));
             if constexpr (OP == OP_CFMA) z = lf::cfma<N>(x, y, w);
@@ -79,7 +95,10 @@ template <int N, int OP> __global__ void __launch_bounds__(256) elementwise_kern
             if constexpr (OP == OP_ADD) z = add<N>(x, y);
             else if constexpr (OP == OP_SUB) z = sub<N>(x, y);
             else if constexpr (OP == OP_MUL) z = mul<N>(x, y);
-            else if constexpr (OP == OP_DIV) z = div<N>(x, y);
+            else if constexpr (OP == OP_DIV) {
+                if (!cd_div<N>(x, y, cd_divisor<N>(y.w), z))
+                    z = div<N>(load_num<N>(g.a, g.pa, reload_index(i)), load_num<N>(g.b, g.pb, reload_index(jb)));
+            }
             else {
                 const u32 jc = operand_index(i, g.c_stride, g.c_period);
                 Num<N> w = load_num<N>(g.c, g.pc, jc);
