@@ -312,17 +312,41 @@ template <bool BY_LINE> __device__ __forceinline__ void analyze_line(const Analy
     const auto mn = [](int x, int y) { return min(x, y); };
     u32 status = 0;
     int top = INT_MIN, bottom = INT_MAX;
-#pragma unroll 4
-    for (u32 k = first; k < K; k += step) {
-        const u64 i = base + (u64)k * S.v.ks;
-        const int e = (int)ep[i], sg = (int)sp[i];
-        const u32 st = tp[i];
-        status |= st;
-        if (!st && sg) {
-            top = max(top, e);
-            bottom = min(bottom, e);
+    // a thread's exponents stay in registers for the band passes (INT_MIN: zero, status or past K) where they fit; all
+    // their loads are then in flight together
+    constexpr u32 KEPT = 32;
+    const bool kept = a.K <= KEPT * step;
+    int own[KEPT];
+    if (kept) {
+#pragma unroll
+        for (u32 n = 0; n < KEPT; ++n) {
+            const u32 k = first + n * step;
+            own[n] = INT_MIN;
+            if (k < K) {
+                const u64 i = base + (u64)k * S.v.ks;
+                const int e = (int)ep[i], sg = (int)sp[i];
+                const u32 st = tp[i];
+                status |= st;
+                own[n] = !st && sg ? e : INT_MIN;
+            }
         }
-    }
+#pragma unroll
+        for (u32 n = 0; n < KEPT; ++n) {
+            top = max(top, own[n]);
+            bottom = own[n] == INT_MIN ? bottom : min(bottom, own[n]);
+        }
+    } else
+#pragma unroll 4
+        for (u32 k = first; k < K; k += step) {
+            const u64 i = base + (u64)k * S.v.ks;
+            const int e = (int)ep[i], sg = (int)sp[i];
+            const u32 st = tp[i];
+            status |= st;
+            if (!st && sg) {
+                top = max(top, e);
+                bottom = min(bottom, e);
+            }
+        }
     status = (u32)line_reduce<BY_LINE>((int)status, red, [](int x, int y) { return x | y; });
     top = line_reduce<BY_LINE>(top, red, mx);
     bottom = line_reduce<BY_LINE>(bottom, red, mn);
@@ -347,7 +371,15 @@ template <bool BY_LINE> __device__ __forceinline__ void analyze_line(const Analy
     }
     while (BY_LINE ? __syncthreads_or(more) != 0 : more) {
         int lo = hi, next = INT_MIN;
-        if (more)
+        if (more && kept) {
+#pragma unroll
+            for (u32 n = 0; n < KEPT; ++n) {
+                const int e = own[n];
+                if (e == INT_MIN || e > hi) continue;
+                if ((long)e >= (long)hi - a.G) lo = min(lo, e);
+                else next = max(next, e);
+            }
+        } else if (more)
 #pragma unroll 4
             for (u32 k = first; k < K; k += step) {
                 const u64 i = base + (u64)k * S.v.ks;
@@ -1021,10 +1053,10 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
     const std::size_t Kp = std::max<std::size_t>((std::max<std::size_t>(P.K, 1) + 63) / 64 * 64, 64);
     const std::size_t Mp = (Me + PT - 1) / PT * PT, Np = (Ne + PT - 1) / PT * PT; // product tiles
     PoolBuf dig_l1{3}, dig_l0{4}, dig_r1{5}, dig_r0{6}, dres{7}, dlist[3] = {{8}, {9}, {10}};
-    // events bounding the stages: start, digits done, products done, rebuild done, exact dots done
+    // events bounding the stages: start, digits done, products done, rebuild done, exact dots done (attached to the
+    // kernels' own dispatches instead, they cost the 98 us of a small product 13 us more)
     hipEvent_t* ev = nullptr;
     GEMM_HIP(stage_events(&ev), "hipEventCreate");
-    hipEvent_t e0 = ev[0], e1 = ev[4];
     const int WX = lf::rebuild_words(N, plan.wx_class);
     const DigitTable* dt = nullptr;
     CrtSet crt{};
@@ -1047,7 +1079,7 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
         }
     if (rep) rep->upload_seconds = since(t0);
     t0 = Clock::now();
-    GEMM_HIP(hipEventRecord(e0, P.stream), "hipEventRecord");
+    GEMM_HIP(hipEventRecord(ev[0], P.stream), "hipEventRecord");
     if (any_pair) {
         // the digits kernel writes every byte of the lines' rows; the padding rows past them only feed residues
         // that nothing reads
@@ -1203,11 +1235,13 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
             first = last;
         }
     }
-    GEMM_HIP(hipEventRecord(e1, P.stream), "hipEventRecord");
+    if (fallback_outputs) GEMM_HIP(hipEventRecord(ev[4], P.stream), "hipEventRecord");
     GEMM_HIP(hipStreamSynchronize(P.stream), "device execution (linalg)");
     float ms = 0, stage_ms[4] = {};
-    GEMM_HIP(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
-    for (int q = 0; q < 4; ++q) GEMM_HIP(hipEventElapsedTime(&stage_ms[q], ev[q], ev[q + 1]), "hipEventElapsedTime");
+    for (int q = 0; q < (fallback_outputs ? 4 : 3); ++q) {
+        GEMM_HIP(hipEventElapsedTime(&stage_ms[q], ev[q], ev[q + 1]), "hipEventElapsedTime");
+        ms += stage_ms[q];
+    }
     if (device_ms) *device_ms = ms;
     if (rep) {
         rep->gpu_seconds = ms * 1e-3;

@@ -37,14 +37,20 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 // LDS and writes every band row of its lines as 16-byte chunks, zero where the entry is not a member of that
 // band (or is zero, carries a status, or lies past K).  Rows past the last line are left as they are: no
 // kernel reads the residues they give.
-// What bounds it is the reduction of each residue (about 20 instructions): the two reductions by 16-bit chunks
-// and a table of shift powers that this replaces took 32 multiply-adds of 16-bit chunks and as much again.
+// What bounds it is the reduction of each residue (about 17 instructions) and the LDS that limits the workgroups in
+// flight: each wavefront keeps its entries' bytes in registers over the moduli, so that the digit bytes' stage takes
+// the place of the mantissas.  On the operands of a 512-bit 512^3 product joined to one band (123 moduli) two
+// launches of 16-bit chunks by powers, reduced twice, took 260 us, this form 107 us with both in LDS and 102 us so.
 constexpr u32 DIG_QB = 32;                      // moduli per LDS batch
 constexpr u32 DIG_STAGE_ROW = 2 * 256 + 16;     // bytes of a modulus's stage row: both digits of 256 entries
 // a shifted mantissa's LDS row: an odd number of 16-byte chunks, so that the 16 lanes of a fragment read hit
 // distinct banks
 __host__ __device__ constexpr u32 digits_row_bytes(u32 bytes) { return bytes + 16; }
-__host__ __device__ constexpr u64 digits_lds_bytes(u32 bytes) { return (u64)256 * digits_row_bytes(bytes) + DIG_QB * DIG_STAGE_ROW + 256 + 64; }
+__host__ __device__ constexpr u32 digits_area(u32 bytes) // the mantissas, then the stage
+{
+    return 256 * digits_row_bytes(bytes) > DIG_QB * DIG_STAGE_ROW ? 256 * digits_row_bytes(bytes) : DIG_QB * DIG_STAGE_ROW;
+}
+__host__ __device__ constexpr u64 digits_lds_bytes(u32 bytes) { return digits_area(bytes) + 256 + 64; }
 
 __device__ __forceinline__ u32 byte_eq_mask(u32 x, u32 b4)
 {
@@ -54,12 +60,12 @@ __device__ __forceinline__ u32 byte_eq_mask(u32 x, u32 b4)
     return (z >> 7) * 0xffu;
 }
 
-template <int N> __global__ void __launch_bounds__(256) digits_kernel(DigitsArgs g)
+template <int N> __global__ void __launch_bounds__(256, 2) digits_kernel(DigitsArgs g)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const u32 rowb = digits_row_bytes(g.bytes);
-    unsigned char* stage = lds + 256u * rowb;
-    unsigned char* bandof = stage + DIG_QB * DIG_STAGE_ROW;
+    unsigned char* stage = lds;
+    unsigned char* bandof = lds + digits_area(g.bytes);
     u32* signs = reinterpret_cast<u32*>(bandof + 256); // bit e % 32 of word e / 32: entry e is negative
     const bool second = blockIdx.x >= g.side[0].blocks;
     const DigitsSide S = second ? g.side[1] : g.side[0];
@@ -115,19 +121,28 @@ template <int N> __global__ void __launch_bounds__(256) digits_kernel(DigitsArgs
     // waves 0-3: entries 64 wave + 32 h + (lane % 32); bytes 32 step + 16 (lane / 32) of each
     const u32 steps = g.bytes / 32u, r = lane & 31u, kh = lane >> 5;
     const u32 sg[2] = {signs[2u * wave], signs[2u * wave + 1u]};
+    constexpr u32 STEPS = (4 * N + 67 + 31) / 32; // a CRT class holds bands of at most 534 bits
+    v4i a[STEPS][2];
+#pragma unroll
+    for (u32 st = 0; st < STEPS; ++st)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            if (st < steps) a[st][h] = *(const v4i*)(lds + (64u * wave + 32u * h + r) * rowb + 32u * st + 16u * kh);
+    __syncthreads(); // the mantissas' LDS becomes the stage
     for (u32 qb = 0; qb < g.L; qb += DIG_QB) {
         const u32 q = qb + r < g.L ? qb + r : g.L - 1; // lanes past the last modulus repeat it
         const int8_t* tab = g.table + (u64)q * 2 * DIGIT_TABLE_BYTES + 16u * kh;
         v16i s1[2] = {}, s0[2] = {};
-        for (u32 st = 0; st < steps; ++st) {
-            const v4i b1 = *(const v4i*)(tab + 32u * st), b0 = *(const v4i*)(tab + DIGIT_TABLE_BYTES + 32u * st);
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const v4i a = *(const v4i*)(lds + (64u * wave + 32u * h + r) * rowb + 32u * st + 16u * kh);
-                s1[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b1, s1[h], 0, 0, 0);
-                s0[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b0, s0[h], 0, 0, 0);
+        for (u32 st = 0; st < STEPS; ++st)
+            if (st < steps) {
+                const v4i b1 = *(const v4i*)(tab + 32u * st), b0 = *(const v4i*)(tab + DIGIT_TABLE_BYTES + 32u * st);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    s1[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[st][h], b1, s1[h], 0, 0, 0);
+                    s0[h] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[st][h], b0, s0[h], 0, 0, 0);
+                }
             }
-        }
         const int m = (int)g.moduli[q], half = m >> 1, off = g.offset[q];
         const float inv = g.inverse[q];
 #pragma unroll
@@ -135,27 +150,29 @@ template <int N> __global__ void __launch_bounds__(256) digits_kernel(DigitsArgs
 #pragma unroll
             for (int i4 = 0; i4 < 4; ++i4) {
                 // accumulator element 4 i4 + i: entry row 8 i4 + 4 (lane / 32) + i, modulus column lane % 32
-                u32 w1 = 0, w0 = 0;
                 const u32 e = 8u * i4 + 4u * kh;
+                u32 v[4], v1[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int T = s1[h][4 * i4 + i] * 256 + s0[h][4 * i4 + i] + off;
-                    int v = T - residue_mul24((int)__builtin_rintf((float)T * inv), m);
-                    v -= v > half ? m : 0;
-                    v += v < -half ? m : 0;
+                    const int T = (int)((u32)s1[h][4 * i4 + i] << 8) + s0[h][4 * i4 + i] + off;
+                    // T - q m + half lies in (-m, 2m): one unsigned minimum takes a negative value up by m, one a value
+                    // from m on down by m
+                    u32 u = (u32)(T + half - residue_mul24((int)__builtin_rintf((float)T * inv), m));
+                    u = min(u, u + (u32)m);
+                    u = min(u, u - (u32)m);
                     const int neg = -(int)((sg[h] >> (e + i)) & 1u);
-                    v = (v ^ neg) - neg;
-                    const int d0 = (v << 24) >> 24, d1 = (v - d0) >> 8;
-                    w0 |= ((u32)d0 & 0xffu) << (8 * i);
-                    w1 |= ((u32)d1 & 0xffu) << (8 * i);
+                    v[i] = (u32)(((int)u - half) ^ neg) - (u32)neg;
+                    v1[i] = v[i] + 128u; // its second byte is the high digit, v's first the low one
                 }
+                const u32 w0 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(v[3], v[2], 0x0c0c0400u), __builtin_amdgcn_perm(v[1], v[0], 0x0c0c0400u), 0x05040100u);
+                const u32 w1 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(v1[3], v1[2], 0x0c0c0501u), __builtin_amdgcn_perm(v1[1], v1[0], 0x0c0c0501u), 0x05040100u);
                 unsigned char* at = stage + r * DIG_STAGE_ROW + 64u * wave + 32u * h + e;
                 *reinterpret_cast<u32*>(at) = w1;
                 *reinterpret_cast<u32*>(at + 256) = w0;
             }
         __syncthreads();
-        // chunk j: 16 entries (c16) of digit plane pl of modulus qb + qi, written to every band row of their line
         const u32 nq = g.L - qb < DIG_QB ? g.L - qb : DIG_QB;
+        // chunk j: 16 entries (c16) of digit plane pl of modulus qb + qi, written to every band row of their line
         for (u32 j = t; j < nq * 32u; j += 256u) {
             const u32 c16 = j & 15u, pl = (j >> 4) & 1u, qi = j >> 5;
             const u32 line = line0 + 16u * c16 / tk, kk = k0 + 16u * c16 % tk;
@@ -180,6 +197,53 @@ template <int N> __global__ void __launch_bounds__(256) digits_kernel(DigitsArgs
 }
 
 // ---------------------------------------------------------------- CRT rebuild
+// The symmetric representative of X' = sum y_q (M/m_q) 2^t < L M' (Mb: M', then floor(M'/2)): X becomes its magnitude;
+// returns its sign (+1/-1).
+template <int WX> __device__ __forceinline__ int crt_reduce(const u32* Mb, u32 (&X)[WX])
+{
+    // X' < L M' with M' normalised to bit 32(WX-1)-1: estimate q = floor(X'/M') from the top words
+    const u64 xt = ((u64)X[WX - 1] << 32) | X[WX - 2];
+    u64 qe = xt / ((u64)Mb[WX - 2] + 1u);
+    // X' -= qe * M'
+    u64 bw = 0;
+#pragma unroll
+    for (int w = 0; w < WX; ++w) {
+        const u64 p = qe * Mb[w] + bw;
+        const u32 lo = (u32)p, old = X[w];
+        X[w] = old - lo;
+        bw = (p >> 32) + (old < lo ? 1u : 0u);
+    }
+    for (int rep = 0; rep < 3; ++rep) {
+        int cmp = 0;
+#pragma unroll
+        for (int w = WX - 1; w >= 0; --w)
+            if (cmp == 0 && X[w] != Mb[w]) cmp = X[w] > Mb[w] ? 1 : -1;
+        if (cmp < 0) break;
+        u32 b2 = 0;
+#pragma unroll
+        for (int w = 0; w < WX; ++w) {
+            const u64 v = (u64)X[w] - Mb[w] - b2;
+            X[w] = (u32)v;
+            b2 = (u32)(v >> 63);
+        }
+    }
+    // symmetric range: X' > floor(M'/2) means the negative value X' - M'
+    const u32* H = Mb + WX;
+    int cmp = 0;
+#pragma unroll
+    for (int w = WX - 1; w >= 0; --w)
+        if (cmp == 0 && X[w] != H[w]) cmp = X[w] > H[w] ? 1 : -1;
+    if (cmp <= 0) return 1;
+    u32 b3 = 0;
+#pragma unroll
+    for (int w = 0; w < WX; ++w) {
+        const u64 v = (u64)Mb[w] - X[w] - b3;
+        X[w] = (u32)v;
+        b3 = (u32)(v >> 63);
+    }
+    return -1;
+}
+
 // X' = |sum| * 2^t from the L values y_q = r_q (M/m_q)^-1 mod m_q at (row, col) (the product kernel writes
 // the residues already multiplied by that factor); returns the sign (+1/-1) of the symmetric value.  The
 // CRT words come from LDS (staged by the kernel, rows padded to whole 16-byte groups, read 16 bytes at a
@@ -240,48 +304,7 @@ __device__ __forceinline__ int crt_rebuild(const Args& g, const u32* tab, u32 ro
         X[w] = (u32)v;
         carry = v >> 32;
     }
-    // X' < L M' with M' normalised to bit 32(WX-1)-1: estimate q = floor(X'/M') from the top words
-    const u32* Mb = g.bound;
-    const u64 xt = ((u64)X[WX - 1] << 32) | X[WX - 2];
-    u64 qe = xt / ((u64)Mb[WX - 2] + 1u);
-    // X' -= qe * M'
-    u64 bw = 0;
-#pragma unroll
-    for (int w = 0; w < WX; ++w) {
-        const u64 p = qe * Mb[w] + bw;
-        const u32 lo = (u32)p, old = X[w];
-        X[w] = old - lo;
-        bw = (p >> 32) + (old < lo ? 1u : 0u);
-    }
-    for (int rep = 0; rep < 3; ++rep) {
-        int cmp = 0;
-#pragma unroll
-        for (int w = WX - 1; w >= 0; --w)
-            if (cmp == 0 && X[w] != Mb[w]) cmp = X[w] > Mb[w] ? 1 : -1;
-        if (cmp < 0) break;
-        u32 b2 = 0;
-#pragma unroll
-        for (int w = 0; w < WX; ++w) {
-            const u64 v = (u64)X[w] - Mb[w] - b2;
-            X[w] = (u32)v;
-            b2 = (u32)(v >> 63);
-        }
-    }
-    // symmetric range: X' > floor(M'/2) means the negative value X' - M'
-    const u32* H = g.bound + WX;
-    int cmp = 0;
-#pragma unroll
-    for (int w = WX - 1; w >= 0; --w)
-        if (cmp == 0 && X[w] != H[w]) cmp = X[w] > H[w] ? 1 : -1;
-    if (cmp <= 0) return 1;
-    u32 b3 = 0;
-#pragma unroll
-    for (int w = 0; w < WX; ++w) {
-        const u64 v = (u64)Mb[w] - X[w] - b3;
-        X[w] = (u32)v;
-        b3 = (u32)(v >> 63);
-    }
-    return -1;
+    return crt_reduce<WX>(g.bound, X);
 }
 
 template <int N> __device__ __forceinline__ void store_out(u32* base, u64 pitch, u64 stride, u32 i, u32 j, bool mirror, const Num<N>& r)
@@ -365,37 +388,115 @@ template <int WX> __device__ __forceinline__ int read_stage(const RebuildArgs& g
     return (int)src[WX * wstride];
 }
 
+// The value of lane `SRC` of this lane's quad, and of the lane one or two places away in it.
+template <int CTRL> __device__ __forceinline__ u32 quad_read(u32 v) { return (u32)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xF, 0xF, false); }
+
 // One pass from the residues to the rounded output where every line is one band: nothing is staged between the
-// CRT and the rounding.  One lane an output, outputs of one row a workgroup: 256 where the CRT words are staged
-// in LDS for the workgroup, else 64, so that a small product spreads over the GPU.
-constexpr u32 round_block(int wx) { return wx >= CRT_LDS_MIN_WX ? 256u : 64u; }
-template <int N, int WX> __global__ void __launch_bounds__(round_block(WX)) crt_round_kernel(RoundArgs g)
+// CRT and the rounding.  Four consecutive outputs of a row form a quad of lanes, and each lane forms one quarter
+// of the CRT words of all four, then the quad exchanges quarters: a lane's multiply-adds are as many as for one
+// output of its own, and it reads a quarter of the table from LDS.  What bounds it is those multiply-adds; with the
+// whole table read by every lane (17 16-byte reads a modulus at 67 words against 5) it was LDS bound: 158 us on
+// the 512-bit 512^3 product joined to one band, 145 us so; 34 and 27 us on the 256-bit SYRK of 2048 x 512.
+constexpr u32 ROUND_BLOCK = 256;
+constexpr int quarter_words(int wx) { return (wx + 3) / 4; }
+constexpr int quarter_pitch(int wx) { return (quarter_words(wx) + 3) & ~3; }
+constexpr u64 round_table_bytes(u32 L, int wx) { return (u64)L * 4 * quarter_pitch(wx) * 4; }
+template <int N, int WX> __global__ void __launch_bounds__(ROUND_BLOCK) crt_round_kernel(RoundArgs g)
 {
-    constexpr int WXP = (WX + 3) & ~3;
-    constexpr u32 ROUND_BLOCK = round_block(WX);
+    constexpr int QW = quarter_words(WX), QP = quarter_pitch(WX);
     extern __shared__ __attribute__((aligned(16))) u32 tab[];
-    const u32 nblocks = (g.n + ROUND_BLOCK - 1) / ROUND_BLOCK;
-    const u32 i = blockIdx.x / nblocks, j0 = (blockIdx.x % nblocks) * ROUND_BLOCK, j = j0 + threadIdx.x;
+    const u32 block = blockDim.x, nblocks = (g.n + block - 1) / block;
+    const u32 i = blockIdx.x / nblocks, j0 = (blockIdx.x % nblocks) * block, j = j0 + threadIdx.x, quarter = threadIdx.x & 3u;
     if (g.syrk && j0 > i) return; // the whole workgroup lies above the diagonal
-    if constexpr (WX >= CRT_LDS_MIN_WX) {
-        for (u32 k = threadIdx.x; k < g.L * WXP; k += ROUND_BLOCK) {
-            const u32 q = k / WXP, w = k % WXP;
-            tab[k] = w < (u32)WX ? g.crt[q * WX + w] : 0u;
-        }
-        __syncthreads();
+    for (u32 k = threadIdx.x; k < g.L * 4 * QP; k += block) {
+        const u32 q = k / (4 * QP), p = (k / QP) % 4u, w = p * QW + k % QP;
+        tab[k] = k % QP < (u32)QW && w < (u32)WX ? g.crt[q * WX + w] : 0u;
     }
-    if (j >= g.n || (g.syrk && j > i)) return;
-    const bool mirror = g.syrk && !g.lower_only;
+    __syncthreads();
+    const bool inside = j < g.n && !(g.syrk && j > i);
     const GemmLine* Li = g.left + i;
-    const GemmLine* Lj = g.right + j;
+    const GemmLine* Lj = g.right + (inside ? j : 0u);
+    const bool live = inside && Li->cls == 0 && Lj->cls == 0;
+    u64 sum[4][QW];
+#pragma unroll
+    for (int o = 0; o < 4; ++o)
+#pragma unroll
+        for (int w = 0; w < QW; ++w) sum[o][w] = 0;
+    // a SYRK's members are in line order, so the row's is the larger: the product's lower triangle
+    const u64 plane = (u64)g.Mp * g.Np, at = live ? (u64)(u32)Li->member[0] * g.Np + (u32)Lj->member[0] : 0;
+    // residues in batches of 8 moduli, the next batch's loads in flight while this one accumulates
+    constexpr u32 RB = 8;
+    u32 rr[RB], rn[RB];
+#pragma unroll
+    for (u32 u = 0; u < RB; ++u) rr[u] = live && u < g.L ? (u32)g.res[(u64)u * plane + at] : 0u;
+    for (u32 q0 = 0; q0 < g.L; q0 += RB) {
+#pragma unroll
+        for (u32 u = 0; u < RB; ++u) rn[u] = live && q0 + RB + u < g.L ? (u32)g.res[(u64)(q0 + RB + u) * plane + at] : 0u;
+#pragma unroll
+        for (u32 u = 0; u < RB; ++u) {
+            const u32 q = q0 + u;
+            if (q >= g.L) break;
+            u32 y[4] = {quad_read<0x00>(rr[u]), quad_read<0x55>(rr[u]), quad_read<0xAA>(rr[u]), quad_read<0xFF>(rr[u])};
+            const uint4* C4 = reinterpret_cast<const uint4*>(tab + (q * 4 + quarter) * QP);
+#pragma unroll
+            for (int w4 = 0; w4 < QP / 4; ++w4) {
+                const uint4 c = C4[w4];
+                const u32 cw[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (4 * w4 + k < QW)
+#pragma unroll
+                        for (int o = 0; o < 4; ++o) sum[o][4 * w4 + k] += (u64)y[o] * cw[k];
+            }
+        }
+#pragma unroll
+        for (u32 u = 0; u < RB; ++u) rr[u] = rn[u];
+    }
+    // each quarter's words and the carry out of it; then lane k of the quad takes the quarters of output k
+    u32 x[4][QW + 1];
+#pragma unroll
+    for (int o = 0; o < 4; ++o) {
+        u64 carry = 0;
+#pragma unroll
+        for (int w = 0; w < QW; ++w) {
+            const u64 v = sum[o][w] + carry;
+            x[o][w] = (u32)v;
+            carry = v >> 32;
+        }
+        x[o][QW] = (u32)carry; // below L 2^16
+    }
+    const bool odd = quarter & 1u, high = quarter & 2u;
+#pragma unroll
+    for (int w = 0; w <= QW; ++w) {
+#pragma unroll
+        for (int o = 0; o < 4; o += 2) { // neighbours exchange (o, o + 1)
+            const u32 r = quad_read<0xB1>(odd ? x[o][w] : x[o + 1][w]);
+            x[o][w] = odd ? r : x[o][w];
+            x[o + 1][w] = odd ? x[o + 1][w] : r;
+        }
+#pragma unroll
+        for (int o = 0; o < 2; ++o) { // pairs exchange (o, o + 2)
+            const u32 r = quad_read<0x4E>(high ? x[o][w] : x[o + 2][w]);
+            x[o][w] = high ? r : x[o][w];
+            x[o + 2][w] = high ? x[o + 2][w] : r;
+        }
+    }
+    if (!inside) return;
+    const bool mirror = g.syrk && !g.lower_only;
     if (Li->cls == 1 || Lj->cls == 1) { // zero or status line
         store_out<N>(g.out, g.out_pitch, g.out_stride, i, j, mirror, zero<N>(Li->status | Lj->status));
         return;
     }
-    if (Li->cls != 0 || Lj->cls != 0) return; // exact dot kernels
+    if (!live) return; // exact dot kernels
     u32 X[WX];
-    // a SYRK's members are in line order, so the row's is the larger: the product's lower triangle
-    const int sg = crt_rebuild<WX>(g, tab, (u32)Li->member[0], (u32)Lj->member[0], X);
+    u32 from = 0, cy = 0;
+#pragma unroll
+    for (int w = 0; w < WX; ++w) {
+        const int p = w / QW, k = w % QW;
+        if (k == 0) from = p ? x[p - 1][QW] : 0u;
+        X[w] = add_carry(x[p][k], k == 0 ? from : 0u, cy);
+    }
+    const int sg = crt_reduce<WX>(g.bound, X);
     const i64 scale = (i64)Li->low + Lj->low - 2 * (32 * N - 1) - g.t;
     store_out<N>(g.out, g.out_pitch, g.out_stride, i, j, mirror, pack<N, WX>(X, scale, sg, ST_OK));
 }

@@ -12,7 +12,7 @@ template <int N> hipError_t launch_digits(const DigitsArgs& g, hipStream_t s)
 {
     const u32 blocks = g.side[0].blocks + g.side[1].blocks;
     if (!g.K || !blocks || !g.L) return hipSuccess;
-    if (g.Kp % 32u || g.bytes % 32u || g.bytes > DIGIT_TABLE_BYTES) return hipErrorInvalidValue;
+    if (g.Kp % 32u || g.bytes % 32u || g.bytes > DIGIT_TABLE_BYTES || g.bytes > (4 * N + 67 + 31) / 32 * 32) return hipErrorInvalidValue;
     const u64 lds = digits_lds_bytes(g.bytes);
     if (lds > (u64(64) << 10))
         if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&digits_kernel<N>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
@@ -23,11 +23,12 @@ template <int N> hipError_t launch_digits(const DigitsArgs& g, hipStream_t s)
 
 template <int N, int WX> hipError_t launch_round_wx(const RoundArgs& g, hipStream_t s)
 {
-    const u64 lds = crt_table_bytes(g.L, WX);
+    const u64 lds = round_table_bytes(g.L, WX);
     if (lds > (u64(64) << 10))
         if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&crt_round_kernel<N, WX>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
             return e;
-    constexpr u32 RB = round_block(WX);
+    // small products in workgroups of one wavefront, to spread over the GPU
+    const u32 RB = (u64)g.m * g.n >= 65536 ? ROUND_BLOCK : 64u;
     hipLaunchKernelGGL((crt_round_kernel<N, WX>), dim3(((g.n + RB - 1) / RB) * g.m), dim3(RB), lds, s, g);
     return hipGetLastError();
 }
