@@ -301,7 +301,7 @@ typedef struct lf_chain_bucket {
     uint64_t count;
 } lf_chain_bucket;
 /* One launch per bucket, in order, on `stream`.  block[i]: lanes per workgroup of bucket i (64, 128 or
- * 256; NULL or 0 = the autotuned size of that width, else 256). */
+ * 256; NULL or 0 = the autotuned size of that width, else 64). */
 int lf_mixed_chains(const lf_chain_bucket* buckets, int nbuckets, const unsigned* block, void* stream);
 /* One hipGraph with one persistent kernel node per group of eight widths (2-8, 9-16, 17-24, 25-32 limbs) and
  * no edges between them; each node runs all of its group's buckets (launch with lf_graph_launch, free with
