@@ -171,12 +171,12 @@ int update(int bits, const lf_linalg_options& o, bool syrk, const lf::MatView& l
 
 double since(Clock::time_point t) { return std::chrono::duration<double>(Clock::now() - t).count(); }
 
-// wavefronts (and scratch slots) of a look-ahead update: four for each of 256 tiles
-constexpr uint64_t LOOKAHEAD_WAVES = 1024;
+// wavefronts (and scratch slots) of a look-ahead update: eight for each of 256 tiles
+constexpr uint64_t LOOKAHEAD_WAVES = 2048;
 // wavefronts (and scratch slots) of a direct off-block solve update
-constexpr uint64_t SOLVE_UPDATE_WAVES = 2048;
+constexpr uint64_t SOLVE_UPDATE_WAVES = 4096;
 // Off-block solve updates of up to this many multiply-add terms (rows x right-hand sides x block) also run
-// as direct exact dots: on 2048 wavefronts 2^20 terms of 256 bits take about 30 us, less than one update
+// as direct exact dots: on 4096 wavefronts 2^20 terms of 256 bits take about 30 us, less than one update
 // GEMM's planning round trip (band analysis, line-table download, constants, about 0.4 ms of host time per
 // update at n = 512 with 64 right-hand sides).  Both forms round the same exact value once.
 constexpr double SOLVE_DIRECT_TERMS = 4194304.0;

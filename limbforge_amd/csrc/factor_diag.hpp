@@ -13,7 +13,7 @@ template <int N> constexpr int wd_frac() { return wd_recip<N>(); }
 // the integer digit in lane 2F; their digits from lane F up serve as the next a with A0 = F, with no shift.
 template <int F, int FROM, int A0> __device__ __forceinline__ i64 wd_columns(u32 a, u32 b, u32 lane)
 {
-    u64 S = 0;
+    i64 S = 0;
     u32 bs = b;
     if constexpr (FROM > 0) {
         bs = (u32)__shfl((int)b, (int)((lane - (u32)FROM) & 63u));
@@ -21,10 +21,19 @@ template <int F, int FROM, int A0> __device__ __forceinline__ i64 wd_columns(u32
     }
 #pragma unroll
     for (int i = FROM; i <= F; ++i) {
-        S += (u64)wd_read(a, A0 + i) * bs;
+        S += (i64)(int)wd_read(a, A0 + i) * (int)bs;
         bs = wave_from_previous_lane(bs);
     }
-    return (i64)S;
+    return S;
+}
+// Columns split into their three balanced digits and added up, no carries after that: signed digits below 2^26.1 in
+// magnitude, which serve as factors where a result's exact digits are not needed.  Balanced, a small column of either
+// sign stays in its lane, so the digits of a raised number end at lane 2F.
+__device__ __forceinline__ u32 wd_loose(i64 S)
+{
+    const i64 T = S + ((i64)1 << (WD_BITS - 1)) + ((i64)1 << (2 * WD_BITS - 1));
+    const u32 lo = (u32)T & WD_MASK, mid = (u32)(T >> WD_BITS) & WD_MASK, hi = (u32)(int)(T >> (2 * WD_BITS));
+    return lo + wave_from_previous_lane(mid + wave_from_previous_lane(hi)) - (1u << WD_BITS);
 }
 // raised <-> aligned digits
 template <int F> __device__ __forceinline__ u32 wd_align(u32 d, u32 lane)
@@ -120,24 +129,43 @@ template <int N> __device__ __forceinline__ bool wd_sqrt(const WaveNum& s, u32 l
     u32 y = 0;
     if (sh >= 0 && sh < 64) y = (u32)(z >> sh) & WD_MASK;
     else if (sh < 0 && sh > -WD_BITS) y = (u32)(z << -sh) & WD_MASK;
-    y = wd_rsqrt<N, 164>(wd_rsqrt_first<F>(y, uh, lane), uh, lane);
-    // the root
-    const u32 p0 = wd_resolve(wd_columns<F, 0, 0>(y, uh, lane), lane);
-    const u32 r0 = wd_align<F>(p0, lane);
-    const u32 d2 = wd_resolve((i64)wd_raise<F>(uh, lane) - 2 * wd_columns<F, 0, 0>(r0, r0, lane), lane);
-    const u32 p = wd_resolve(wd_columns<F, 0, F>(d2, y, lane) + (lane >= (u32)F ? 2 * (i64)p0 : 0), lane);
-    constexpr int sigma = 2 * WD_BITS * F - 32 * N;
-    l.m = wd_shift_right(p, sigma, lane);
-    l.e = e;
-    l.s = 1;
-    const u32 g = wd_below(p, sigma);
-    if (g == 0x7fffffu || g == 0x800000u) return false;
-    if (g >> 23) l.m = wd_increment<N>(l.m, l.e, lane);
-    if (l.e != e) return false; // rounded up to the next power of two
-    // the reciprocal
-    const u32 r = wd_shift_left(l.m, WD_BITS * F - (32 * N - 1), lane);
-    const u32 c = wd_resolve(((int)lane == 2 * F ? (i64)4 : 0) - wd_columns<F, 0, 0>(y, r, lane), lane);
-    R = wd_shift_right(wd_resolve(wd_columns<F, 0, F>(c, y, lane), lane), 2 * WD_BITS * F - 32 * N - 63, lane);
+    const u32 uhr = wd_raise<F>(uh, lane);
+    u32 p, g, r, c;
+    auto root = [&](int sigma) -> bool {
+        l.m = wd_shift_right(p, sigma, lane);
+        l.e = e;
+        l.s = 1;
+        g = wd_below(p, sigma);
+        if (g == 0x7fffffu || g == 0x800000u) return false;
+        if (g >> 23) l.m = wd_increment<N>(l.m, l.e, lane);
+        if (l.e != e) return false; // rounded up to the next power of two
+        r = wd_shift_left(l.m, WD_BITS * F - (32 * N - 1), lane);
+        return true;
+    };
+    if constexpr (2 * 164 - 4 >= 32 * N + 40) {
+        // the first step's 164 bits are half enough: on loose digits, with Y = 8 y (k = 1/2 - uh y^2, Y = 8 y +
+        // y k (8 + 12 k)), q0 = uh Y = 2 sqrt(M), 128 sqrt(M) = 64 q0 + (32 uh - q0^2) Y, and Y (32 - l Y) / 256 = 1 / l
+        constexpr int A = F > 3 ? F - 3 : 0, B = F > 6 ? F - 6 : 0, C = F > 8 ? F - 8 : 0;
+        const u32 y2 = wd_loose(wd_columns<F, A, 0>(y, y, lane));
+        const u32 k = wd_loose(((int)lane == 2 * F - 1 ? (i64)1 << (WD_BITS - 1) : 0) - wd_columns<F, B, F>(y2, uh, lane));
+        const u32 k12 = 12u * wd_align<F>(k, lane) + ((int)lane == F ? 8u : 0u);
+        const u32 q = wd_loose(wd_columns<F, C, F>(k, k12, lane));
+        const u32 Y = wd_align<F>(wd_loose(wd_columns<F, C, F>(q, y, lane) + 8 * (i64)wd_raise<F>(y, lane)), lane);
+        const u32 q0 = wd_loose(wd_columns<F, 0, 0>(Y, uh, lane)), qa = wd_align<F>(q0, lane);
+        const u32 d = wd_loose(32 * (i64)uhr - wd_columns<F, 0, 0>(qa, qa, lane));
+        p = wd_resolve(wd_columns<F, 0, F>(d, Y, lane) + (lane >= (u32)F ? 64 * (i64)(int)q0 : 0), lane);
+        if (!root(2 * WD_BITS * F - 32 * N + 8)) return false;
+        c = wd_loose(((int)lane == 2 * F ? (i64)32 : 0) - wd_columns<F, 0, 0>(Y, r, lane));
+        R = wd_shift_right(wd_resolve(wd_columns<F, 0, F>(c, Y, lane), lane), 2 * WD_BITS * F - 32 * N - 57, lane);
+    } else {
+        y = wd_rsqrt<N, 164>(wd_rsqrt_first<F>(y, uh, lane), uh, lane);
+        const u32 p0 = wd_resolve(wd_columns<F, 0, 0>(y, uh, lane), lane), r0 = wd_align<F>(p0, lane);
+        const u32 d2 = wd_resolve((i64)uhr - 2 * wd_columns<F, 0, 0>(r0, r0, lane), lane);
+        p = wd_resolve(wd_columns<F, 0, F>(d2, y, lane) + (lane >= (u32)F ? 2 * (i64)p0 : 0), lane);
+        if (!root(2 * WD_BITS * F - 32 * N)) return false;
+        c = wd_resolve(((int)lane == 2 * F ? (i64)4 : 0) - wd_columns<F, 0, 0>(y, r, lane), lane);
+        R = wd_shift_right(wd_resolve(wd_columns<F, 0, F>(c, y, lane), lane), 2 * WD_BITS * F - 32 * N - 63, lane);
+    }
     const u32 low = (u32)((((u64)wd_read(R, 2) << (2 * WD_BITS)) | ((u64)wd_read(R, 1) << WD_BITS)) >> 32);
     return low != 0u && low != 0xffffffffu;
 }
@@ -162,7 +190,7 @@ template <int N> __device__ __forceinline__ u32 wd_recip_word(u32 R, u32 lane)
 // columns done, and chol_diag_kernel does the rest (a failed pivot, a status, spreads past the columns).
 // What bounds it is the chain of wave 0's wave-parallel products in A: nine for the root and the reciprocal at
 // 256 bits.  A 32-column block at 256 bits took 512 us with an exact dot a wavefront per entry and one-lane roots
-// and divisions, and 194 us with twelve products for the pivot and the rows rounded after it.
+// and divisions, 194 us with twelve products for the pivot and the rows rounded after it, and 131 us so.
 constexpr int DIAG_WAVES = 16;
 template <int N> struct DiagLds {
     i64 acc[3][WD_ROWS][WD_COLS + 1]; // column j: acc[j % 3], row i

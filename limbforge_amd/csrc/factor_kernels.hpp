@@ -48,7 +48,7 @@ struct DotScratch {
 };
 
 template <int N>
-__device__ __noinline__ Num<N> dot_sub_clusters(const Num<N>& c, const VecView& x, const VecView& y, u32 K, const DotScratch& sc)
+__device__ __forceinline__ Num<N> dot_sub_clusters_inline(const Num<N>& c, const VecView& x, const VecView& y, u32 K, const DotScratch& sc)
 {
     constexpr i64 NONE = -((i64)1 << 62);
     int logk = 0;
@@ -171,6 +171,13 @@ __device__ __noinline__ Num<N> dot_sub_clusters(const Num<N>& c, const VecView& 
         }
     }
     return pack<N, EW>(ext, scale1 - 32 * DW, sign1, ST_OK);
+}
+
+// As a call, which takes the registers it likes (248 at 256 bits); inlined, it lives within its kernel's bound.
+template <int N>
+__device__ __noinline__ Num<N> dot_sub_clusters(const Num<N>& c, const VecView& x, const VecView& y, u32 K, const DotScratch& sc)
+{
+    return dot_sub_clusters_inline<N>(c, x, y, K, sc);
 }
 
 // ---------------------------------------------------------------- one exact dot per wavefront
@@ -411,7 +418,7 @@ __device__ __forceinline__ Num<N> wave_round(const u64 (&S)[(factor_window(N) + 
     return round_words<N>(m, rw >> 31, sticky, scale + 32 * (i64)top + 31 - lz, sign, ST_OK);
 }
 
-template <int N>
+template <int N, bool INLINE = false>
 __device__ Num<N> wave_dot_sub(const Num<N>& c, const VecView& x, const VecView& y, u32 K, u32 lane, WaveLds<N>& L, const DotScratch& sc)
 {
     constexpr int W = factor_window(N);
@@ -483,7 +490,10 @@ __device__ Num<N> wave_dot_sub(const Num<N>& c, const VecView& x, const VecView&
     while ((1 << logc) < count) ++logc;
     if (top - lo + logc + 1 > 32 * W) {
         Num<N> r = zero<N>(ST_OK);
-        if (lane == 0) r = dot_sub_clusters<N>(c, x, y, K, sc);
+        if (lane == 0) {
+            if constexpr (INLINE) r = dot_sub_clusters_inline<N>(c, x, y, K, sc);
+            else r = dot_sub_clusters<N>(c, x, y, K, sc);
+        }
         return r;
     }
     // pass 2: rows of exact products, column sums

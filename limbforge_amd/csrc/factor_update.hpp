@@ -7,7 +7,7 @@ namespace lf {
 
 // Tiles of rows x columns entries, at most UPD_ENTRIES of them from at most UPD_LINES lines (rows and columns
 // together) of at most 32 terms.
-constexpr u32 UPD_ENTRIES = 64, UPD_LINES = 17, UPD_WAVES = 4;
+constexpr u32 UPD_ENTRIES = 64, UPD_LINES = 17, UPD_WAVES = 8;
 template <int N> struct UpdLds {
     i64 acc[UPD_ENTRIES][WD_COLS + 1];
     int digit[wd_grid<N>()][WD_ROWS * UPD_LINES]; // number (line, k) at k * UPD_LINES + line
@@ -20,15 +20,15 @@ template <int N> struct UpdLds {
 __host__ __device__ __forceinline__ u32 upd_cols(u32 cols) { return cols < 8u ? cols : 8u; }
 __host__ __device__ __forceinline__ u32 upd_rows(u32 tc) { return UPD_LINES - tc < UPD_ENTRIES / tc ? UPD_LINES - tc : UPD_ENTRIES / tc; }
 
-// One workgroup of four wavefronts a tile.  The lines' terms are turned into signed grid digits once; every
+// One workgroup of eight wavefronts a tile.  The lines' terms are turned into signed grid digits once; every
 // entry's accumulator is placed under its largest term; then each lane adds the products of one entry, two
-// wavefronts to a term (half of the row's digits each) and two terms at a time; and the accumulators are
-// rounded a digit a lane, 16 a wavefront.  A term costs its lane about 150 instructions and an entry's
+// wavefronts to a term (half of the row's digits each) and four terms at a time; and the accumulators are
+// rounded a digit a lane, eight a wavefront.  A term costs its lane about 150 instructions and an entry's
 // rounding 120 instructions of a wavefront, where one wavefront per entry (an exact dot of 32 terms) took
-// about 1,500: at 256 bits 62 us for 15,360 entries, 27 us here, and 52 against 30 us for the updates of a
-// solve with 64 right-hand sides.  Entries that this does not decide (a status, terms
+// about 1,500: at 256 bits 62 us for 15,360 entries, 23 us here (27 with four wavefronts a tile), and 52
+// against 30 us for the updates of a solve with 64 right-hand sides.  Entries that this does not decide (a status, terms
 // spread past the columns) take the exact dot.
-template <int N> __global__ void __launch_bounds__(64 * UPD_WAVES) update_wave_kernel(UpdateArgs g)
+template <int N> __global__ void __launch_bounds__(64 * UPD_WAVES, 4) update_wave_kernel(UpdateArgs g)
 {
     constexpr int GD = wd_grid<N>(), H = (GD + 1) / 2;
     constexpr std::size_t bytes = sizeof(UpdLds<N>) > UPD_WAVES * sizeof(WaveLds<N>) ? sizeof(UpdLds<N>) : UPD_WAVES * sizeof(WaveLds<N>);
@@ -94,7 +94,7 @@ template <int N> __global__ void __launch_bounds__(64 * UPD_WAVES) update_wave_k
                 fits = false;
                 continue;
             }
-            if (k % 2u != wave >> 1) continue;
+            if (k % (UPD_WAVES / 2) != wave >> 1) continue;
             int xd[H], yd[GD];
 #pragma unroll
             for (int q = 0; q < H; ++q) {
@@ -107,7 +107,8 @@ template <int N> __global__ void __launch_bounds__(64 * UPD_WAVES) update_wave_k
         }
         __syncthreads();
         const u64 good = L.odd ? 0 : __ballot(fits);
-        u64 rest = __ballot(live) & (0xffffull << (16u * wave)); // this wavefront's entries
+        constexpr u32 OWN = UPD_ENTRIES / UPD_WAVES;
+        u64 rest = __ballot(live) & ((((u64)1 << OWN) - 1u) << (OWN * wave)); // this wavefront's entries
         for (u64 todo = rest & good; todo; todo &= todo - 1) {
             const int e = (int)__builtin_ctzll(todo);
             WaveNum v;
@@ -121,7 +122,7 @@ template <int N> __global__ void __launch_bounds__(64 * UPD_WAVES) update_wave_k
             const u32 e = (u32)__builtin_ctzll(rest), i = r0 + e / tc, j = c0 + e % tc;
             const VecView x{g.x, g.xpitch, g.xbase + (i64)i * g.xr, g.xk}, y{g.y, g.ypitch, g.ybase + (i64)j * g.yc, g.yk};
             const u64 at = (u64)(g.obase + (i64)i * g.orow + (i64)j * g.ocol);
-            const Num<N> v = wave_dot_sub<N>(load_out<N>(g.out, g.opitch, at), x, y, g.K, lane, reinterpret_cast<WaveLds<N>*>(lds)[wave], sc);
+            const Num<N> v = wave_dot_sub<N, true>(load_out<N>(g.out, g.opitch, at), x, y, g.K, lane, reinterpret_cast<WaveLds<N>*>(lds)[wave], sc);
             if (lane == 0) store_out<N>(g.out, g.opitch, 0, 0, (u32)at, false, v);
         }
     }
