@@ -251,9 +251,11 @@ template <int N> struct TriLds {
 // first index of column k of the strict lower triangle: rows k + 1 .. WD_ROWS - 1
 __device__ __forceinline__ u32 wd_col_start(u32 k) { return k * (2 * WD_ROWS - 1 - k) / 2; }
 
+// Workgroup scope: the diagonal block's and the updates' accumulators take the terms of several wavefronts between
+// two barriers (the triangular blocks' belong to one; the instruction is the same).
 __device__ __forceinline__ void lds_add(i64* p, i64 v)
 {
-    __hip_atomic_fetch_add((u64*)p, (u64)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    __hip_atomic_fetch_add((u64*)p, (u64)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // Adds x * l to columns from `at` on, for one lane: H digits of x and GD digits of l.
