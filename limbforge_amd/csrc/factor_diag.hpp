@@ -226,15 +226,15 @@ template <int N> __global__ void __launch_bounds__(DIAG_WAVES * 64) chol_diag_wa
             const Num<N> a = load_out<N>(f.w, f.pitch, (u64)(f.k0 + i) * f.n + f.k0 + k);
             if (a.st || (i == k && !a.s)) L.slow[2] = 1;
             int d[GD], o;
-            lane_to_grid<N>(a, d, o);
+            lane_to_grid<N>(a, d, o); // (a record of sign 0 is zero whatever its limbs hold, and its accumulator starts from its digits)
             if (i == k) {
 #pragma unroll
-                for (int j = 0; j < GD; ++j) L.ddigit[j][i] = a.s < 0 ? -d[j] : d[j];
+                for (int j = 0; j < GD; ++j) L.ddigit[j][i] = a.s < 0 ? -d[j] : a.s ? d[j] : 0;
                 L.dorigin[i] = a.s ? o : WD_ZERO;
             } else {
                 const u32 at = wd_at(i, k);
 #pragma unroll
-                for (int j = 0; j < GD; ++j) L.digit[j][at] = a.s < 0 ? -d[j] : d[j];
+                for (int j = 0; j < GD; ++j) L.digit[j][at] = a.s < 0 ? -d[j] : a.s ? d[j] : 0;
                 L.origin[at] = a.s ? o : WD_ZERO;
             }
         }

@@ -86,3 +86,39 @@ def test_squares_of_short_factors(capi, oracle, bits):
     got, info = capi.cholesky(bits, A, n, block=32)
     assert info.pivot == piv == n
     assert (got == want).all()
+
+
+@pytest.mark.parametrize("bits", [64, 256, 640, 672])
+def test_sign_zero_is_zero_whatever_the_limbs(capi, oracle, bits):
+    """Records of sign 0 whose limbs and exponents are not zero, in the matrix, the factor and the right-hand sides:
+    each is a zero, as with zero limbs."""
+    rng = np.random.default_rng(11 * bits)
+    n, nrhs, block, w = 67, 3, 32, bits // 32
+    A = spd(oracle, rng, bits, n, "moderate")
+    i, j = np.tril_indices(n, -1)
+    pick = rng.random(i.size) < 0.3
+    i, j = i[pick], j[pick]
+    for x, y in ((i, j), (j, i)):
+        A[x * n + y] = lfcases.random_records(rng, bits, i.size, 6)
+        A[x * n + y, w + 1] = 0
+    d = np.arange(n) * (n + 1)
+    A[d, w] = lfcases.i32(lfcases.get_exp(A[d], bits) + 8)  # diagonally dominant: positive definite whatever went to zero
+    clean = A.copy()
+    clean[clean[:, w + 1] == 0] = lfcases.zero(bits)
+    want, piv, _, _ = oracle.cholesky(bits, clean, n, block)
+    assert piv == n
+    got, info = capi.cholesky(bits, A, n, block=block)
+    assert info.pivot == n
+    bad = np.nonzero((got != want).any(axis=1))[0]
+    assert bad.size == 0, f"{bad.size} entries differ, first ({bad[0] // n},{bad[0] % n})"
+    L, B = want.copy(), lfcases.random_records(rng, bits, n * nrhs, 8)
+    L[i * n + j] = A[i * n + j]
+    B[rng.random(n * nrhs) < 0.3, w + 1] = 0
+    cl, cb = L.copy(), B.copy()
+    cl[cl[:, w + 1] == 0] = lfcases.zero(bits)
+    cb[cb[:, w + 1] == 0] = lfcases.zero(bits)
+    for passes in (1, 2):
+        want = oracle.solve(bits, cl, n, cb, nrhs, block, passes)
+        got, _, _ = capi.solve(bits, passes, L, n, B, nrhs, block=block)
+        bad = np.nonzero((got != want).any(axis=1))[0]
+        assert bad.size == 0, f"passes={passes}: {bad.size} entries differ, first row {bad[0] // nrhs}"
