@@ -122,3 +122,25 @@ def test_sign_zero_is_zero_whatever_the_limbs(capi, oracle, bits):
         got, _, _ = capi.solve(bits, passes, L, n, B, nrhs, block=block)
         bad = np.nonzero((got != want).any(axis=1))[0]
         assert bad.size == 0, f"passes={passes}: {bad.size} entries differ, first row {bad[0] // nrhs}"
+
+
+@pytest.mark.parametrize("bits", [64, 256, 640])
+def test_sign_zero_entry_at_every_digit_offset(capi, oracle, bits):
+    """One record of sign 0 with limbs in a column whose other terms are zeros, at every offset of its mantissa in the
+    26-bit digits: on some of them a block that takes its limbs for a value still decides the entry's rounding."""
+    rng = np.random.default_rng(bits)
+    n, w = 3, bits // 32
+    A = np.stack([lfcases.zero(bits)] * (n * n))
+    for i in range(n):
+        A[i * n + i] = lfcases.random_records(rng, bits, 1, 0)[0]
+        A[i * n + i, w + 1] = 1
+    clean = A.copy()
+    want, piv, _, _ = oracle.cholesky(bits, clean, n, 32)
+    assert piv == n
+    for e in range(-13, 13):
+        A[n] = lfcases.random_records(rng, bits, 1, 0)[0]
+        A[n, w], A[n, w + 1] = lfcases.i32(e), 0
+        got, info = capi.cholesky(bits, A, n, block=32)
+        assert info.pivot == n
+        bad = np.nonzero((got != want).any(axis=1))[0]
+        assert bad.size == 0, f"exponent {e}: {bad.size} entries differ, first ({bad[0] // n},{bad[0] % n})"
