@@ -652,34 +652,15 @@ template <int N> __global__ void __launch_bounds__(256) zero_upper_kernel(u32* w
 }
 
 // ---------------------------------------------------------------- triangular blocks
-// One block of a forward or backward solve, or of the rows below a Cholesky block, one wavefront per
-// right-hand side (row): the wave-parallel recurrence as far as it goes, then the general one.  What bounds it
-// is one wavefront's instruction count: at 256 bits a 32-row block took 163-167 us with the general recurrence
-// (an exact dot of the row's terms and a one-lane division per row).  With a digit per lane the solve of 512
-// unknowns and 64 right-hand sides went from 7.70 to 4.00 ms, the factorization of n = 512 from 12.3 to 10.9 ms.
-template <int N> constexpr u32 tri_waves() { return wd_fits<N>() ? TRI_WAVES : 1; }
-template <int N> __global__ void __launch_bounds__(64 * tri_waves<N>()) tri_block_kernel(TriArgs g)
+// Rows i .. B - 1 of right-hand side c by the general recurrence, one wavefront (c, i and B uniform).  Its own stores
+// are terms of its later rows.
+template <int N> __device__ __forceinline__ void tri_rows(const TriArgs& g, u32 c, u32 i, u32 B, u32 lane, WaveLds<N>& L)
 {
-    constexpr std::size_t bytes = wd_fits<N>() ? sizeof(TriLds<N>) : sizeof(WaveLds<N>);
-    __shared__ __attribute__((aligned(16))) unsigned char lds[bytes];
-    const u32 wave = threadIdx.x / 64u, lane = threadIdx.x % 64u, c = blockIdx.x * tri_waves<N>() + wave;
-    u32 B = g.rows;
-    if (g.info) {
-        const int32_t p = g.info->pivot;
-        if (p >= 0) B = (u32)p > g.k0 ? (u32)p - g.k0 : 0u; // (nothing where an earlier block failed)
-    }
-    u32 i = 0;
-    if constexpr (wd_fits<N>())
-        if (B <= WD_ROWS) i = tri_block_fast<N>(g, c, B, wave, lane, *reinterpret_cast<TriLds<N>*>(lds));
-    if (i >= B || c >= g.count) return;
-    // the general recurrence, in the LDS of this wavefront's accumulators; its own stores are terms of later rows
-    static_assert(!wd_fits<N>() || sizeof(WaveLds<N>) <= sizeof(i64) * WD_ROWS * (WD_COLS + 1), "the exact dot's rows fit the accumulators");
-    WaveLds<N>& L = *reinterpret_cast<WaveLds<N>*>(lds + wave * sizeof(i64) * WD_ROWS * (WD_COLS + 1));
     const DotScratch sc{g.scratch + (u64)c * 2 * g.swords, g.swords, g.error};
     const i64 xb = g.xbase + (i64)c * g.xc;
     const VecView xv{g.x, g.xpitch, xb, g.xr};
     for (; i < B; ++i) {
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         const VecView li{g.f, g.fpitch, g.fbase + (i64)i * g.fr, g.fk};
         const u64 at = (u64)(xb + (i64)i * g.xr);
         const Num<N> v = wave_dot_sub<N>(load_out<N>(g.x, g.xpitch, at), li, xv, i, lane, L, sc);
@@ -690,6 +671,37 @@ template <int N> __global__ void __launch_bounds__(64 * tri_waves<N>()) tri_bloc
             store_out<N>(g.x, g.xpitch, 0, 0, (u32)at, false, div_by_reciprocal<N>(v, l, rv));
         }
     }
+}
+// Rows of the block before a failed pivot (all of them where none failed, none where an earlier block did).
+__device__ __forceinline__ u32 tri_limit(const TriArgs& g)
+{
+    const int32_t p = g.info ? g.info->pivot : -1;
+    return p < 0 ? g.rows : (u32)p > g.k0 ? (u32)p - g.k0 : 0u;
+}
+
+// One block of a forward or backward solve, or of the rows below a Cholesky block, one wavefront per
+// right-hand side (row): the wave-parallel recurrence as far as it goes, then the general one.  What bounds it
+// is one wavefront's instruction count: at 256 bits a 32-row block took 163-167 us with the general recurrence
+// (an exact dot of the row's terms and a one-lane division per row).  With a digit per lane the solve of 512
+// unknowns and 64 right-hand sides went from 7.70 to 4.00 ms, the factorization of n = 512 from 12.3 to 10.9 ms.
+template <int N> __global__ void __launch_bounds__(64 * TRI_WAVES) tri_block_kernel(TriArgs g)
+{
+    __shared__ __attribute__((aligned(16))) unsigned char lds[sizeof(TriLds<N>)];
+    // (as a scalar: what follows from the wavefront's number is the same in all its lanes)
+    const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), lane = threadIdx.x % 64u;
+    const u32 c = blockIdx.x * TRI_WAVES + wave, B = tri_limit(g);
+    const u32 i = tri_block_fast<N>(g, c, B, wave, lane, *reinterpret_cast<TriLds<N>*>(lds));
+    if (i >= B || c >= g.count) return;
+    // the general recurrence, in the LDS of this wavefront's accumulators
+    static_assert(sizeof(WaveLds<N>) <= sizeof(i64) * WD_ROWS * (WD_COLS + 1), "the exact dot's rows fit the accumulators");
+    tri_rows<N>(g, c, i, B, lane, *reinterpret_cast<WaveLds<N>*>(lds + wave * sizeof(i64) * WD_ROWS * (WD_COLS + 1)));
+}
+
+// Blocks that the wave-parallel form does not take (more than 32 rows, values wider than 640 bits).
+template <int N> __global__ void __launch_bounds__(64) tri_general_kernel(TriArgs g)
+{
+    __shared__ WaveLds<N> L;
+    tri_rows<N>(g, blockIdx.x, 0, tri_limit(g), threadIdx.x, L);
 }
 
 // Measurement support: cycles (s_memtime) of one of the factorization's per-row steps on one wavefront

@@ -28,7 +28,12 @@ template <int N> hipError_t launch_chol_diag(const FactorArgs& f, uint32_t threa
 template <int N> hipError_t launch_tri_block(const TriArgs& g, hipStream_t s)
 {
     if (!g.count || !g.rows) return hipSuccess;
-    hipLaunchKernelGGL((tri_block_kernel<N>), dim3((g.count + tri_waves<N>() - 1) / tri_waves<N>()), dim3(64 * tri_waves<N>()), 0, s, g);
+    if constexpr (wd_fits<N>())
+        if (g.rows <= WD_ROWS) {
+            hipLaunchKernelGGL((tri_block_kernel<N>), dim3((g.count + TRI_WAVES - 1) / TRI_WAVES), dim3(64 * TRI_WAVES), 0, s, g);
+            return hipGetLastError();
+        }
+    hipLaunchKernelGGL((tri_general_kernel<N>), dim3(g.count), dim3(64), 0, s, g);
     return hipGetLastError();
 }
 
