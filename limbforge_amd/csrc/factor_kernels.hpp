@@ -179,7 +179,6 @@ __device__ __noinline__ Num<N> dot_sub_clusters(const Num<N>& c, const VecView& 
 {
     return dot_sub_clusters_inline<N>(c, x, y, K, sc);
 }
-
 // ---------------------------------------------------------------- one exact dot per wavefront
 // D(c; x, y; K) = RN(c - sum_{k<K} x_k y_k) with one rounding (the contract of the reference's
 // exact_dot_add with subtract, linalg.hpp:268-318): zero with the OR of the statuses of c and of every
@@ -199,9 +198,15 @@ constexpr int DOT_ROWS = 32; // terms per chunk
 // Row stride of the exact-dot rows: the W-word window plus one word, odd (W is even), so that the lanes
 // storing one column of their rows hit distinct banks.
 template <int N> constexpr int dot_row_stride() { return factor_window(N) + 1; }
+// The rows of one exact dot: a row a term of a chunk, then row c (the addend) and row c + 1 (per word: the negative terms
+// whose sign fill starts there).
+template <int N> struct DotRows {
+    u32 (*row)[dot_row_stride<N>()];
+    int c;
+};
 template <int N> struct alignas(16) WaveLds {
-    u32 row[DOT_ROWS + 1][dot_row_stride<N>()]; // row DOT_ROWS holds c
-    u32 neg[factor_window(N) + 1];              // per word: negative terms whose sign fill starts there
+    u32 row[DOT_ROWS + 2][dot_row_stride<N>()];
+    __device__ __forceinline__ DotRows<N> rows() { return {row, DOT_ROWS}; }
 };
 
 __device__ __forceinline__ void wave_sync()
@@ -267,7 +272,7 @@ template <bool MAX> __device__ __forceinline__ int wave_extreme32(int v)
 // at word offset o = rel / 32, two's complement within those words for a negative term; the rest of a
 // negative term's W-word two's complement (ones from word o+S+1 up) is left out and counted in neg[o+S+1]
 // instead, for the column sums to take off (sg in {-1, 0, 1}; rel >= 0 and the term fits: rel + 32S <= 32W - 1).
-template <int N, int S> __device__ __forceinline__ void put_row(WaveLds<N>& L, int r, const u32 (&src)[S], i64 rel, int sg)
+template <int N, int S> __device__ __forceinline__ void put_row(const DotRows<N>& L, int r, const u32 (&src)[S], i64 rel, int sg)
 {
     constexpr int W = factor_window(N);
     static_assert(S + 1 <= W, "a term fits the window");
@@ -291,21 +296,21 @@ template <int N, int S> __device__ __forceinline__ void put_row(WaveLds<N>& L, i
             q[t] = (u32)v;
             c = (u32)(v >> 32);
         }
-        if (nonzero && o + S + 1 < W) atomicAdd(&L.neg[o + S + 1], 1u);
+        if (nonzero && o + S + 1 < W) atomicAdd(&L.row[L.c + 1][o + S + 1], 1u);
     }
     u32* row = &L.row[r][o];
 #pragma unroll
     for (int t = 0; t <= S; ++t) row[t] = q[t];
 }
 
-// Clear the rows and the sign-fill counts of a wave's exact-dot LDS (all lanes, 16-byte stores).
-template <int N> __device__ __forceinline__ void clear_rows(WaveLds<N>& L, u32 lane)
+// Clear the rows and the sign-fill counts of a wave's exact dot (all lanes, 16-byte stores; the rows start at a multiple of
+// 16 bytes).
+template <int N> __device__ __forceinline__ void clear_rows(const DotRows<N>& L, u32 lane)
 {
-    static_assert(sizeof(WaveLds<N>) % 4 == 0, "whole words");
-    constexpr u32 words = sizeof(WaveLds<N>) / 4, quads = words / 4;
-    uint4* q = reinterpret_cast<uint4*>(&L);
+    const u32 words = (u32)(L.c + 2) * dot_row_stride<N>(), quads = words / 4;
+    uint4* q = reinterpret_cast<uint4*>(L.row);
     for (u32 k = lane; k < quads; k += WAVE) q[k] = make_uint4(0u, 0u, 0u, 0u);
-    u32* w = reinterpret_cast<u32*>(&L);
+    u32* w = &L.row[0][0];
     for (u32 k = 4 * quads + lane; k < words; k += WAVE) w[k] = 0u;
 }
 
@@ -419,7 +424,7 @@ __device__ __forceinline__ Num<N> wave_round(const u64 (&S)[(factor_window(N) + 
 }
 
 template <int N, bool INLINE = false>
-__device__ Num<N> wave_dot_sub(const Num<N>& c, const VecView& x, const VecView& y, u32 K, u32 lane, WaveLds<N>& L, const DotScratch& sc)
+__device__ Num<N> wave_dot_sub(const Num<N>& c, const VecView& x, const VecView& y, u32 K, u32 lane, const DotRows<N>& L, const DotScratch& sc)
 {
     constexpr int W = factor_window(N);
     constexpr int CPL = (W + WAVE - 1) / WAVE; // window columns per lane
@@ -519,17 +524,17 @@ __device__ Num<N> wave_dot_sub(const Num<N>& c, const VecView& x, const VecView&
             }
         }
         const bool with_c = kb == 0 && c.s != 0;
-        if (with_c && lane == WAVE - 1) put_row<N, N>(L, DOT_ROWS, c.w, (i64)c.e - (32 * N - 1) - lo, c.s);
+        if (with_c && lane == WAVE - 1) put_row<N, N>(L, L.c, c.w, (i64)c.e - (32 * N - 1) - lo, c.s);
         wave_sync();
 #pragma unroll
         for (int t = 0; t < CPL; ++t) {
             const int w = (int)lane + WAVE * t;
             if (w < W) {
-                u64 sum = with_c ? (u64)L.row[DOT_ROWS][w] : 0u;
+                u64 sum = with_c ? (u64)L.row[L.c][w] : 0u;
 #pragma unroll 8
                 for (u32 r = 0; r < rows; ++r) sum += L.row[r][w];
                 S[t] += sum;
-                H[t] += L.neg[w];
+                H[t] += L.row[L.c + 1][w];
             }
         }
         wave_sync();
@@ -551,13 +556,6 @@ template <int N> __device__ __forceinline__ Num<N> element(const FactorArgs& f, 
     return load_out<N>(f.w, f.pitch, (u64)i * f.n + j);
 }
 
-// The reciprocal of the pivot or diagonal entry i: its leading N+1 words (limb_core.hpp reciprocal) are the last
-// planes stored.
-template <int N> __device__ __forceinline__ void load_recip(const u32* r, u64 rpitch, u64 i, u32 (&v)[N + 1])
-{
-#pragma unroll
-    for (int k = 0; k <= N; ++k) v[k] = r[(u64)(k + recip_words<N>() - (N + 1)) * rpitch + i];
-}
 template <int N> __device__ __forceinline__ void store_recip(u32* r, u64 rpitch, u32 i, const Num<N>& d)
 {
     u32 v[recip_words<N>()];
@@ -593,7 +591,7 @@ template <int N> __global__ void __launch_bounds__(diag_waves<N>() * WAVE) chol_
     __shared__ WaveLds<N> lds[DW];
     __shared__ int stop;
     const u32 wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    WaveLds<N>& L = lds[wave];
+    const DotRows<N> L = lds[wave].rows();
     const DotScratch sc{f.scratch + (u64)wave * 2 * f.swords, f.swords, f.error};
     if (f.info->pivot >= 0) return; // a block before this one failed
     for (u32 j = f.k0 + (resume ? (u32)f.info->resume : 0u); j < f.k1; ++j) {
@@ -654,7 +652,7 @@ template <int N> __global__ void __launch_bounds__(256) zero_upper_kernel(u32* w
 // ---------------------------------------------------------------- triangular blocks
 // Rows i .. B - 1 of right-hand side c by the general recurrence, one wavefront (c, i and B uniform).  Its own stores
 // are terms of its later rows.
-template <int N> __device__ __forceinline__ void tri_rows(const TriArgs& g, u32 c, u32 i, u32 B, u32 lane, WaveLds<N>& L)
+template <int N> __device__ __forceinline__ void tri_rows(const TriArgs& g, u32 c, u32 i, u32 B, u32 lane, const DotRows<N>& L)
 {
     const DotScratch sc{g.scratch + (u64)c * 2 * g.swords, g.swords, g.error};
     const i64 xb = g.xbase + (i64)c * g.xc;
@@ -680,28 +678,23 @@ __device__ __forceinline__ u32 tri_limit(const TriArgs& g)
 }
 
 // One block of a forward or backward solve, or of the rows below a Cholesky block, one wavefront per
-// right-hand side (row): the wave-parallel recurrence as far as it goes, then the general one.  What bounds it
-// is one wavefront's instruction count: at 256 bits a 32-row block took 163-167 us with the general recurrence
-// (an exact dot of the row's terms and a one-lane division per row).  With a digit per lane the solve of 512
-// unknowns and 64 right-hand sides went from 7.70 to 4.00 ms, the factorization of n = 512 from 12.3 to 10.9 ms.
+// right-hand side (row).  What bounds it is one wavefront's instruction count: at 256 bits a 32-row block took
+// 163-167 us with the general recurrence (an exact dot of the row's terms and a one-lane division per row).  With a
+// digit per lane the solve of 512 unknowns and 64 right-hand sides went from 7.70 to 4.00 ms, the factorization of
+// n = 512 from 12.3 to 10.9 ms.
 template <int N> __global__ void __launch_bounds__(64 * TRI_WAVES) tri_block_kernel(TriArgs g)
 {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[sizeof(TriLds<N>)];
+    __shared__ TriLds<N> lds;
     // (as a scalar: what follows from the wavefront's number is the same in all its lanes)
     const u32 wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64u), lane = threadIdx.x % 64u;
-    const u32 c = blockIdx.x * TRI_WAVES + wave, B = tri_limit(g);
-    const u32 i = tri_block_fast<N>(g, c, B, wave, lane, *reinterpret_cast<TriLds<N>*>(lds));
-    if (i >= B || c >= g.count) return;
-    // the general recurrence, in the LDS of this wavefront's accumulators
-    static_assert(sizeof(WaveLds<N>) <= sizeof(i64) * WD_ROWS * (WD_COLS + 1), "the exact dot's rows fit the accumulators");
-    tri_rows<N>(g, c, i, B, lane, *reinterpret_cast<WaveLds<N>*>(lds + wave * sizeof(i64) * WD_ROWS * (WD_COLS + 1)));
+    tri_block<N>(g, blockIdx.x * TRI_WAVES + wave, tri_limit(g), wave, lane, lds);
 }
 
 // Blocks that the wave-parallel form does not take (more than 32 rows, values wider than 640 bits).
 template <int N> __global__ void __launch_bounds__(64) tri_general_kernel(TriArgs g)
 {
     __shared__ WaveLds<N> L;
-    tri_rows<N>(g, blockIdx.x, 0, tri_limit(g), threadIdx.x, L);
+    tri_rows<N>(g, blockIdx.x, 0, tri_limit(g), threadIdx.x, L.rows());
 }
 
 // Measurement support: cycles (s_memtime) of one of the factorization's per-row steps on one wavefront
@@ -714,7 +707,8 @@ template <int N, int STEP>
 __global__ void __launch_bounds__(64) factor_steps_kernel(const u32* v, u64 pitch, u32* scratch, u64 swords, int32_t* err, int reps, u64* out,
                                                          u32* sink)
 {
-    __shared__ WaveLds<N> L;
+    __shared__ WaveLds<N> lds;
+    const DotRows<N> L = lds.rows();
     const u32 lane = threadIdx.x;
     u32 chk = 0;
     if constexpr (STEP == 0) {

@@ -122,7 +122,7 @@ template <int N> __global__ void __launch_bounds__(64 * UPD_WAVES, 4) update_wav
             const u32 e = (u32)__builtin_ctzll(rest), i = r0 + e / tc, j = c0 + e % tc;
             const VecView x{g.x, g.xpitch, g.xbase + (i64)i * g.xr, g.xk}, y{g.y, g.ypitch, g.ybase + (i64)j * g.yc, g.yk};
             const u64 at = (u64)(g.obase + (i64)i * g.orow + (i64)j * g.ocol);
-            const Num<N> v = wave_dot_sub<N, true>(load_out<N>(g.out, g.opitch, at), x, y, g.K, lane, reinterpret_cast<WaveLds<N>*>(lds)[wave], sc);
+            const Num<N> v = wave_dot_sub<N, true>(load_out<N>(g.out, g.opitch, at), x, y, g.K, lane, reinterpret_cast<WaveLds<N>*>(lds)[wave].rows(), sc);
             if (lane == 0) store_out<N>(g.out, g.opitch, 0, 0, (u32)at, false, v);
         }
     }
@@ -132,7 +132,8 @@ template <int N> __global__ void __launch_bounds__(64 * UPD_WAVES, 4) update_wav
 // scratch slot b.
 template <int N> __global__ void __launch_bounds__(64) update_kernel(UpdateArgs g)
 {
-    __shared__ WaveLds<N> L;
+    __shared__ WaveLds<N> lds;
+    const DotRows<N> L = lds.rows();
     const u32 lane = threadIdx.x;
     const u64 entries = (u64)g.rows * g.cols;
     const DotScratch sc{g.scratch + (u64)blockIdx.x * 2 * g.swords, g.swords, g.error};

@@ -231,6 +231,22 @@ template <int N, int M> __device__ __forceinline__ void reciprocal_words(const u
     for (int j = M - 2; j >= 0; --j) v[j] = knuth_step<N>(R, b, 0xffffffffu, inv);
 }
 
+// The reciprocal of the pivot or diagonal entry i: its leading N+1 words (limb_core.hpp reciprocal) are the last
+// planes stored.
+template <int N> __device__ __forceinline__ void load_recip(const u32* r, u64 rpitch, u64 i, u32 (&v)[N + 1])
+{
+#pragma unroll
+    for (int k = 0; k <= N; ++k) v[k] = r[(u64)(k + recip_words<N>() - (N + 1)) * rpitch + i];
+}
+// A wave number from a record in LDS (its status apart).
+template <int N> __device__ __forceinline__ WaveNum wd_from_record(const u32* rec, u32 lane)
+{
+    const u32 wi = WD_BITS * lane / 32u, s = WD_BITS * lane % 32u;
+    const u32 lo = wi < (u32)N ? rec[wi] : 0u, hi = wi + 1 < (u32)N ? rec[wi + 1] : 0u;
+    return {(u32)((((u64)hi << 32) | lo) >> s) & WD_MASK, (i64)__builtin_amdgcn_readfirstlane((int)rec[N]),
+            __builtin_amdgcn_readfirstlane((int)rec[N + 1])};
+}
+
 // ------------------------------------------------------------------ triangular blocks
 // LDS of a block: the signed grid digits of the strict lower triangle packed by columns with their origins (zero
 // entries: WD_ZERO), the reciprocals of the diagonal between zeros, so that lane c reads digit c - i without a
@@ -240,12 +256,12 @@ constexpr u32 WD_ROWS = 32;
 constexpr int WD_TRI = WD_ROWS * (WD_ROWS - 1) / 2;
 constexpr int WD_ZERO = 0x7fffffff;
 constexpr u32 TRI_WAVES = 4;
-template <int N> struct TriLds {
+template <int N> struct alignas(16) TriLds {
     i64 acc[TRI_WAVES][WD_ROWS][WD_COLS + 1];
     int digit[wd_grid<N>()][WD_TRI];
     int origin[WD_TRI];
     u32 recip[WD_ROWS][wd_mant<N>() - 1 + WD_COLS];
-    int odd; // a status in the block, or a zero on its diagonal
+    u32 odd; // rows with a status in the block
 };
 
 // first index of column k of the strict lower triangle: rows k + 1 .. WD_ROWS - 1
@@ -271,13 +287,56 @@ template <int GD, int H> __device__ __forceinline__ void wd_accumulate(i64* at, 
     }
 }
 
+// Row i's exact dot and its one-lane division, for rows that the wave-parallel forms do not decide: the dot's record
+// goes to `rec`, the division replaces it by the quotient's and stores x_i.  `rec` is also the dot's LDS, of rows
+// 0 .. i + 1.  Both read the kernel's arguments again, through a pointer that the compiler cannot follow, so that neither
+// they nor what is formed from them takes scalar registers of the recurrence's loop (which spilled them: 57 instead of
+// 52 us a block).
+__device__ __forceinline__ TriArgs tri_args_again()
+{
+    typedef const __attribute__((address_space(4))) TriArgs* args_ptr; // the kernel's one argument
+    args_ptr p = (args_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const TriArgs*)p;
+}
+template <int N> __device__ __forceinline__ void tri_exact_dot(u32 c, u32 i, u32 lane, u32* rec)
+{
+    const TriArgs g = tri_args_again();
+    const i64 xb = g.xbase + (i64)c * g.xc;
+    wave_sync();
+    const Num<N> d = wave_dot_sub<N>(load_out<N>(g.x, g.xpitch, (u64)(xb + (i64)i * g.xr)), VecView{g.f, g.fpitch, g.fbase + (i64)i * g.fr, g.fk},
+                                     VecView{g.x, g.xpitch, xb, g.xr}, i, lane,
+                                     DotRows<N>{reinterpret_cast<u32(*)[dot_row_stride<N>()]>(rec), (int)i},
+                                     DotScratch{g.scratch + (u64)c * 2 * g.swords, g.swords, g.error});
+    if (lane == 0) store_out<N>(rec, 1, 0, 0, 0, false, d);
+    wave_sync();
+}
+template <int N> __device__ __forceinline__ void tri_exact_divide(u32 c, u32 i, u32 lane, u32* rec)
+{
+    const TriArgs g = tri_args_again();
+    if (lane == 0) {
+        u32 rv[N + 1];
+        load_recip<N>(g.recip, g.rpitch, (u64)(g.rbase + (i64)i * g.rstep), rv);
+        const Num<N> l = load_out<N>(g.f, g.fpitch, (u64)(g.fbase + (i64)i * (g.fr + g.fk)));
+        const Num<N> q = div_by_reciprocal<N>(load_out<N>(rec, 1, 0), l, rv);
+        store_out<N>(g.x, g.xpitch, 0, 0, (u32)(g.xbase + (i64)c * g.xc + (i64)i * g.xr), false, q);
+        store_out<N>(rec, 1, 0, 0, 0, false, q);
+    }
+    wave_sync();
+}
+
 // The recurrence x_r = (b_r - sum_{k<r} l_rk x_k) / l_rr over the rows of a block of up to 32 rows, one
 // rounding of the exact sum and one of the quotient per row, for right-hand side c on one wavefront of the
-// workgroup.  Returns the rows done: all of them, or the first one that needs the general routines (a status, a
-// zero divisor, terms spread past the accumulator's columns, a quotient too close to a rounding boundary).
+// workgroup.  A row whose terms spread past its columns takes the exact dot of them instead (in the LDS of the
+// accumulators up to its own, which no later row needs), a quotient too close to a rounding boundary the one-lane
+// division, and the recurrence goes on from their result: where most rows of a block need the exact dot, the division
+// and the sums that stay in their columns still pay for the digits (terms spread over 700 bits, 256-bit values: 164 us a
+// block, 640 bits: 330 us; with the exact dot and the one-lane division for every row 169 and 400 us, and 259 and 680 us
+// where the digits gave up the rest of a block at its first such row).  After the first row that ends in a status every row
+// is a zero with the statuses of its terms, which are all that it reads.
 // The block is staged by the whole workgroup: its loads' latency, 16 rounds of them for one wavefront, was about
 // a quarter of the kernel.
-template <int N> __device__ __forceinline__ u32 tri_block_fast(const TriArgs& g, u32 c, u32 B, u32 wave, u32 lane, TriLds<N>& L)
+template <int N> __device__ __forceinline__ void tri_block(const TriArgs& g, u32 c, u32 B, u32 wave, u32 lane, TriLds<N>& L)
 {
     constexpr int D = wd_mant<N>(), GD = wd_grid<N>(), RD = wd_recip<N>(), H = (GD + 1) / 2;
     const u32 t = 64u * wave + lane, row = lane & 31u, half = lane >> 5;
@@ -295,7 +354,7 @@ template <int N> __device__ __forceinline__ u32 tri_block_fast(const TriArgs& g,
     for (u32 k = t >> 5; k < B; k += 2u * TRI_WAVES)
         if (row > k && row < B) {
             const Num<N> l = load_out<N>(g.f, g.fpitch, (u64)(g.fbase + (i64)row * g.fr + (i64)k * g.fk));
-            if (l.st) L.odd = 1;
+            if (l.st) atomicOr(&L.odd, 1u << row);
             int d[GD], o;
             lane_to_grid<N>(l, d, o);
             const u32 at = wd_col_start(k) + (row - k - 1);
@@ -337,52 +396,99 @@ template <int N> __device__ __forceinline__ u32 tri_block_fast(const TriArgs& g,
         }
     }
     __syncthreads();
-    if (!mine) return B;
-    if (L.odd || __ballot(odd)) return 0;
+    if (!mine) return;
+    // the first row with a status or a zero divisor: it and all rows after it end in a status
+    const u32 odds = L.odd | (u32)__ballot(odd), first = odds ? (u32)__builtin_ctz(odds) : WD_ROWS;
     // both lanes of a row carry its origin
     alpha = __shfl(alpha, (int)row);
     placed = __shfl((int)placed, (int)row) != 0;
     i64(&acc)[WD_ROWS][WD_COLS + 1] = L.acc[wave];
-    u64 outside = 0; // rows with a term outside their columns
-    for (u32 i = 0; i < B; ++i) {
-        if ((outside >> i) & 1u) return i;
-        u32 Rs[D];
+    static_assert(2 * dot_row_stride<N>() * 4 <= (WD_COLS + 1) * 8, "the rows of an exact dot of i terms fit the accumulators of rows 0 .. i");
+    u32* rec = reinterpret_cast<u32*>(&acc[0][0]);
+    u32 outside = 0; // rows with a term outside their columns
+    WaveNum v, x{0, 0, 0};
+    for (u32 i = 0;; ++i) {
+        // rows as far as the digits decide them; what they do not decide stays out of this loop, whose registers it would
+        // spill (57 instead of 52 us a block)
+        bool summed = false;
+        for (; i < B; ++i) {
+            if (x.s) { // the terms of row k = i - 1
+                const u32 k = i - 1;
+                int xo;
+                const int gx = (int)wd_to_grid<N>(x, xo);
+                const int sx = x.s > 0 ? -gx : gx; // the term is subtracted
+                int xd[H];
 #pragma unroll
-        for (int k = 0; k < D; ++k) Rs[k] = L.recip[i][D - 1 + (int)lane - k];
-        const i64 S = acc[i][lane];
-        WaveNum v, x;
-        if (!wd_round<N>(S, (i64)(int)wd_read((u32)alpha, (int)i), lane, v)) return i;
-        if (!wd_divide<N>(v, Rs, (i64)(int)wd_read((u32)le, (int)i), (int)wd_read((u32)ls, (int)i), lane, x)) return i;
-        wd_store<N>(g.x, g.xpitch, xb + (u64)((i64)i * g.xr), x, lane);
-        if (!x.s || i + 1 >= B) continue;
-        int xo;
-        const int gx = (int)wd_to_grid<N>(x, xo);
-        const int sx = x.s > 0 ? -gx : gx; // the term is subtracted
-        int xd[H];
+                for (int j = 0; j < H; ++j) xd[j] = __shfl(sx, j + H * (int)half);
+                const bool live = row > k && row < B;
+                const u32 at = wd_col_start(k) + (live ? row - k - 1 : 0u);
+                const int lo = live ? L.origin[at] : WD_ZERO;
+                bool bad = false;
+                if (lo != WD_ZERO) {
+                    if (!placed) {
+                        alpha = lo + xo + 2 * GD - 1 - wd_center<N>();
+                        placed = true;
+                    }
+                    const int o = lo + xo - alpha;
+                    bad = o < 0 || o + 2 * GD - 1 > WD_TOP;
+                    if (!bad) {
+                        int ld[GD];
 #pragma unroll
-        for (int j = 0; j < H; ++j) xd[j] = __shfl(sx, j + H * (int)half);
-        const bool live = row > i && row < B;
-        const u32 at = wd_col_start(i) + (live ? row - i - 1 : 0u);
-        const int lo = live ? L.origin[at] : WD_ZERO;
-        bool bad = false;
-        if (lo != WD_ZERO) {
-            if (!placed) {
-                alpha = lo + xo + 2 * GD - 1 - wd_center<N>();
-                placed = true;
+                        for (int j = 0; j < GD; ++j) ld[j] = L.digit[j][at];
+                        wd_accumulate<GD, H>(&acc[row][o + H * (int)half], xd, ld);
+                    }
+                }
+                const u64 bads = __ballot(bad); // either lane of a row
+                outside |= (u32)bads | (u32)(bads >> 32);
+                wave_sync();
             }
-            const int o = lo + xo - alpha;
-            bad = o < 0 || o + 2 * GD - 1 > WD_TOP;
-            if (!bad) {
-                int ld[GD];
+            summed = false;
+            if (i >= first || ((outside >> i) & 1u)) break;
+            u32 Rs[D];
 #pragma unroll
-                for (int j = 0; j < GD; ++j) ld[j] = L.digit[j][at];
-                wd_accumulate<GD, H>(&acc[row][o + H * (int)half], xd, ld);
-            }
+            for (int k = 0; k < D; ++k) Rs[k] = L.recip[i][D - 1 + (int)lane - k];
+            const i64 S = acc[i][lane];
+            if (!wd_round<N>(S, (i64)(int)wd_read((u32)alpha, (int)i), lane, v)) break;
+            summed = true;
+            if (!wd_divide<N>(v, Rs, (i64)(int)wd_read((u32)le, (int)i), (int)wd_read((u32)ls, (int)i), lane, x)) break;
+            wd_store<N>(g.x, g.xpitch, xb + (u64)((i64)i * g.xr), x, lane);
         }
-        outside |= __ballot(bad);
-        wave_sync();
+        if (i >= B) return;
+        // row i by the exact dot, the one-lane division, or both
+        bool divided = false;
+        if (!summed) {
+            tri_exact_dot<N>(c, i, lane, rec);
+            v = wd_from_record<N>(rec, lane);
+            if (i < first && !__builtin_amdgcn_readfirstlane((int)rec[N + 2])) {
+                u32 Rs[D];
+#pragma unroll
+                for (int k = 0; k < D; ++k) Rs[k] = L.recip[i][D - 1 + (int)lane - k];
+                divided = wd_divide<N>(v, Rs, (i64)(int)wd_read((u32)le, (int)i), (int)wd_read((u32)ls, (int)i), lane, x);
+            }
+        } else {
+            wave_sync();
+            const u32 w = wd_record_word<N>(v, lane);
+            if (lane < (u32)N + 3) rec[lane] = w;
+            wave_sync();
+        }
+        if (divided) {
+            wd_store<N>(g.x, g.xpitch, xb + (u64)((i64)i * g.xr), x, lane);
+            continue;
+        }
+        tri_exact_divide<N>(c, i, lane, rec);
+        x = wd_from_record<N>(rec, lane);
+        if (!__builtin_amdgcn_readfirstlane((int)rec[N + 2])) continue;
+        // the rows after one that ended in a status
+        for (++i; i < B; ++i) {
+            const u64 fat = (u64)(g.fbase + (i64)i * g.fr + (i64)lane * g.fk), xat = xb + (u64)((i64)lane * g.xr);
+            wave_sync();
+            u32 st = 0;
+            if (lane <= i) st = g.f[(u64)(N + 2) * g.fpitch + fat] | g.x[(u64)(N + 2) * g.xpitch + xat];
+            st = (u32)wave_or((int)st);
+            if (lane < (u32)N + 3) g.x[(u64)lane * g.xpitch + xb + (u64)((i64)i * g.xr)] = lane == (u32)N + 2 ? st : 0u;
+        }
+        return;
     }
-    return B;
 }
 
 } // namespace lf

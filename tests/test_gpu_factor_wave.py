@@ -144,3 +144,34 @@ def test_sign_zero_entry_at_every_digit_offset(capi, oracle, bits):
         assert info.pivot == n
         bad = np.nonzero((got != want).any(axis=1))[0]
         assert bad.size == 0, f"exponent {e}: {bad.size} entries differ, first ({bad[0] // n},{bad[0] % n})"
+
+
+@pytest.mark.parametrize("bits", [64, 256, 640])
+@pytest.mark.parametrize("where", ["rhs", "factor", "diagonal", "zero", "overflow", "underflow"])
+def test_statuses_part_way(capi, oracle, bits, where):
+    """A right-hand side's status, a factor entry's, a diagonal entry's, a zero divisor, and quotients past the exponent
+    range, in the first, a middle and the last row of a block: the rows before them, those after them in the block, and
+    the updates of later blocks, in columns with and without them."""
+    rng = np.random.default_rng(bits + sum(map(ord, where)))
+    n, nrhs, w = 70, 5, bits // 32
+    for i in (0, 13, 31, 45):
+        L = triangle(rng, bits, n, 30)
+        B = lfcases.random_records(rng, bits, n * nrhs, 30)
+        if where == "rhs":
+            B[i * nrhs + 1, w + 2], B[i * nrhs + 3, w + 2] = 2, 4
+        elif where == "factor":
+            L[max(i, 1) * n + max(i, 1) // 2, w + 2] = 4
+        elif where == "diagonal":
+            L[i * (n + 1), w + 2] = 1
+        elif where == "zero":
+            L[i * (n + 1)] = lfcases.zero(bits)
+        else:
+            sign = 1 if where == "overflow" else -1
+            L[i * (n + 1), w] = lfcases.i32(-sign * 600000000)
+            B[i * nrhs + 2, w] = lfcases.i32(sign * 600000000)
+        print(f"[gpu] solve {where} bits={bits} row {i}", flush=True)
+        for passes in (1, 2):
+            want = oracle.solve(bits, L, n, B, nrhs, 32, passes)
+            got, _, _ = capi.solve(bits, passes, L, n, B, nrhs, block=32)
+            bad = np.nonzero((got != want).any(axis=1))[0]
+            assert bad.size == 0, f"row {i} passes={passes}: {bad.size} entries differ, first ({bad[0] // nrhs},{bad[0] % nrhs})"
