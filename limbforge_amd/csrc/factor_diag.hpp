@@ -105,7 +105,9 @@ template <int N, int BITS> __device__ __forceinline__ u32 wd_rsqrt(u32 y, u32 uh
 // from below, 2 r0 + (uh - 2 r0^2) y is sqrt(M) / 2 to all of them, and y (4 - l y) / 4 is 1 / l.  A root is never
 // halfway between two mantissas; false when the 24 bits below the last one do not tell which side of halfway it
 // lies on (about one root in 2^23), or when R's last words are too close to a carry for its leading words to be
-// those of the exact quotient.
+// those of the exact quotient (about one in 2^31 of the others).  That would be every root that is a power of two
+// (2^(64N + 64) / L is one itself), and such roots are common: a unit diagonal's, an identity's, those of scaled integers.
+// Their reciprocal, ones in all its bits, is known.
 template <int N> __device__ __forceinline__ bool wd_sqrt(const WaveNum& s, u32 lane, WaveNum& l, u32& R)
 {
     constexpr int D = wd_mant<N>(), F = wd_frac<N>();
@@ -131,6 +133,13 @@ template <int N> __device__ __forceinline__ bool wd_sqrt(const WaveNum& s, u32 l
     else if (sh < 0 && sh > -WD_BITS) y = (u32)(z << -sh) & WD_MASK;
     const u32 uhr = wd_raise<F>(uh, lane);
     u32 p, g, r, c;
+    auto power_of_two = [&]() -> bool {
+        constexpr int ones = 32 * N + 65; // bits of 2^(32N + 65) - 1
+        if (wd_read(l.m, D - 1) != 1u << (32 * N - 1 - WD_BITS * (D - 1)) || __ballot(l.m != 0) != (u64)1 << (D - 1)) return false;
+        const int left = ones - WD_BITS * (int)lane;
+        R = left >= WD_BITS ? WD_MASK : left > 0 ? (1u << left) - 1u : 0u;
+        return true;
+    };
     auto root = [&](int sigma) -> bool {
         l.m = wd_shift_right(p, sigma, lane);
         l.e = e;
@@ -155,6 +164,7 @@ template <int N> __device__ __forceinline__ bool wd_sqrt(const WaveNum& s, u32 l
         const u32 d = wd_loose(32 * (i64)uhr - wd_columns<F, 0, 0>(qa, qa, lane));
         p = wd_resolve(wd_columns<F, 0, F>(d, Y, lane) + (lane >= (u32)F ? 64 * (i64)(int)q0 : 0), lane);
         if (!root(2 * WD_BITS * F - 32 * N + 8)) return false;
+        if (power_of_two()) return true;
         c = wd_loose(((int)lane == 2 * F ? (i64)32 : 0) - wd_columns<F, 0, 0>(Y, r, lane));
         R = wd_shift_right(wd_resolve(wd_columns<F, 0, F>(c, Y, lane), lane), 2 * WD_BITS * F - 32 * N - 57, lane);
     } else {
@@ -163,6 +173,7 @@ template <int N> __device__ __forceinline__ bool wd_sqrt(const WaveNum& s, u32 l
         const u32 d2 = wd_resolve((i64)uhr - 2 * wd_columns<F, 0, 0>(r0, r0, lane), lane);
         p = wd_resolve(wd_columns<F, 0, F>(d2, y, lane) + (lane >= (u32)F ? 2 * (i64)p0 : 0), lane);
         if (!root(2 * WD_BITS * F - 32 * N)) return false;
+        if (power_of_two()) return true;
         c = wd_resolve(((int)lane == 2 * F ? (i64)4 : 0) - wd_columns<F, 0, 0>(y, r, lane), lane);
         R = wd_shift_right(wd_resolve(wd_columns<F, 0, F>(c, y, lane), lane), 2 * WD_BITS * F - 32 * N - 63, lane);
     }

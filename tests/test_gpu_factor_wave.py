@@ -175,3 +175,45 @@ def test_statuses_part_way(capi, oracle, bits, where):
             got, _, _ = capi.solve(bits, passes, L, n, B, nrhs, block=32)
             bad = np.nonzero((got != want).any(axis=1))[0]
             assert bad.size == 0, f"row {i} passes={passes}: {bad.size} entries differ, first ({bad[0] // nrhs},{bad[0] % nrhs})"
+
+
+@pytest.mark.parametrize("bits", [64, 256, 288, 640])
+@pytest.mark.parametrize("diagonal", ["ones", "powers", "mixed"])
+def test_pivots_that_are_powers_of_two(capi, oracle, bits, diagonal):
+    """Roots that are powers of two, whose reciprocals are too: a unit diagonal (the first pivot of every such matrix), a
+    diagonal matrix of powers of four and of two (every pivot, every other one), and such blocks beside general ones."""
+    rng = np.random.default_rng(bits + len(diagonal))
+    n, w = 67, bits // 32
+    A = np.stack([lfcases.zero(bits)] * (n * n))
+    for i in range(n):
+        e = 0 if diagonal == "ones" else int(rng.integers(-9, 10))
+        A[i * n + i] = lfcases.one(bits, e)
+        for j in range(i):
+            if diagonal == "ones" or (diagonal == "mixed" and i >= 32 and rng.random() < 0.3):
+                x = lfcases.random_records(rng, bits, 1, 0)[0]
+                x[w] = lfcases.i32(-22 - int(rng.integers(0, 9)))
+                A[i * n + j] = A[j * n + i] = x
+    want, piv, _, _ = oracle.cholesky(bits, A, n, 32)
+    got, info = capi.cholesky(bits, A, n, block=32)
+    assert info.pivot == piv == n
+    bad = np.nonzero((got != want).any(axis=1))[0]
+    assert bad.size == 0, f"{bad.size} entries differ, first ({bad[0] // n},{bad[0] % n})"
+
+
+@pytest.mark.parametrize("bits", [b for b in range(64, 641, 32) if b not in BITS])
+def test_every_width(capi, oracle, bits):
+    """The widths between those above: the digit counts, the room of the columns and the pivot's iteration differ at each."""
+    rng = np.random.default_rng(17 * bits)
+    n, nrhs, block = 40, 3, 32
+    for kind in ("moderate", "spread"):
+        A = spd(oracle, rng, bits, n, kind)
+        want, piv, psign, pstat = oracle.cholesky(bits, A, n, block)
+        got, info = capi.cholesky(bits, A, n, block=block)
+        assert (info.pivot, info.pivot_sign, info.pivot_status) == (piv, psign, pstat)
+        assert (got == want).all(), kind
+    for span in (30, 600):
+        L = triangle(rng, bits, n, span)
+        B = special_mantissas(rng, lfcases.random_records(rng, bits, n * nrhs, span), bits)
+        for passes in (1, 2):
+            got, _, _ = capi.solve(bits, passes, L, n, B, nrhs, block=block)
+            assert (got == oracle.solve(bits, L, n, B, nrhs, block, passes)).all(), f"span={span} passes={passes}"
