@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstring>
 #include <limits>
+#include <map>
 #include <string>
 #include <thread>
 #include <vector>
@@ -502,6 +503,9 @@ void route_capacity(Side& s, int wx_class)
     }
 }
 
+// What a thread keeps for a device is found by the device's own number (a node in a partitioned mode shows more devices
+// than GPUs) in a std::map, whose entries stay where they are when another device's is added.
+
 // Five timing events per host thread and device, created once and reused by every product.
 hipError_t stage_events(hipEvent_t** out)
 {
@@ -513,10 +517,10 @@ hipError_t stage_events(hipEvent_t** out)
                 if (x) (void)hipEventDestroy(x);
         }
     };
-    thread_local Set sets[16];
+    thread_local std::map<int, Set> sets;
     int device = 0;
     if (hipError_t err = hipGetDevice(&device)) return err;
-    Set& s = sets[device & 15];
+    Set& s = sets[device];
     for (auto& x : s.e)
         if (!x)
             if (hipError_t err = hipEventCreate(&x)) return err;
@@ -561,18 +565,12 @@ struct PoolBuf {
     void* p = nullptr;
     hipError_t alloc(std::size_t bytes)
     {
-        thread_local std::vector<std::pair<int, Workspace>> pools; // (device, buffers)
+        thread_local std::map<int, Workspace> pools;
         int dev = 0;
         if (hipError_t e = hipGetDevice(&dev)) return e;
-        Workspace* ws = nullptr;
-        for (auto& d : pools)
-            if (d.first == dev) ws = &d.second;
-        if (!ws) {
-            pools.emplace_back(dev, Workspace{});
-            ws = &pools.back().second;
-        }
-        if (ws->slots.size() <= std::size_t(slot)) ws->slots.resize(slot + 1, {nullptr, 0});
-        auto& s = ws->slots[slot];
+        Workspace& ws = pools[dev];
+        if (ws.slots.size() <= std::size_t(slot)) ws.slots.resize(slot + 1, {nullptr, 0});
+        auto& s = ws.slots[slot];
         bytes = std::max<std::size_t>(bytes, 16);
         if (s.second < bytes) {
             if (s.first) (void)hipFree(s.first);
@@ -597,10 +595,10 @@ struct PinnedTable {
 };
 hipError_t pinned_table(std::size_t lines, GemmLine** out)
 {
-    thread_local PinnedTable tables[16];
+    thread_local std::map<int, PinnedTable> tables;
     int dev = 0;
     if (hipError_t e = hipGetDevice(&dev)) return e;
-    PinnedTable& t = tables[dev & 15];
+    PinnedTable& t = tables[dev];
     if (t.lines < lines) {
         if (t.p) (void)hipHostFree(t.p);
         t.p = nullptr;
@@ -680,8 +678,8 @@ struct ConstantCache {
 };
 ConstantCache& constant_cache(int dev)
 {
-    thread_local ConstantCache caches[16];
-    return caches[dev & 15];
+    thread_local std::map<int, ConstantCache> caches;
+    return caches[dev];
 }
 
 // Uploads `words` into new device memory, complete on return.
@@ -1293,10 +1291,10 @@ struct HostStage {
 };
 HostStage& host_stage()
 {
-    thread_local HostStage stages[16];
+    thread_local std::map<int, HostStage> stages;
     int device = 0;
     (void)hipGetDevice(&device);
-    return stages[device & 15];
+    return stages[device];
 }
 
 } // namespace
