@@ -565,20 +565,38 @@ struct PoolBuf {
     void* p = nullptr;
     hipError_t alloc(std::size_t bytes)
     {
+        std::pair<void*, std::size_t>* s = nullptr;
+        if (hipError_t e = find(&s)) return e;
+        bytes = std::max<std::size_t>(bytes, 16);
+        if (s->second < bytes) {
+            if (hipError_t e = release()) return e;
+            void* q = nullptr;
+            if (hipError_t e = hipMalloc(&q, bytes)) return e;
+            *s = {q, bytes};
+        }
+        p = s->first;
+        return hipSuccess;
+    }
+    // the slot's memory back to the device
+    hipError_t release()
+    {
+        std::pair<void*, std::size_t>* s = nullptr;
+        if (hipError_t e = find(&s)) return e;
+        if (s->first) (void)hipFree(s->first);
+        *s = {nullptr, 0};
+        p = nullptr;
+        return hipSuccess;
+    }
+
+private:
+    hipError_t find(std::pair<void*, std::size_t>** s) const
+    {
         thread_local std::map<int, Workspace> pools;
         int dev = 0;
         if (hipError_t e = hipGetDevice(&dev)) return e;
         Workspace& ws = pools[dev];
         if (ws.slots.size() <= std::size_t(slot)) ws.slots.resize(slot + 1, {nullptr, 0});
-        auto& s = ws.slots[slot];
-        bytes = std::max<std::size_t>(bytes, 16);
-        if (s.second < bytes) {
-            if (s.first) (void)hipFree(s.first);
-            s = {nullptr, 0};
-            if (hipError_t e = hipMalloc(&s.first, bytes)) return e;
-            s.second = bytes;
-        }
-        p = s.first;
+        *s = &ws.slots[slot];
         return hipSuccess;
     }
 };
@@ -809,7 +827,8 @@ bool plan_moduli(Plan& p, int bits, int logk)
 std::size_t digit_bytes(int N, int width) { return (std::size_t(4 * N) + (width + 7) / 8 + 31) / 32 * 32; }
 // Nanoseconds of the three large stages, from their measured rates on an MI355X: 2.8 per 32-deep step of a 128 x 128
 // product tile, 16 CRT multiply-adds per picosecond-thousand and 0.06 per staged band pair and output, 0.7 per
-// thousand residues.  It only has to rank two plans of one product, which differ by their moduli and rows.
+// thousand residues.  It only has to rank two plans of one product, which differ by their moduli and rows; memory is not
+// part of it (a joined plan that does not fit gives way when its buffers are reserved).
 double plan_cost(const Plan& p, int N, std::size_t rows, std::size_t cols, std::size_t lines, std::size_t K, double pairs, bool syrk)
 {
     const double tr = double((rows + PT - 1) / PT), tc = double((cols + PT - 1) / PT), tiles = syrk ? tr * (tr + 1) / 2 : tr * tc;
@@ -977,12 +996,11 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
             }
         }
     }
-    const unsigned L = plan.L;
     // extended operands: band-major member lists (linalg.mm:326-330); a side whose lines are all one band in the
     // device's table is its own list
     bool upload = false;
     auto assign_members = [&](Side& s, const Count& c) {
-        if (c.lines0 == s.count && single && !(plan.joined && P.subtract)) return c.lines0;
+        if (c.lines0 == s.count && single && !(plan.joined && P.subtract)) return;
         upload = upload || s.count;
         std::size_t next = 0;
         if (plan.joined)
@@ -996,7 +1014,6 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
         for (int b = 0; b < GEMM_MAX_BANDS; ++b)
             for (std::size_t i = 0; i < s.count; ++i)
                 if (s.lines[i].cls == 0 && s.lines[i].nb > b) s.lines[i].member[b] = int(next++);
-        return next;
     };
     if (rep) {
         rep->band_slots = uint32_t(std::min<std::size_t>(ls.histogram.size(), 65));
@@ -1044,13 +1061,38 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
         trivial = pairs_of(P.m, P.n) - gpu_out;
     }
     const uint64_t fallback_outputs = (lists[0].size() + lists[1].size() + lists[2].size()) / 2;
-    const std::size_t Me = assign_members(ls, cl), Ne = P.syrk ? Me : assign_members(rs, cr);
-    t0 = Clock::now();
-    if (upload) GEMM_HIP(hipMemcpyAsync(dtab.p, htab, sizeof(GemmLine) * nlines, hipMemcpyHostToDevice, P.stream), "upload lines");
-    // residue path
+    // digits and residues of the plan that runs.  A joined plan needs more of them than the bands where few lines have
+    // several; one that does not fit the device's free memory gives way to the bands.
     const std::size_t Kp = std::max<std::size_t>((std::max<std::size_t>(P.K, 1) + 63) / 64 * 64, 64);
-    const std::size_t Mp = (Me + PT - 1) / PT * PT, Np = (Ne + PT - 1) / PT * PT; // product tiles
+    std::size_t Mp = 0, Np = 0; // extended rows and columns in whole product tiles
     PoolBuf dig_l1{3}, dig_l0{4}, dig_r1{5}, dig_r0{6}, dres{7}, dlist[3] = {{8}, {9}, {10}};
+    const auto reserve = [&]() -> hipError_t {
+        const auto tiles = [&](const Count& c) { return ((plan.joined ? c.lines0 : c.rows) + PT - 1) / PT * PT; };
+        Mp = tiles(cl);
+        Np = tiles(cr);
+        if (!any_pair) return hipSuccess;
+        if (hipError_t e = dig_l1.alloc(plan.L * Mp * Kp)) return e;
+        if (hipError_t e = dig_l0.alloc(plan.L * Mp * Kp)) return e;
+        if (!P.syrk) {
+            if (hipError_t e = dig_r1.alloc(plan.L * Np * Kp)) return e;
+            if (hipError_t e = dig_r0.alloc(plan.L * Np * Kp)) return e;
+        }
+        return dres.alloc(plan.L * Mp * Np * 2);
+    };
+    t0 = Clock::now();
+    hipError_t reserved = reserve();
+    if (reserved == hipErrorOutOfMemory && plan.joined) {
+        (void)hipGetLastError(); // taken care of here
+        for (PoolBuf* b : {&dig_l1, &dig_l0, &dig_r1, &dig_r0, &dres}) GEMM_HIP(b->release(), "hipFree (digits, residues)");
+        plan = bands;
+        single = false;
+        reserved = reserve();
+    }
+    GEMM_HIP(reserved, "hipMalloc (digits, residues)");
+    const unsigned L = plan.L;
+    assign_members(ls, cl);
+    if (!P.syrk) assign_members(rs, cr);
+    if (upload) GEMM_HIP(hipMemcpyAsync(dtab.p, htab, sizeof(GemmLine) * nlines, hipMemcpyHostToDevice, P.stream), "upload lines");
     // events bounding the stages: start, digits done, products done, rebuild done, exact dots done (attached to the
     // kernels' own dispatches instead, they cost the 98 us of a small product 13 us more)
     hipEvent_t* ev = nullptr;
@@ -1061,14 +1103,6 @@ int lf::run_product(const Product& P, lf_linalg_report* rep, float* device_ms)
     if (any_pair) {
         GEMM_HIP(digit_table(&dt), "digit table");
         GEMM_HIP(crt_constants(L, WX, &crt), "CRT constants");
-        const std::size_t lplane = Mp * Kp, rplane = Np * Kp;
-        GEMM_HIP(dig_l1.alloc(L * lplane), "hipMalloc (digits)");
-        GEMM_HIP(dig_l0.alloc(L * lplane), "hipMalloc (digits)");
-        if (!P.syrk) {
-            GEMM_HIP(dig_r1.alloc(L * rplane), "hipMalloc (digits)");
-            GEMM_HIP(dig_r0.alloc(L * rplane), "hipMalloc (digits)");
-        }
-        GEMM_HIP(dres.alloc(std::size_t(L) * Mp * Np * 2), "hipMalloc (residues)");
     }
     for (int c = 0; c < 3; ++c)
         if (!lists[c].empty()) {

@@ -3,6 +3,9 @@ into one band each (whichever the planner's cost rule takes), extended rows that
 list (zero, status and fallback lines in between), operands whose lines are adjacent in memory or whose entries
 are, shapes around the digit kernel's 32 and 256 entries and the product's 128 x 128 tiles, and the widest and
 narrowest precisions."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
@@ -63,3 +66,62 @@ def test_symmetric_products(capi, oracle, bits, kind, rows, cols):
     lower, _, _, _ = capi.syrk(bits, A, rows, cols, lower_only=True)
     keep = np.tril(np.ones((cols, cols), bool)).reshape(-1)
     assert (lower[keep] == want[keep]).all()
+
+
+def on_a_thread(call):
+    """Runs `call` on a thread of its own, whose planner buffers go back to the device with it."""
+    failed = []
+
+    def run():
+        try:
+            call()
+        except Exception as e:  # noqa: BLE001
+            failed.append(e)
+
+    t = threading.Thread(target=run)
+    t.start()
+    t.join()
+    assert failed == []
+
+
+def free_memory(capi):
+    free, total = C.c_size_t(), C.c_size_t()
+    assert capi.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0  # the HIP runtime that the library is linked with
+    return free.value
+
+
+def test_joined_plan_that_does_not_fit_gives_way_to_the_bands(capi, oracle):
+    """A product whose few lines of two bands make the joined plan the cheaper one and the larger one, with device memory
+    left for the band plan alone: the outputs are those of the joined plan, and the oracle's in a few rows."""
+    bits, m, k = 64, 9000, 32
+    rng = np.random.default_rng(5)
+    A, B = entries(rng, bits, m * k, "rare"), entries(rng, bits, k * m, "rare")
+
+    a, b, c = capi.Buffer(bits, m * k), capi.Buffer(bits, k * m), capi.Buffer(bits, m * m)
+    a.upload(A)
+    b.upload(B)
+    on_a_thread(lambda: capi.gemm_resident(bits, False, a, b, m, m, k, c))
+    want = c.download()
+
+    def side(x, lines_first):  # lines in tiles, bands in tiles, widest line (every band is at most 30 wide)
+        e = lfcases.get_exp(x, bits).reshape((m, k) if lines_first else (k, m))
+        e = np.where((lfcases.get_sign(x, bits) != 0).reshape(e.shape), e, 10**6)
+        e = e if lines_first else e.T
+        high, low = (abs(e) <= 20).any(axis=1), (e < -100).any(axis=1)
+        return -(-m // 128) * 128, -(-int(high.sum() + low.sum()) // 128) * 128, int(max(r[r < 10**5].max() - r.min() for r in e))
+
+    (jr, br, wa), (jc, bc, wb) = side(A, True), side(B, False)
+    digits_residues = lambda width, rows, cols: ((135 + 2 * width) // 16 + 1) * (2 * rows * cols + 2 * 64 * (rows + cols))  # noqa: E731
+    joined, bands = digits_residues(max(wa, wb), jr, jc), digits_residues(30, br, bc) + 2**30  # (and their CRT stage)
+    assert joined > bands + 2**29
+    c.upload(np.zeros_like(want))
+    fill = capi.DeviceMemory(free_memory(capi) - (joined + bands) // 2)
+    print(f"[gpu] joined {joined / 2**30:.2f} GiB, bands {bands / 2**30:.2f} GiB, left {free_memory(capi) / 2**30:.2f} GiB", flush=True)
+    try:
+        on_a_thread(lambda: capi.gemm_resident(bits, False, a, b, m, m, k, c))
+    finally:
+        fill.free()
+    got = c.download()
+    assert np.array_equal(got, want)
+    for i in (0, 17, m - 1):
+        assert (got[i * m:(i + 1) * m] == oracle.gemm(bits, False, A[i * k:(i + 1) * k], B, 1, m, k)).all(), f"row {i}"
