@@ -392,7 +392,7 @@ template <int WX> __device__ __forceinline__ int read_stage(const RebuildArgs& g
 template <int CTRL> __device__ __forceinline__ u32 quad_read(u32 v) { return (u32)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, 0xF, 0xF, false); }
 
 // One pass from the residues to the rounded output where every line is one band: nothing is staged between the
-// CRT and the rounding.  Four consecutive outputs of a row form a quad of lanes, and each lane forms one quarter
+// CRT and the rounding.  Four consecutive outputs form a quad of lanes, and each lane forms one quarter
 // of the CRT words of all four, then the quad exchanges quarters: a lane's multiply-adds are as many as for one
 // output of its own, and it reads a quarter of the table from LDS.  What bounds it is those multiply-adds; with the
 // whole table read by every lane (17 16-byte reads a modulus at 67 words against 5) it was LDS bound: 158 us on
@@ -405,17 +405,22 @@ template <int N, int WX> __global__ void __launch_bounds__(ROUND_BLOCK) crt_roun
 {
     constexpr int QW = quarter_words(WX), QP = quarter_pitch(WX);
     extern __shared__ __attribute__((aligned(16))) u32 tab[];
-    const u32 block = blockDim.x, nblocks = (g.n + block - 1) / block;
-    const u32 i = blockIdx.x / nblocks, j0 = (blockIdx.x % nblocks) * block, j = j0 + threadIdx.x, quarter = threadIdx.x & 3u;
-    if (g.syrk && j0 > i) return; // the whole workgroup lies above the diagonal
+    // outputs in row order, whatever the rows' length: a workgroup takes consecutive ones
+    const u32 block = blockDim.x, total = g.m * g.n, first = blockIdx.x * block, idx = first + threadIdx.x, quarter = threadIdx.x & 3u;
+    if (g.syrk) { // nothing to do where the whole workgroup lies above the diagonal, in one row
+        const u32 i0 = first / g.n, i1 = min(first + block, total) - 1u;
+        if (first - i0 * g.n > i0 && i1 / g.n == i0) return;
+    }
     for (u32 k = threadIdx.x; k < g.L * 4 * QP; k += block) {
         const u32 q = k / (4 * QP), p = (k / QP) % 4u, w = p * QW + k % QP;
         tab[k] = k % QP < (u32)QW && w < (u32)WX ? g.crt[q * WX + w] : 0u;
     }
     __syncthreads();
-    const bool inside = j < g.n && !(g.syrk && j > i);
+    const u32 i = idx < total ? idx / g.n : 0u, j = idx < total ? idx - i * g.n : 0u;
+    const bool inside = idx < total && !(g.syrk && j > i);
+    if (!__ballot(inside)) return;
     const GemmLine* Li = g.left + i;
-    const GemmLine* Lj = g.right + (inside ? j : 0u);
+    const GemmLine* Lj = g.right + j;
     const bool live = inside && Li->cls == 0 && Lj->cls == 0;
     u64 sum[4][QW];
 #pragma unroll

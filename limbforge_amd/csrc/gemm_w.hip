@@ -29,7 +29,7 @@ template <int N, int WX> hipError_t launch_round_wx(const RoundArgs& g, hipStrea
             return e;
     // small products in workgroups of one wavefront, to spread over the GPU
     const u32 RB = (u64)g.m * g.n >= 65536 ? ROUND_BLOCK : 64u;
-    hipLaunchKernelGGL((crt_round_kernel<N, WX>), dim3(((g.n + RB - 1) / RB) * g.m), dim3(RB), lds, s, g);
+    hipLaunchKernelGGL((crt_round_kernel<N, WX>), dim3((unsigned)(((u64)g.m * g.n + RB - 1) / RB)), dim3(RB), lds, s, g);
     return hipGetLastError();
 }
 

@@ -125,3 +125,43 @@ def test_joined_plan_that_does_not_fit_gives_way_to_the_bands(capi, oracle):
     assert np.array_equal(got, want)
     for i in (0, 17, m - 1):
         assert (got[i * m:(i + 1) * m] == oracle.gemm(bits, False, A[i * k:(i + 1) * k], B, 1, m, k)).all(), f"row {i}"
+
+
+@pytest.mark.parametrize("bits", [64, 512])
+@pytest.mark.parametrize("m,n,k", [(30000, 3, 5), (3, 30000, 5), (66001, 1, 3), (257, 256, 2), (640, 75, 4)])
+def test_outputs_in_row_order_whatever_the_rows_length(capi, oracle, bits, m, n, k):
+    """Workgroups of 64 and of 256 consecutive outputs over rows of 1, 3, 75, 256 and 30,000."""
+    rng = np.random.default_rng(bits + m)
+    A, B = entries(rng, bits, m * k, "single"), entries(rng, bits, k * n, "single")
+    if m > 4:
+        A[2 * k:3 * k] = lfcases.zero(bits)
+        A[4 * k, bits // 32 + 2] = 2
+    got, _, _, _ = capi.gemm(bits, False, A, B, m, n, k)
+    assert (got == oracle.gemm(bits, False, A, B, m, n, k)).all()
+
+
+@pytest.mark.parametrize("cols", [63, 200, 300])
+def test_symmetric_outputs_in_row_order(capi, oracle, cols):
+    """Workgroups that cross the diagonal, lie above it, or hold the end of one row and the start of the next."""
+    bits, rows = 96, 5
+    A = entries(np.random.default_rng(cols), bits, rows * cols, "single")
+    want = oracle.syrk(bits, A, rows, cols, lower_only=False)
+    full, _, _, _ = capi.syrk(bits, A, rows, cols, lower_only=False)
+    assert (full == want).all()
+    lower, _, _, _ = capi.syrk(bits, A, rows, cols, lower_only=True)
+    keep = np.tril(np.ones((cols, cols), bool)).reshape(-1)
+    assert (lower[keep] == want[keep]).all()
+
+
+def test_more_rows_than_a_launch_has_workgroups_of_one(capi):
+    """2^24 rows of one output: with a workgroup of 256 a row, more threads than a launch can have.  K = 1, so the
+    product is the element-wise one with a broadcast factor."""
+    bits, m = 64, 1 << 24
+    rng = np.random.default_rng(3)
+    A, B = lfcases.random_records(rng, bits, m, 9), lfcases.random_records(rng, bits, 1, 9)
+    a, b, c, want = capi.Buffer(bits, m), capi.Buffer(bits, 1), capi.Buffer(bits, m), capi.Buffer(bits, m)
+    a.upload(A)
+    b.upload(B)
+    on_a_thread(lambda: capi.gemm_resident(bits, False, a, b, m, 1, 1, c))  # (60 GB of buffers)
+    capi.elementwise(bits, "mul", a, b, None, want, b_index=(1, 1))
+    assert np.array_equal(c.download(), want.download())

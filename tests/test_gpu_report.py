@@ -138,3 +138,29 @@ def test_report_matches_the_planning_rules(capi, bits, kind, k):
             assert rep.int8_gemms == 3 * want["moduli"]
             assert rep.npairs == min(64, want["pairs"])
             assert rep.gemm_rows == want["rows"] and rep.gemm_cols == want["cols"]
+
+
+@pytest.mark.parametrize("bits", [64, 256])
+@pytest.mark.parametrize("kind", ["single", "bands3", "mixed"])
+@pytest.mark.parametrize("k", [2048, 2049, 5000])
+def test_long_lines(capi, oracle, bits, kind, k):
+    """Lines whose exponents stay in registers over the band passes (up to 2,048) and lines that are read again: every
+    output against the oracle and the bands against the planning rules, rows and columns of A as the lines, with a zero
+    line, a status and a line of too many bands whose odd entries lie past entry 2,048."""
+    rng = np.random.default_rng(bits + k + len(kind))
+    m, n, w = 19, 18, bits // 32
+    A, B = entries(rng, bits, m * k, kind), entries(rng, bits, k * n, kind)
+    A[2 * k:3 * k] = lfcases.zero(bits)
+    A[4 * k + k - 1, w + 2] = 2
+    A[7 * k + k - 1, w] = lfcases.i32(-430)
+    B[(k - 1) * n + 5, w + 2] = 4
+    for j in range(6):
+        B[(k - 1 - j) * n + 17, w] = lfcases.i32(-75 * j)
+    want, plan = oracle.gemm(bits, False, A, B, m, n, k), expected(bits, A, B, m, n, k)
+    At = np.ascontiguousarray(A.reshape(m, k, -1).transpose(1, 0, 2)).reshape(k * m, -1)
+    for transposed, left in ((False, A), (True, At)):
+        print(f"[gpu] bits={bits} {kind} k={k} transposed={transposed}", flush=True)
+        got, rep, _, _ = capi.gemm(bits, transposed, left, B, m, n, k)
+        assert (got == want).all()
+        assert list(rep.bands("left")) == plan["left"][0] and rep.left_fallback == plan["left"][1]
+        assert list(rep.bands("right")) == plan["right"][0] and rep.right_fallback == plan["right"][1]
