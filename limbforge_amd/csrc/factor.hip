@@ -12,8 +12,8 @@
 //      SYRK product of the update GEMM (band analysis on the device, residue GEMM on int8 MFMA plus
 //      exact-dot lines, gemm.hip) on a second stream.
 // Every entry is one rounding of the same exact value in either part, so the bits are those of the serial
-// order.  The solves run block by block: the in-block recurrence on one wavefront per right-hand side, the
-// off-block updates as products of the update GEMM.
+// order.  The solves run block by block: the in-block recurrence on one wavefront per right-hand side
+// (tri_block_kernel), the off-block updates by update_wave_kernel, the largest as products of the update GEMM.
 #include "factor_launch.hpp"
 #include "gemm_plan.hpp"
 #include "host_copy.hpp"
@@ -64,7 +64,7 @@ struct OwnedStream {
     }
 };
 
-typedef hipError_t (*diag_fn)(const lf::FactorArgs&, uint32_t, hipStream_t);
+typedef hipError_t (*diag_fn)(const lf::FactorArgs&, hipStream_t);
 typedef hipError_t (*tri_fn)(const lf::TriArgs&, hipStream_t);
 typedef hipError_t (*update_fn)(const lf::UpdateArgs&, uint32_t, hipStream_t);
 typedef hipError_t (*invalid_fn)(uint32_t*, uint64_t, uint32_t, uint32_t, hipStream_t);
@@ -176,9 +176,11 @@ constexpr uint64_t LOOKAHEAD_WAVES = 2048;
 // wavefronts (and scratch slots) of a direct off-block solve update
 constexpr uint64_t SOLVE_UPDATE_WAVES = 4096;
 // Off-block solve updates of up to this many multiply-add terms (rows x right-hand sides x block) also run
-// as direct exact dots: on 4096 wavefronts 2^20 terms of 256 bits take about 30 us, less than one update
-// GEMM's planning round trip (band analysis, line-table download, constants, about 0.4 ms of host time per
-// update at n = 512 with 64 right-hand sides).  Both forms round the same exact value once.
+// directly: one launch on the stream, where the update GEMM takes four and two waits of the host.  Whole solves with
+// every update direct and with every update a product (ms): 256 bits, n = 512, 64 right-hand sides (updates of up to
+// 10^6 terms) 2.5 and 4.4; n = 1024, 128 (4 10^6) 6.7 and 9.6; n = 2048, 64 (4 10^6) 13.4 and 20.7; 512 bits,
+// n = 1024, 128 11.6 and 14.2.  Beyond it the products keep their place, unmeasured.  Both forms round the same exact
+// value once.
 constexpr double SOLVE_DIRECT_TERMS = 4194304.0;
 
 } // namespace
@@ -274,7 +276,7 @@ int lf_cholesky(int bits, const lf_operand* A, uint64_t n, const lf_operand* L, 
     auto panel = [&](uint64_t q, uint64_t a, uint64_t b) -> int {
         const lf::FactorArgs f{W, pitch, n32, uint32_t(a), uint32_t(b), (lf::FactorInfo*)dinfo.p, hinfo.p, derror, (uint32_t*)dscratch.p, swords,
                                (uint32_t*)drecip.p, rpitch};
-        FACTOR_HIP(tables().diag[N](f, uint32_t(std::min<uint64_t>(256, (b - a + 63) / 64 * 64)), s), "panel launch");
+        FACTOR_HIP(tables().diag[N](f, s), "panel launch");
         // the rows below: row i is the right-hand side of L_block l_i = a_i
         const lf::TriArgs t{W, pitch, int64_t(a * n + a), int64_t(n), 1, W, pitch, int64_t(b * n + a), 1, int64_t(n), (const uint32_t*)drecip.p,
                             rpitch, int64_t(a), 1, uint32_t(b - a), uint32_t(n - b), (uint32_t*)dscratch.p, swords, derror, f.info, uint32_t(a)};

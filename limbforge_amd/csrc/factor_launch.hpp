@@ -81,7 +81,7 @@ inline uint64_t factor_scratch_words(int N, uint64_t K)
     return bits / 32 + 4;
 }
 
-template <int N> hipError_t launch_chol_diag(const FactorArgs& f, uint32_t threads, hipStream_t s);
+template <int N> hipError_t launch_chol_diag(const FactorArgs& f, hipStream_t s);
 // one wavefront timing the per-row steps (factor_steps_kernel)
 template <int N>
 hipError_t launch_factor_steps(const uint32_t* v, uint64_t pitch, uint32_t* scratch, uint64_t swords, int32_t* err, int reps, uint64_t* out,

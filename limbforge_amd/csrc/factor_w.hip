@@ -10,9 +10,8 @@
 
 namespace lf {
 
-template <int N> hipError_t launch_chol_diag(const FactorArgs& f, uint32_t threads, hipStream_t s)
+template <int N> hipError_t launch_chol_diag(const FactorArgs& f, hipStream_t s)
 {
-    (void)threads;
     if (f.k1 <= f.k0) return hipSuccess;
     uint32_t resume = 0;
     if constexpr (wd_fits<N>())
@@ -86,7 +85,7 @@ hipError_t launch_factor_steps(const uint32_t* v, uint64_t pitch, uint32_t* scra
     return hipGetLastError();
 }
 
-template hipError_t launch_chol_diag<LF_WORDS>(const FactorArgs&, uint32_t, hipStream_t);
+template hipError_t launch_chol_diag<LF_WORDS>(const FactorArgs&, hipStream_t);
 template hipError_t launch_factor_steps<LF_WORDS>(const uint32_t*, uint64_t, uint32_t*, uint64_t, int32_t*, int, uint64_t*, uint32_t*, hipStream_t);
 template hipError_t launch_tri_block<LF_WORDS>(const TriArgs&, hipStream_t);
 template hipError_t launch_update<LF_WORDS>(const UpdateArgs&, uint32_t, hipStream_t);

@@ -313,8 +313,10 @@ template <bool BY_LINE> __device__ __forceinline__ void analyze_line(const Analy
     const auto mn = [](int x, int y) { return min(x, y); };
     u32 status = 0;
     int top = INT_MIN, bottom = INT_MAX;
-    // a thread's exponents stay in registers for the band passes (INT_MIN: zero, status or past K) where they fit; all
-    // their loads are then in flight together
+    // a thread's exponents stay in registers for the band passes (INT_MIN: zero, status or past K) where they fit, in 32
+    // registers for lines of up to 2,048 entries; all their loads are then in flight together.  Longer lines are read
+    // again by each pass: 64 lines of 2,048 and of 2,112 entries take 27 and 43 us with adjacent entries (one band), 30
+    // and 57 with adjacent lines (three bands).
     constexpr u32 KEPT = 32;
     const bool kept = a.K <= KEPT * step;
     int own[KEPT];
@@ -825,9 +827,9 @@ bool plan_moduli(Plan& p, int bits, int logk)
     return p.wx_class < 2;
 }
 std::size_t digit_bytes(int N, int width) { return (std::size_t(4 * N) + (width + 7) / 8 + 31) / 32 * 32; }
-// Nanoseconds of the three large stages, from their measured rates on an MI355X: 2.8 per 32-deep step of a 128 x 128
-// product tile, 16 CRT multiply-adds per picosecond-thousand and 0.06 per staged band pair and output, 0.7 per
-// thousand residues.  It only has to rank two plans of one product, which differ by their moduli and rows; memory is not
+// Nanoseconds of the three large stages, from their measured rates on an MI355X: 2.8 for a 32-deep step of a 128 x 128
+// product tile of one modulus; 6.2e-5 for each modulus and CRT word of an output (16 multiply-adds a picosecond) and
+// 0.06 for each band pair of an output that passes through the stage; 7e-4 for a residue's digits.  It only has to rank two plans of one product, which differ by their moduli and rows; memory is not
 // part of it (a joined plan that does not fit gives way when its buffers are reserved).
 double plan_cost(const Plan& p, int N, std::size_t rows, std::size_t cols, std::size_t lines, std::size_t K, double pairs, bool syrk)
 {

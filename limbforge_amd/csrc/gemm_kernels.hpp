@@ -19,6 +19,7 @@
 //   dot_cluster_kernel  exponent clusters with a sticky sign for outputs whose terms spread further
 #pragma once
 #include "gemm_common.hpp"
+#include "gemm_launch.hpp"
 #include "limb_core.hpp"
 #include "residue_reduce.hpp"
 
@@ -121,7 +122,7 @@ template <int N> __global__ void __launch_bounds__(256, 2) digits_kernel(DigitsA
     // waves 0-3: entries 64 wave + 32 h + (lane % 32); bytes 32 step + 16 (lane / 32) of each
     const u32 steps = g.bytes / 32u, r = lane & 31u, kh = lane >> 5;
     const u32 sg[2] = {signs[2u * wave], signs[2u * wave + 1u]};
-    constexpr u32 STEPS = (4 * N + 67 + 31) / 32; // a CRT class holds bands of at most 534 bits
+    constexpr u32 STEPS = digit_bytes_max(N) / 32;
     v4i a[STEPS][2];
 #pragma unroll
     for (u32 st = 0; st < STEPS; ++st)
@@ -251,8 +252,8 @@ template <int WX> __device__ __forceinline__ int crt_reduce(const u32* Mb, u32 (
 // factor still applied here): 67-word rows 300 us scalar against 173 us staged; 39-word rows 500 us scalar
 // against 531 us staged.
 constexpr int CRT_LDS_MIN_WX = 48;
-template <int WX, class Args>
-__device__ __forceinline__ int crt_rebuild(const Args& g, const u32* tab, u32 row, u32 col, u32 (&X)[WX])
+template <int WX>
+__device__ __forceinline__ int crt_rebuild(const RebuildArgs& g, const u32* tab, u32 row, u32 col, u32 (&X)[WX])
 {
     // tab (LDS, when WX >= CRT_LDS_MIN_WX): the L rows of WX CRT words
     constexpr bool STAGED = WX >= CRT_LDS_MIN_WX;
@@ -405,8 +406,10 @@ template <int N, int WX> __global__ void __launch_bounds__(ROUND_BLOCK) crt_roun
 {
     constexpr int QW = quarter_words(WX), QP = quarter_pitch(WX);
     extern __shared__ __attribute__((aligned(16))) u32 tab[];
-    // outputs in row order, whatever the rows' length: a workgroup takes consecutive ones
-    const u32 block = blockDim.x, total = g.m * g.n, first = blockIdx.x * block, idx = first + threadIdx.x, quarter = threadIdx.x & 3u;
+    // outputs in row order, whatever the rows' length: a workgroup takes consecutive ones (of one wavefront instead of
+    // four it was no faster from 4,096 outputs to 200,000: 87.6 and 86.4 us the 256-bit 96 x 75 x 130 product)
+    constexpr u32 block = ROUND_BLOCK;
+    const u32 total = g.m * g.n, first = blockIdx.x * block, idx = first + threadIdx.x, quarter = threadIdx.x & 3u;
     if (g.syrk) { // nothing to do where the whole workgroup lies above the diagonal, in one row
         const u32 i0 = first / g.n, i1 = min(first + block, total) - 1u;
         if (first - i0 * g.n > i0 && i1 / g.n == i0) return;

@@ -12,7 +12,7 @@ template <int N> hipError_t launch_digits(const DigitsArgs& g, hipStream_t s)
 {
     const u32 blocks = g.side[0].blocks + g.side[1].blocks;
     if (!g.K || !blocks || !g.L) return hipSuccess;
-    if (g.Kp % 32u || g.bytes % 32u || g.bytes > DIGIT_TABLE_BYTES || g.bytes > (4 * N + 67 + 31) / 32 * 32) return hipErrorInvalidValue;
+    if (g.Kp % 32u || g.bytes % 32u || g.bytes > DIGIT_TABLE_BYTES || g.bytes > digit_bytes_max(N)) return hipErrorInvalidValue;
     const u64 lds = digits_lds_bytes(g.bytes);
     if (lds > (u64(64) << 10))
         if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&digits_kernel<N>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
@@ -27,9 +27,7 @@ template <int N, int WX> hipError_t launch_round_wx(const RoundArgs& g, hipStrea
     if (lds > (u64(64) << 10))
         if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&crt_round_kernel<N, WX>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds))
             return e;
-    // small products in workgroups of one wavefront, to spread over the GPU
-    const u32 RB = (u64)g.m * g.n >= 65536 ? ROUND_BLOCK : 64u;
-    hipLaunchKernelGGL((crt_round_kernel<N, WX>), dim3((unsigned)(((u64)g.m * g.n + RB - 1) / RB)), dim3(RB), lds, s, g);
+    hipLaunchKernelGGL((crt_round_kernel<N, WX>), dim3((unsigned)(((u64)g.m * g.n + ROUND_BLOCK - 1) / ROUND_BLOCK)), dim3(ROUND_BLOCK), lds, s, g);
     return hipGetLastError();
 }
 

@@ -88,8 +88,9 @@ unsigned block_for(const unsigned* block, int i, int bits)
     std::lock_guard<std::mutex> lock(tuned_mutex);
     auto it = tuned.find({dev, bits});
     // untuned: one wavefront a workgroup.  The kernels share nothing within a workgroup, and the wavefronts of a larger
-    // one end with their longest chain and hold its place until then: the graph of 10^6 values took 865 us with 256
-    // threads, 805 with 128, 789 with 64; 50,000 values took 485-495 us with each.
+    // one end with their longest chain and hold its place until then: launches of the graph of 10^6 values back to back,
+    // on the same operands, took 865 us each with 256 threads, 808 with 128, 790 with 64 (916 and 892 us with 256 and
+    // 64 where every launch has other operands); 50,000 values took 485-495 us with each.
     return it == tuned.end() ? 64u : it->second;
 }
 

@@ -165,3 +165,17 @@ def test_more_rows_than_a_launch_has_workgroups_of_one(capi):
     on_a_thread(lambda: capi.gemm_resident(bits, False, a, b, m, 1, 1, c))  # (60 GB of buffers)
     capi.elementwise(bits, "mul", a, b, None, want, b_index=(1, 1))
     assert np.array_equal(c.download(), want.download())
+
+
+@pytest.mark.parametrize("bits", [64, 544, 1024])
+@pytest.mark.parametrize("width", [534, 539, 541, 542, 600])
+def test_bands_around_the_widest_of_the_crt_classes(capi, oracle, bits, width):
+    """Lines of one band as wide as the wider CRT class holds (542 bits less those of the terms), below it and past it."""
+    rng = np.random.default_rng(bits + width)
+    m, n = 5, 7
+    for k in (2, 3):
+        A, B = lfcases.random_records(rng, bits, m * k, 0), lfcases.random_records(rng, bits, k * n, 0)
+        A[:, bits // 32] = lfcases.i32(np.where(np.arange(m * k) % k == 0, 0, -width))
+        B[:, bits // 32] = lfcases.i32(np.where(np.arange(k * n) // n == k - 1, 0, -width))
+        got, _, _, _ = capi.gemm(bits, False, A, B, m, n, k, options=capi.LinalgOptions.default(band_bits=1024, max_spread=8192))
+        assert (got == oracle.gemm(bits, False, A, B, m, n, k)).all(), k
