@@ -290,8 +290,8 @@ template <int GD, int H> __device__ __forceinline__ void wd_accumulate(i64* at, 
 // Row i's exact dot and its one-lane division, for rows that the wave-parallel forms do not decide: the dot's record
 // goes to `rec`, the division replaces it by the quotient's and stores x_i.  `rec` is also the dot's LDS, of rows
 // 0 .. i + 1.  Both read the kernel's arguments again, through a pointer that the compiler cannot follow, so that neither
-// they nor what is formed from them takes scalar registers of the recurrence's loop (which spilled them: 57 instead of
-// 52 us a block).
+// they nor what is formed from them takes scalar registers of the recurrence's loop (52.8 and 51.9 us a block at 256 bits
+// without and with it).
 __device__ __forceinline__ TriArgs tri_args_again()
 {
     typedef const __attribute__((address_space(4))) TriArgs* args_ptr; // the kernel's one argument
