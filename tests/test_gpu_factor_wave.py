@@ -217,3 +217,46 @@ def test_every_width(capi, oracle, bits):
         for passes in (1, 2):
             got, _, _ = capi.solve(bits, passes, L, n, B, nrhs, block=block)
             assert (got == oracle.solve(bits, L, n, B, nrhs, block, passes)).all(), f"span={span} passes={passes}"
+
+
+def hard_pivots(rng, bits, count):
+    """Positive records whose roots and reciprocals lie at the edges of their roundings: all ones and one unit less, powers
+    of two and one unit more, squares of short and of long mantissas, and the values nearest to squares halfway between
+    two mantissas."""
+    w, out = bits // 32, []
+    for i in range(count):
+        kind, e, full = i % 7, int(rng.integers(-3, 4)), 1 << (bits - 1)
+        long = full | int.from_bytes(rng.bytes(bits // 8), "little") >> 1
+        if kind < 4:
+            m = (2 * full - 1, 2 * full - 2, full, full + 1)[kind]
+        else:
+            root = (int(rng.integers(3, 1 << 16)), long >> (bits // 2) << (bits // 2), 2 * long + 1)[kind - 4]
+            square = root * root
+            shift = square.bit_length() - bits
+            m = square << -shift if shift <= 0 else (square + (1 << (shift - 1))) >> shift
+            if m >> bits:
+                m, shift = m >> 1, shift + 1
+            e = 2 * (e // 2) + (square.bit_length() - 1) % 2  # an exponent of the square's parity
+        x = lfcases.one(bits, e)
+        x[:w] = [(m >> (32 * k)) & 0xFFFFFFFF for k in range(w)]
+        out.append(x)
+    return np.stack(out)
+
+
+@pytest.mark.parametrize("bits", range(64, 641, 32))
+def test_pivots_at_the_edges_of_their_roundings(capi, oracle, bits):
+    """Two blocks of such pivots with nothing between them, and rows below that each pivot's reciprocal divides."""
+    rng = np.random.default_rng(bits)
+    n, k, w = 70, 64, bits // 32
+    A = np.stack([lfcases.zero(bits)] * (n * n))
+    A[np.arange(k) * (n + 1)] = hard_pivots(rng, bits, k)
+    for i in range(k, n):
+        A[i * (n + 1)] = lfcases.one(bits, 24)
+        row = special_mantissas(rng, lfcases.random_records(rng, bits, k, 3), bits)
+        for j in range(k):
+            A[i * n + j] = A[j * n + i] = row[j]
+    want, piv, _, _ = oracle.cholesky(bits, A, n, 32)
+    got, info = capi.cholesky(bits, A, n, block=32)
+    assert info.pivot == piv == n
+    bad = np.nonzero((got != want).any(axis=1))[0]
+    assert bad.size == 0, f"{bad.size} entries differ, first ({bad[0] // n},{bad[0] % n})"
